@@ -33,7 +33,7 @@ __device__ __forceinline__ T *as_global(T *p)
 __device__ __forceinline__ DevScene global_scene(const DevScene &S)
 {
     return DevScene{as_global(S.records), as_global(S.root), as_global(S.prims), as_global(S.prim_index),
-                    as_global(S.flags), as_global(S.stats)};
+                    as_global(S.disks), as_global(S.disk_limit), as_global(S.flags), as_global(S.stats)};
 }
 
 struct BatchScene {

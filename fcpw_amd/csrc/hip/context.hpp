@@ -25,6 +25,19 @@ struct fcpw_hip_ctx {
     int32_t *rec_parent = nullptr, *leaf_refs = nullptr;
     uint32_t *leaf_links = nullptr;
     unsigned int *counters = nullptr;
+    // the leaf-slot range below every child slot, the slots sorted by its size,
+    // and the disks with the distance they hold up to: parts of range_mem, which
+    // is null for a tree over instances.  by_range: the leaves lie in order, so
+    // the ranges are valid
+    void *range_mem = nullptr;
+    float4 *disks = nullptr;
+    int4 *top = nullptr;
+    int2 *ranges = nullptr;
+    int *big = nullptr, *frontier = nullptr, *range_info = nullptr;
+    uint32_t *range_mark = nullptr, *range_sums = nullptr;
+    float *disk_limit = nullptr;
+    bool by_range = false;
+    int n_big = 0, n_top = 0, n_frontier = 0;
     int *flags = nullptr;
     unsigned long long *stats = nullptr; // internal nodes, primitive tests, queries (option "stats")
     // silhouettes (fcpw_hip_upload_silhouettes): cones per child slot and root, leaf ranges, records
@@ -124,10 +137,18 @@ static void free_silhouettes(fcpw_hip_ctx *c)
 static void free_scene(fcpw_hip_ctx *c)
 {
     void *bufs[] = {c->records, c->root, c->prims, c->prim_index, c->prim_vids, c->V,
-                    c->rec_parent, c->leaf_refs, c->leaf_links, c->counters, c->inst, c->obj_table};
+                    c->rec_parent, c->leaf_refs, c->leaf_links, c->counters, c->inst, c->obj_table, c->range_mem};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     free_silhouettes(c);
+    c->range_mem = nullptr;
+    c->disks = nullptr;
+    c->top = nullptr;
+    c->ranges = nullptr;
+    c->big = c->frontier = c->range_info = nullptr;
+    c->range_mark = c->range_sums = nullptr;
+    c->disk_limit = nullptr;
+    c->by_range = false;
     c->inst = nullptr;
     c->obj_table = nullptr;
     c->instanced = false;
@@ -149,7 +170,7 @@ static inline int sil_xcd_arg(const fcpw_hip_ctx *c) { return c->sil_xcds | (c->
 
 static DevScene dev_scene(fcpw_hip_ctx *c)
 {
-    return DevScene{c->records, c->root, c->prims, c->prim_index, c->flags, c->stats};
+    return DevScene{c->records, c->root, c->prims, c->prim_index, c->disks, c->disk_limit, c->flags, c->stats};
 }
 
 static int grow(fcpw_hip_ctx *c, void **buf, size_t *cap, size_t bytes)

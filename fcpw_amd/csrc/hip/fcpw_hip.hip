@@ -60,6 +60,103 @@ struct BuildScratch {
     }
 };
 
+// grid of the kernels that share slots out by size (k_refit_ranges, k_build_disks)
+static int slot_own_blocks(const fcpw_hip_ctx *c) { return (2 * c->n_records + DISK_BLOCK - 1) / DISK_BLOCK; }
+static dim3 slot_grid(const fcpw_hip_ctx *c)
+{
+    return dim3((unsigned)(slot_own_blocks(c) + (c->n_big + DISK_BLOCK / 64 - 1) / (DISK_BLOCK / 64)));
+}
+
+// the disks of a single object's tree, from its records, primitives and ranges
+static int launch_disks(fcpw_hip_ctx *c, hipStream_t s)
+{
+    if (!c->by_range) return FCPW_HIP_OK;
+    const int n_slots = 2 * c->n_records;
+    if (c->dim == 3)
+        hipLaunchKernelGGL(k_build_disks<3>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->root, c->prims,
+                           c->ranges, n_slots, c->big, c->n_big, slot_own_blocks(c), c->disks, c->disk_limit);
+    else
+        hipLaunchKernelGGL(k_build_disks<2>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->root, c->prims,
+                           c->ranges, n_slots, c->big, c->n_big, slot_own_blocks(c), c->disks, c->disk_limit);
+    HIPCHECK(c, hipGetLastError());
+    return FCPW_HIP_OK;
+}
+
+// ranges, slot lists and disks of a tree whose slots were (re)numbered
+template <int DIM>
+static int compute_ranges(fcpw_hip_ctx *c)
+{
+    c->by_range = false;
+    c->n_big = c->n_top = c->n_frontier = 0;
+    const float none = -1.0f;
+    HIPCHECK(c, hipMemcpy(c->disk_limit, &none, sizeof(float), hipMemcpyHostToDevice));
+    if (c->n_records <= 0) return FCPW_HIP_OK; // a root leaf has no slots
+    const int n_slots = 2 * c->n_records, t = 256;
+    const dim3 gs((unsigned)((n_slots + t - 1) / t));
+    HIPCHECK(c, hipMemset(c->range_info, 0, 4 * sizeof(int)));
+    HIPCHECK(c, hipMemset(c->range_mark, 0, ((size_t)c->n_prims + 1) * sizeof(uint32_t)));
+    hipLaunchKernelGGL(k_slot_ranges<DIM>, dim3((unsigned)((c->n_records + t - 1) / t)), dim3(t), 0, 0, c->records,
+                       c->n_records, c->ranges, c->range_info);
+    HIPCHECK(c, hipGetLastError());
+    int info[4];
+    HIPCHECK(c, hipMemcpy(info, c->range_info, sizeof(info), hipMemcpyDeviceToHost));
+    if (info[0]) return FCPW_HIP_OK; // leaves out of order: boxes alone, refitted by climbing
+    hipLaunchKernelGGL(k_slot_lists<DIM>, gs, dim3(t), 0, 0, c->ranges, c->root, n_slots, c->big, c->top,
+                       c->range_mark, c->range_info);
+    const int st = exclusive_scan(c, c->range_mark, (int64_t)c->n_prims + 1, c->range_sums, 0);
+    if (st) return st;
+    hipLaunchKernelGGL(k_slot_frontier<DIM>, gs, dim3(t), 0, 0, c->ranges, c->root, n_slots, c->range_mark, c->top,
+                       c->frontier, c->range_info);
+    HIPCHECK(c, hipGetLastError());
+    uint32_t n_frontier = 0;
+    HIPCHECK(c, hipMemcpy(info, c->range_info, sizeof(info), hipMemcpyDeviceToHost));
+    HIPCHECK(c, hipMemcpy(&n_frontier, c->range_mark + c->n_prims, sizeof(uint32_t), hipMemcpyDeviceToHost));
+    c->n_big = info[1];
+    c->n_top = info[2];
+    c->n_frontier = (int)n_frontier;
+    c->by_range = true;
+    return launch_disks(c, 0);
+}
+
+static int compute_ranges(fcpw_hip_ctx *c) { return c->dim == 3 ? compute_ranges<3>(c) : compute_ranges<2>(c); }
+
+// allocates the ranges, lists and disks of a freshly uploaded or built tree (one
+// allocation) and computes them; c's counts, dimension and tree must be set
+static int upload_ranges(fcpw_hip_ctx *c)
+{
+    const size_t n_slots = (size_t)2 * c->n_records, n_prims = (size_t)c->n_prims;
+    // slots above DISK_MAX_PRIMS are disjoint at each of at most STACK_TOTAL - 1 levels,
+    // and every marked slot is a child of one of their records or of the root
+    const size_t cap_top = std::min(n_slots, (size_t)STACK_TOTAL * (n_prims / DISK_MAX_PRIMS + 1));
+    const size_t cap_front = std::min(n_slots, 2 * cap_top + 2);
+    const size_t segs = (n_prims + 1 + SCAN_SEG - 1) / SCAN_SEG;
+    size_t bytes = 0;
+    auto take = [&bytes](size_t b) {
+        const size_t at = bytes;
+        bytes += (b + 255) / 256 * 256;
+        return at;
+    };
+    const size_t at_disks = take(n_slots * sizeof(float4)), at_top = take(cap_top * sizeof(int4)),
+                 at_ranges = take(n_slots * sizeof(int2)), at_big = take(n_slots * sizeof(int)),
+                 at_front = take(cap_front * sizeof(int)), at_mark = take((n_prims + 1) * sizeof(uint32_t)),
+                 at_sums = take(segs * sizeof(uint32_t)), at_info = take(4 * sizeof(int)), at_limit = take(sizeof(float));
+    HIPCHECK(c, hipMalloc((void **)&c->range_mem, bytes));
+    char *m = (char *)c->range_mem;
+    c->disks = (float4 *)(m + at_disks);
+    c->top = (int4 *)(m + at_top);
+    c->ranges = (int2 *)(m + at_ranges);
+    c->big = (int *)(m + at_big);
+    c->frontier = (int *)(m + at_front);
+    c->range_mark = (uint32_t *)(m + at_mark);
+    c->range_sums = (uint32_t *)(m + at_sums);
+    c->range_info = (int *)(m + at_info);
+    c->disk_limit = (float *)(m + at_limit);
+    const int st = compute_ranges(c);
+    if (st) return st;
+    HIPCHECK(c, hipDeviceSynchronize());
+    return FCPW_HIP_OK;
+}
+
 static unsigned blocks_for(int64_t n, int t) { return (unsigned)std::max<int64_t>(1, (n + t - 1) / t); }
 
 template <int DIM>
@@ -264,6 +361,8 @@ static int gpu_build(fcpw_hip_ctx *c, const float *positions, int n_vertices, co
     c->max_depth = status[1];
     c->node_slot = std::move(node_slot);
     c->node_leaf_off = std::move(node_leaf_off);
+    const int st_disks = upload_ranges(c);
+    if (st_disks) return st_disks;
     c->uploaded = true;
     c->generation++;
     c->positions_version++;
@@ -575,6 +674,10 @@ static int relayout_records(fcpw_hip_ctx *c, int layout)
         }
         HIPCHECK(c, hipMemcpy(c->cones, cones2.data(), cones2.size() * sizeof(float4), hipMemcpyHostToDevice));
     }
+    if (c->range_mem) {
+        const int st = compute_ranges(c);
+        if (st) return st;
+    }
     HIPCHECK(c, hipDeviceSynchronize());
     c->generation++; // batches re-read their tables
     return FCPW_HIP_OK;
@@ -672,6 +775,7 @@ int fcpw_hip_upload_bvh(fcpw_hip_ctx *c, int dim, int n_nodes, const float *pmin
     c->max_depth = T.max_depth;
     c->node_slot = std::move(T.node_slot);
     c->node_leaf_off = std::move(T.node_leaf_off);
+    if ((st = upload_ranges(c))) return st;
     c->uploaded = true;
     c->generation++;
     c->positions_version++;
@@ -772,10 +876,10 @@ static int launch_rebuild(fcpw_hip_ctx *c, hipStream_t s)
     int threads = 256, blocks = (c->n_prims + threads - 1) / threads;
     if (c->dim == 3)
         hipLaunchKernelGGL(k_rebuild_prims<3>, dim3(blocks), dim3(threads), 0, s, c->prims, c->prim_vids, c->V,
-                           c->n_prims);
+                           c->n_prims, c->disk_limit);
     else
         hipLaunchKernelGGL(k_rebuild_prims<2>, dim3(blocks), dim3(threads), 0, s, c->prims, c->prim_vids, c->V,
-                           c->n_prims);
+                           c->n_prims, c->disk_limit);
     HIPCHECK(c, hipGetLastError());
     return FCPW_HIP_OK;
 }
@@ -817,13 +921,31 @@ int fcpw_hip_refit(fcpw_hip_ctx *c, void *stream)
     hipStream_t s = (hipStream_t)stream;
     if (c->instanced) return instances_refit(c, s);
     int threads = 256, blocks = (c->n_leaves + threads - 1) / threads;
-    if (c->dim == 3)
-        hipLaunchKernelGGL(k_refit<3>, dim3(blocks), dim3(threads), 0, s, c->records, c->root, c->prims,
-                           c->leaf_refs, c->leaf_links, c->rec_parent, c->counters, c->n_leaves);
-    else
-        hipLaunchKernelGGL(k_refit<2>, dim3(blocks), dim3(threads), 0, s, c->records, c->root, c->prims,
-                           c->leaf_refs, c->leaf_links, c->rec_parent, c->counters, c->n_leaves);
+    if (c->by_range) {
+        const int n_slots = 2 * c->n_records;
+        const dim3 gt((unsigned)(c->n_top / (DISK_BLOCK / 64) + 1));
+        if (c->dim == 3) {
+            hipLaunchKernelGGL(k_refit_ranges<3>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->prims,
+                               c->ranges, n_slots, c->big, c->n_big, slot_own_blocks(c));
+            hipLaunchKernelGGL(k_refit_top<3>, gt, dim3(DISK_BLOCK), 0, s, c->records, c->root, c->top, c->n_top,
+                               c->frontier, c->n_frontier);
+        } else {
+            hipLaunchKernelGGL(k_refit_ranges<2>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->prims,
+                               c->ranges, n_slots, c->big, c->n_big, slot_own_blocks(c));
+            hipLaunchKernelGGL(k_refit_top<2>, gt, dim3(DISK_BLOCK), 0, s, c->records, c->root, c->top, c->n_top,
+                               c->frontier, c->n_frontier);
+        }
+    } else {
+        // a root leaf, or a caller's tree whose leaves are out of order
+        if (c->dim == 3)
+            hipLaunchKernelGGL(k_refit<3>, dim3(blocks), dim3(threads), 0, s, c->records, c->root, c->prims,
+                               c->leaf_refs, c->leaf_links, c->rec_parent, c->counters, c->n_leaves);
+        else
+            hipLaunchKernelGGL(k_refit<2>, dim3(blocks), dim3(threads), 0, s, c->records, c->root, c->prims,
+                               c->leaf_refs, c->leaf_links, c->rec_parent, c->counters, c->n_leaves);
+    }
     HIPCHECK(c, hipGetLastError());
+    if ((st = launch_disks(c, s))) return st;
     if (c->has_silhouettes) {
         if (c->dim == 3)
             hipLaunchKernelGGL(k_refit_cones<3>, dim3(blocks), dim3(threads), 0, s, c->records, c->root, c->cones,
