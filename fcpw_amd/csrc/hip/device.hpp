@@ -958,10 +958,11 @@ __device__ __forceinline__ void wave_loop_stats_add(const DevScene &S, uint32_t 
 }
 
 template <int DIM, int K, int OUT, bool STATS>
-__global__ __launch_bounds__(64) void k_closest_points_coop(DevScene S, CpIO io, int xcds, int hold_min)
+__global__ __launch_bounds__(64) void k_closest_points_coop(DevScene S, CpIO io, int xcds, int hold_min,
+                                                            int wave_q)
 {
-    int64_t k = xcd_tile(xcds) * 64 + threadIdx.x;
-    bool valid = k < io.n;
+    int64_t k = xcd_tile(xcds) * wave_q + threadIdx.x;
+    bool valid = (int)threadIdx.x < wave_q && k < io.n;
     int64_t i = valid ? (io.order ? (int64_t)io.order[k] : k) : 0;
     float q[3] = {0.0f, 0.0f, 0.0f}, r2 = -1.0f;
     if (valid) cp_load<DIM, OUT>(io, i, q, r2);
@@ -1135,13 +1136,14 @@ __device__ __forceinline__ uint32_t ray_coop_leaf_pass(const DevScene &S, CoopSh
 
 template <int DIM, int K, bool STATS>
 __global__ __launch_bounds__(64) FCPW_EIGHT_WAVES void k_intersect_coop(DevScene S, const float2 *rays, int64_t n, int occlusion,
-                                                       float2 *out, const uint32_t *order, int xcds, int hold_min)
+                                                       float2 *out, const uint32_t *order, int xcds, int hold_min,
+                                                       int wave_q)
 {
     using G = Geo<DIM>;
     constexpr int BLOCK = 64;
     __shared__ CoopShared sh;
-    const int64_t k = xcd_tile(xcds) * 64 + threadIdx.x;
-    const bool valid = k < n;
+    const int64_t k = xcd_tile(xcds) * wave_q + threadIdx.x;
+    const bool valid = (int)threadIdx.x < wave_q && k < n;
     const int64_t i = valid ? (order ? (int64_t)order[k] : k) : 0;
     float o3[3] = {0.0f, 0.0f, 0.0f}, d3[3] = {0.0f, 0.0f, 0.0f}, di3[3] = {0.0f, 0.0f, 0.0f};
     float tmax = -1.0f;

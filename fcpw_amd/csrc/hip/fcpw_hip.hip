@@ -969,6 +969,22 @@ static dim3 grid_for(fcpw_hip_ctx *, int64_t n, int block)
     return dim3((unsigned)std::max<int64_t>(1, (n + block - 1) / block));
 }
 
+// Queries per wave of the cooperative kernels: 64, halved while the batch makes
+// fewer than eight waves per CU.  A wave ends with its longest query and an idle
+// chip issues nothing in between, so small batches spread out: fewer queries
+// share a wave's lockstep, and its leaf passes still use all lanes.  1,000
+// closest points on 20,480 triangles 64 a wave 215 us, 8 a wave 155, 2 136, 1
+// 118; 12,000 on 300,000 triangles 64 a wave 840 us, 4 690; 65,537 occlusion
+// rays 64 a wave 270 us, 32 242, 16 265; 100,003 closest points 64 a wave 171
+// us, 32 163, 16 171.  With the chip full a part-filled wave only wastes issue:
+// 4.2M rays 64 a wave 1.96 ms, 32 2.48 ms.
+static int wave_queries(const fcpw_hip_ctx *c, int64_t n)
+{
+    int q = 64;
+    while (q > 1 && n < (int64_t)q * 8 * c->n_cus) q >>= 1;
+    return q;
+}
+
 // "timing": a HIP event pair on the launch stream around each traversal launch
 static int timing_begin(fcpw_hip_ctx *c, hipStream_t s)
 {
@@ -1015,6 +1031,8 @@ static int64_t morton_cells(int dim, int morton_bits, int64_t n, int dir_off, in
 static int morton_order_into(fcpw_hip_ctx *c, const float *pts, int stride, int64_t n, hipStream_t s, int morton_bits,
                              int dir_off, uint32_t *codes, uint32_t *perm, uint32_t *hist, uint32_t *sums);
 
+// Morton order of n query points (pts + i * stride floats); returns the
+// permutation, or nullptr when ordering is off or the batch is small
 static int morton_order(fcpw_hip_ctx *c, const float *pts, int stride, int64_t n, hipStream_t s,
                         const uint32_t **perm_out, int dir_off = -1)
 {
@@ -1107,14 +1125,16 @@ static int launch_closest_kernel(fcpw_hip_ctx *c, const CpIO &io, hipStream_t s,
         dim3 g = grid_for(c, n, 64);
         if (c->dim == 3)
             hipLaunchKernelGGL((k_closest_points_coop<3, 16, OUT, true>), g, dim3(64), 0, s, S, io, xcd_arg(c),
-                               c->hold_min);
+                               c->hold_min, 64);
         else
             hipLaunchKernelGGL((k_closest_points_coop<2, 16, OUT, true>), g, dim3(64), 0, s, S, io, xcd_arg(c),
-                               c->hold_min);
+                               c->hold_min, 64);
     } else if (c->coop) {
-        dim3 g = grid_for(c, n, 64);
-#define FCPW_COOP(D, K) \
-    hipLaunchKernelGGL((k_closest_points_coop<D, K, OUT, false>), g, dim3(64), 0, s, S, io, xcd_arg(c), c->hold_min)
+        const int wq = wave_queries(c, n);
+        dim3 g = grid_for(c, n, wq);
+#define FCPW_COOP(D, K)                                                                                       \
+    hipLaunchKernelGGL((k_closest_points_coop<D, K, OUT, false>), g, dim3(64), 0, s, S, io, xcd_arg(c), c->hold_min, \
+                       wq)
         const int k = c->stack; // 0, 4, 6, 8, 12, 16 or 24 LDS entries (2D: 24 runs as 16)
         if (c->dim == 3) {
             if (k == 0) FCPW_COOP(3, 0);
@@ -1204,11 +1224,15 @@ static int launch_intersect(fcpw_hip_ctx *c, const void *rays, int64_t n, int oc
     if (st) return st;
     if ((st = timing_begin(c, s))) return st;
     if (c->ray_coop) {
-        const dim3 g = grid_for(c, n, 64);
+        const int wq = c->stats_on ? 64 : wave_queries(c, n);
+        // a part-filled wave has lanes free for every leaf: it waits for no others
+        // (65,537 occlusion rays, 32 a wave: 250 us waiting for 8, 238 for 1)
+        const int hold = wq < 64 ? 1 : c->ray_hold_min;
+        const dim3 g = grid_for(c, n, wq);
         const int k = c->ray_stack;
 #define FCPW_RCOOP(D, K, ST)                                                                                  \
     hipLaunchKernelGGL((k_intersect_coop<D, K, ST>), g, dim3(64), 0, s, S, (const float2 *)rays, n, occlusion, \
-                       (float2 *)out, order, xcd_arg(c), c->ray_hold_min)
+                       (float2 *)out, order, xcd_arg(c), hold, wq)
         if (c->stats_on) {
             if (c->dim == 3) FCPW_RCOOP(3, 16, true);
             else FCPW_RCOOP(2, 16, true);
@@ -1424,10 +1448,11 @@ static int launch_silhouettes(fcpw_hip_ctx *c, const void *spheres, const uint32
     if (st) return st;
     if (c->coop && c->sil_leaf_max <= 1023) {
         // record indices within a leaf travel in 10 bits of a leaf-pass item
-        const dim3 g = grid_for(c, n, 64);
+        const int wq = wave_queries(c, n);
+        const dim3 g = grid_for(c, n, wq);
 #define FCPW_SIL3(K)                                                                                          \
     hipLaunchKernelGGL((k_closest_silhouettes_coop<3, K>), g, dim3(64), 0, s, S, T, (const float4 *)spheres, flip, n, \
-                       r2min, prec, (float2 *)out, order, sil_xcd_arg(c), c->sil_hold_min)
+                       r2min, prec, (float2 *)out, order, sil_xcd_arg(c), c->sil_hold_min, wq)
         if (c->dim == 3) {
             if (c->sil_stack == 8) FCPW_SIL3(8);
             else if (c->sil_stack == 12) FCPW_SIL3(12);
@@ -1435,7 +1460,7 @@ static int launch_silhouettes(fcpw_hip_ctx *c, const void *spheres, const uint32
         } else
 #undef FCPW_SIL3
             hipLaunchKernelGGL((k_closest_silhouettes_coop<2, 8>), g, dim3(64), 0, s, S, T, (const float4 *)spheres,
-                               flip, n, r2min, prec, (float2 *)out, order, sil_xcd_arg(c), c->sil_hold_min);
+                               flip, n, r2min, prec, (float2 *)out, order, sil_xcd_arg(c), c->sil_hold_min, wq);
     } else if (c->dim == 3)
         hipLaunchKernelGGL((k_closest_silhouettes<3, 128, 8>), dim3(blocks), dim3(128), 0, s, S, T,
                            (const float4 *)spheres, flip, n, r2min, prec, (float2 *)out, order, sil_xcd_arg(c));

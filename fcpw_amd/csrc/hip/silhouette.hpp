@@ -415,15 +415,15 @@ template <int DIM, int K>
 __global__ __launch_bounds__(64) FCPW_EIGHT_WAVES void k_closest_silhouettes_coop(DevScene S, SilScene T, const float4 *spheres,
                                                                  const uint32_t *flip, int64_t n, float r2min,
                                                                  float prec, float2 *out, const uint32_t *order,
-                                                                 int xcds, int hold_min)
+                                                                 int xcds, int hold_min, int wave_q)
 {
     using G = Geo<DIM>;
     using vec = typename G::vec;
     constexpr int BLOCK = 64;
     __shared__ SilShared sh;
     const int lane = threadIdx.x & 63;
-    const int64_t k = xcd_tile(xcds) * 64 + threadIdx.x;
-    const bool valid = k < n;
+    const int64_t k = xcd_tile(xcds) * wave_q + threadIdx.x;
+    const bool valid = (int)threadIdx.x < wave_q && k < n;
     const int64_t i = valid ? (order ? (int64_t)order[k] : k) : 0;
     float4 s4 = make_float4(0.0f, 0.0f, 0.0f, -1.0f);
     bool fl = false;
