@@ -91,6 +91,7 @@ struct fcpw_hip_ctx {
     int sil_hold_min = 3;                // the cooperative silhouette kernel's leaf-pass threshold
     int sil_xcds = 8;                    // the silhouette kernels' XCD grouping
     int inst_seed = 1024;                // instanced closest points: ordered queries per representative wave (0: off)
+    bool inst_seed_auto = true;          // not set by the caller: only batches that gain from it (launch_instances_closest)
     int stats_on = 0, timing = 0;
     int n_cus = 256;
     // device scratch of fcpw_hip_build_bvh, kept (grow-only) for the next build

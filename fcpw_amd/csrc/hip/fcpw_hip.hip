@@ -1634,6 +1634,7 @@ int fcpw_hip_set_option(fcpw_hip_ctx *c, const char *key, int value)
         if (value != 0 && (value < 64 || value > (1 << 20)))
             FAIL(c, FCPW_HIP_ERR_INVALID_ARGUMENT, "inst_seed must be 0 or in [64, 2^20]");
         c->inst_seed = value;
+        c->inst_seed_auto = false;
     } else if (k == "xcd_chunk") {
         if (value < 0 || value > 16) FAIL(c, FCPW_HIP_ERR_INVALID_ARGUMENT, "xcd_chunk must be in [0, 16]");
         c->xcd_chunk = value;

@@ -318,16 +318,16 @@ __global__ __launch_bounds__(64) void k_instances_closest_coop(DevScene T, const
                                                                const float4 *spheres, int64_t n, int record_normals,
                                                                float2 *out, int32_t *object_out,
                                                                const uint32_t *order, int xcds, int hold_min,
-                                                               int64_t n_all, int block, int pass)
+                                                               int64_t n_all, int block, int pass, int wave_q)
 {
     using G = Geo<DIM>;
     using vec = typename G::vec;
     constexpr int BLOCK = 64;
     __shared__ CoopShared sh;
     const int lane = threadIdx.x & 63;
-    const int64_t k = xcd_tile(xcds) * 64 + threadIdx.x;
+    const int64_t k = xcd_tile(xcds) * wave_q + threadIdx.x;
     int64_t pos;
-    const bool valid = seed_position(k, n, n_all, block, pass, pos);
+    const bool valid = lane < wave_q && seed_position(k, n, n_all, block, pass, pos);
     const int64_t i = valid ? (order ? (int64_t)order[pos] : pos) : 0;
     float q[3] = {0.0f, 0.0f, 0.0f};
     float r2 = -1.0f;
@@ -345,6 +345,7 @@ __global__ __launch_bounds__(64) void k_instances_closest_coop(DevScene T, const
     float cur_d2 = 0.0f;
     bool live = false, active = false, holding = false, start = false;
     bool inner = false;                              // walking an object's tree
+    bool disk = false;                               // whose disks hold for the mapped query
     uint32_t leaf_off = 0, leaf_cnt = 0, leaf_j = 0; // the instance leaf being visited
     int base = 0;
     // the instance being visited
@@ -399,6 +400,7 @@ __global__ __launch_bounds__(64) void k_instances_closest_coop(DevScene T, const
                 G::root(O, lo, hi, cur);
                 float d2min, d2max;
                 box_sqdist(lo, hi, xl, d2min, d2max);
+                disk = d2max <= *O.disk_limit; // false for a NaN
                 live = d2min <= r2l;
                 if (live) {
                     r2l = fminf(r2l, d2max);
@@ -433,7 +435,7 @@ __global__ __launch_bounds__(64) void k_instances_closest_coop(DevScene T, const
                             best_inst = ii;
                             best_slot = lbest;
                         }
-                        inner = false;
+                        inner = disk = false;
                         base = 0;
                         if (++leaf_j < leaf_cnt) start = true;
                         else if (n_inst == 1) active = false;
@@ -460,29 +462,47 @@ __global__ __launch_bounds__(64) void k_instances_closest_coop(DevScene T, const
                     vec loA, hiA, loB, hiB;
                     uint32_t lA, lB;
                     G::record(R, cur, loA, hiA, lA, loB, hiB, lB);
+                    float4 dA = make_float4(0.0f, 0.0f, 0.0f, 0.0f), dB = dA;
+                    if (disk) {
+                        const float4 *dk = O.disks + (size_t)cur * 2;
+                        dA = dk[0];
+                        dB = dk[1];
+                    }
                     float a0, a1, b0, b1;
                     box_sqdist(loA, hiA, xq, a0, a1);
-                    const bool oA = a0 <= rr;
+                    bool oA = a0 <= rr;
                     rr = fminf(rr, a1);
                     box_sqdist(loB, hiB, xq, b0, b1);
-                    const bool oB = b0 <= rr;
+                    bool oB = b0 <= rr;
                     rr = fminf(rr, b1);
+                    // an object's subtree beyond its disk is dropped, as in FCPW_COOP_STEP
+                    // (1M queries, 256 instances of 20,480 triangles, in two launches
+                    // with lowered radii: 12.0 -> 9.8 ms; in one: 8.6 ms)
+                    float cA = a0, cB = b0;
+                    if (oA && dA.w != 0.0f) {
+                        cA = fmaxf(a0, disk_bound(loA, hiA, xq, dA));
+                        oA = cA <= rr;
+                    }
+                    if (oB && dB.w != 0.0f) {
+                        cB = fmaxf(b0, disk_bound(loB, hiB, xq, dB));
+                        oB = cB <= rr;
+                    }
                     if (inner) r2l = rr;
                     else r2 = rr;
                     live = oA || oB;
                     if (oA && oB) {
                         uint32_t nearL = lA, farL = lB;
-                        float nearD = a0, farD = b0;
-                        if (b0 < a0) { nearL = lB; farL = lA; nearD = b0; farD = a0; }
+                        float nearD = cA, farD = cB;
+                        if (b0 < a0) { nearL = lB; farL = lA; nearD = cB; farD = cA; }
                         FCPW_PUSH(BLOCK, K, farL, farD, { overflow = true; active = false; live = false; });
                         cur = nearL;
                         cur_d2 = nearD;
                     } else if (oA) {
                         cur = lA;
-                        cur_d2 = a0;
+                        cur_d2 = cA;
                     } else if (oB) {
                         cur = lB;
-                        cur_d2 = b0;
+                        cur_d2 = cB;
                     }
                 }
             }
@@ -1260,18 +1280,24 @@ static int launch_instances_closest(fcpw_hip_ctx *c, const void *spheres, int64_
     if ((st = timing_begin(c, s))) return st;
     DevScene T = dev_scene(c);
     // with ordered queries and inst_seed = B: each block's representatives, then
-    // the rest with radii lowered from them (seeded_r2); otherwise one launch
-    const int block = order && c->inst_seed > 0 ? c->inst_seed : 0;
+    // the rest with radii lowered from them (seeded_r2); otherwise one launch.
+    // Two launches end twice with their longest walks (2.4 ms with 256 instances
+    // of 20,480 triangles, where one launch of 16,384 queries takes all of that),
+    // so unless the caller asked for it the batch has to be large: 1M queries
+    // there 8.6 ms in one launch against 9.8 in two, 4M 24.0 against 20.5.
+    const bool seed = c->inst_seed > 0 && (!c->inst_seed_auto || n >= ((int64_t)1 << 21));
+    const int block = order && seed ? c->inst_seed : 0;
     const bool coop = c->coop && c->max_depth + c->inst_obj_depth < STACK_TOTAL;
     for (int pass = block ? 0 : 1; pass < 2; pass++) {
         const int64_t m = pass == 0 ? (n + block - 1) / block * 64 : n;
         if (coop) {
             // one stack serves both levels, so the two trees' depths must fit it together
-            const dim3 g = grid_for(c, m, 64);
+            const int wq = wave_queries(c, m);
+            const dim3 g = grid_for(c, m, wq);
 #define FCPW_ICOOP(D, K)                                                                                       \
     hipLaunchKernelGGL((k_instances_closest_coop<D, K>), g, dim3(64), 0, s, T, c->inst, c->obj_table,          \
                        c->n_instances, (const float4 *)spheres, m, record_normals, (float2 *)out, object_out, \
-                       order, xcd_arg(c), c->hold_min, n, block, pass)
+                       order, xcd_arg(c), c->hold_min, n, block, pass, wq)
             if (c->dim == 3 && c->inst_stack == 8) FCPW_ICOOP(3, 8);
             else if (c->dim == 3) FCPW_ICOOP(3, INST_COOP_K3);
             else FCPW_ICOOP(2, INST_K);
