@@ -86,6 +86,11 @@ __device__ __forceinline__ float fmin_sq(float a, float b)
 {
     return __uint_as_float(min(__float_as_uint(a), __float_as_uint(b)));
 }
+// the larger of the same
+__device__ __forceinline__ float fmax_sq(float a, float b)
+{
+    return __uint_as_float(max(__float_as_uint(a), __float_as_uint(b)));
+}
 
 // ---------------------------------------------------------------------------
 // traversal stack: the NEWEST (up to) K entries live in LDS, lane-interleaved
@@ -102,6 +107,27 @@ __device__ __forceinline__ float fmin_sq(float a, float b)
 // ds_read/ds_write rather than generic (flat) loads.  K = 0 keeps every entry
 // in the spill array.
 // ---------------------------------------------------------------------------
+// i mod k for a stack index i < STACK_TOTAL = 64 (k <= 24): the quotient by a
+// multiplication of 24 bits.  The compiler's own i % 6 takes two or three
+// multiplications of 32 bits and more registers (48-mesh batch, whose kernel
+// spills to keep eight waves a SIMD, with fmax_sq and DISK_SHRINK: 1.64 -> 1.59
+// ms; the single-scene kernels the same, 16.25 ms for 16.8M on the torus).
+template <int K>
+__device__ __forceinline__ int stack_slot(int i)
+{
+    constexpr int k = K > 0 ? K : 1;
+    if constexpr ((k & (k - 1)) == 0) return i & (k - 1);
+    constexpr uint32_t m = (4096u + k - 1) / k; // floor(i m / 4096) = floor(i / k), checked below
+    constexpr bool exact = [] {
+        for (uint32_t j = 0; j < 64; j++)
+            if (j * m / 4096 != j / k) return false;
+        return true;
+    }();
+    static_assert(STACK_TOTAL <= 64 && exact, "stack_slot: the short quotient is not exact");
+    const int q = (int)(__umul24((uint32_t)i, m) >> 12);
+    return i + __mul24(q, -k);
+}
+
 #define FCPW_STACK_DECL(BLOCK, K)                                                                              \
     __shared__ uint64_t lds_stack[(K) > 0 ? (K) * (BLOCK) : 1];                                              \
     uint32_t stack_spill[2 * (STACK_TOTAL - (K))];                                                           \
@@ -123,7 +149,7 @@ __device__ __forceinline__ float fmin_sq(float a, float b)
             stack_spill[2 * sp] = l_;                                                                         \
             stack_spill[2 * sp + 1] = d_;                                                                     \
         } else {                                                                                              \
-            const int slot_ = (int)((uint32_t)sp % (uint32_t)((K) > 0 ? (K) : 1)) * (BLOCK) + stack_lane;    \
+            const int slot_ = stack_slot<K>(sp) * (BLOCK) + stack_lane;                                       \
             if (sp - stack_lo == (K)) {                                                                       \
                 const uint64_t old_ = lds_stack[slot_];                                                       \
                 stack_spill[2 * stack_lo] = (uint32_t)old_;                                                   \
@@ -139,7 +165,7 @@ __device__ __forceinline__ float fmin_sq(float a, float b)
     do {                                                                                                      \
         sp--;                                                                                                 \
         if ((K) > 0 && sp >= stack_lo) {                                                                     \
-            const uint64_t e_ = lds_stack[(int)((uint32_t)sp % (uint32_t)((K) > 0 ? (K) : 1)) * (BLOCK) + stack_lane]; \
+            const uint64_t e_ = lds_stack[stack_slot<K>(sp) * (BLOCK) + stack_lane];                          \
             (LINK) = (uint32_t)e_;                                                                            \
             (D) = __uint_as_float((uint32_t)(e_ >> 32));                                                      \
         } else {                                                                                              \
@@ -316,10 +342,12 @@ __device__ __forceinline__ void store_p(v2 p, float o[3]) { o[0] = p.x; o[1] = p
 // 16 bytes a slot: {n.x, n.y (f16)} {n.z (f16), o (bf16)} {t, rho (bf16)}
 // {0.5 / |n| (f32); 0: no disk}.  n is rounded first and o, t and rho are
 // measured about the rounded n, then rounded up.  The arithmetic is free to
-// fuse: l^2 is lowered by 4e-6 w.w and the bound by 1e-5 of itself, which
-// covers its rounding and that of the distances it is compared with.
+// fuse: l^2 is lowered by 4e-6 w.w and the bound by 1e-5 of itself (all lengths
+// are stored times DISK_SHRINK), which covers its rounding and that of the
+// distances it is compared with.
 // ---------------------------------------------------------------------------
 constexpr int DISK_MAX_PRIMS = 1024;
+constexpr double DISK_SHRINK = 1.0 - 5e-6; // all lengths of a disk carry this factor
 
 __device__ __forceinline__ float half_lo(float f)
 {
@@ -337,11 +365,11 @@ __device__ __forceinline__ float bf16_hi(float f) { return __uint_as_float(__flo
 __device__ __forceinline__ float disk_bound_of(float hw, float ww, float4 D)
 {
     const float h = hw * D.w;
-    const float l2 = __builtin_fmaf(-h, h, ww * (0.25f * (1.0f - 4e-6f)));
+    const float l2 = __builtin_fmaf(-h, h, ww * (float)(0.25 * (1.0 - 4e-6) * DISK_SHRINK * DISK_SHRINK));
     const float l = __builtin_amdgcn_sqrtf(fmaxf(l2, 0.0f));
     const float r = fmaxf(l - bf16_hi(D.z), 0.0f);
     const float g = fmaxf(fabsf(h - bf16_hi(D.y)) - bf16_lo(D.z), 0.0f);
-    return __builtin_fmaf(r, r, g * g) * (1.0f - 1e-5f);
+    return __builtin_fmaf(r, r, g * g);
 }
 __device__ __forceinline__ float disk_bound(v3 lo, v3 hi, v3 x, float4 D)
 {
@@ -788,11 +816,11 @@ __device__ __forceinline__ void coop_begin(const DevScene &S, CoopShared &sh, Co
                 float cA_ = a0, cB_ = b0;                                                                     \
                 if (DISK) {                                                                                   \
                     if (oA && dA_.w != 0.0f) {                                                                \
-                        cA_ = fmaxf(a0, disk_bound(loA, hiA, (L).x, dA_));                                    \
+                        cA_ = fmax_sq(a0, disk_bound(loA, hiA, (L).x, dA_));                                  \
                         oA = cA_ <= (L).r2;                                                                   \
                     }                                                                                         \
                     if (oB && dB_.w != 0.0f) {                                                                \
-                        cB_ = fmaxf(b0, disk_bound(loB, hiB, (L).x, dB_));                                    \
+                        cB_ = fmax_sq(b0, disk_bound(loB, hiB, (L).x, dB_));                                  \
                         oB = cB_ <= (L).r2;                                                                   \
                     }                                                                                         \
                 }                                                                                             \
@@ -1911,8 +1939,9 @@ __device__ __forceinline__ void disk_round_normal(v3 s, v3 &n, uint32_t &nxy, ui
 __device__ __forceinline__ float4 disk_pack(const DiskSums &D, v3 half, v3 n, uint32_t nxy, uint32_t nz, float inv,
                                             float scale)
 {
-    const float o = __uint_as_float(__float_as_uint(0.5f * (D.lo + D.hi)) & 0xFFFF0000u);
-    const float t0 = fmaxf(D.hi - o, o - D.lo), r0 = sqrtf(D.l2);
+    const float lo = (float)DISK_SHRINK * D.lo, hi = (float)DISK_SHRINK * D.hi;
+    const float o = __uint_as_float(__float_as_uint(0.5f * (lo + hi)) & 0xFFFF0000u);
+    const float t0 = fmaxf(hi - o, o - lo), r0 = (float)DISK_SHRINK * sqrtf(D.l2);
     // 1e-6 of the coordinates: rounding of the closest points and of this
     // kernel; 8e-6 of the disk itself: rounding of the bound near the disk
     const float pad = 1e-6f * scale + 8e-6f * (t0 + r0);
@@ -1924,7 +1953,7 @@ __device__ __forceinline__ float4 disk_pack(const DiskSums &D, v3 half, v3 n, ui
     const float width = fabsf(n.x) * half.x + fabsf(n.y) * half.y + fabsf(n.z) * half.z;
     if (!(t < 0.6f * width)) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     return make_float4(__uint_as_float(nxy), __uint_as_float(nz | __float_as_uint(o)),
-                       __uint_as_float(bf16_up(t) | (bf16_up(r) << 16)), 0.5f * inv);
+                       __uint_as_float(bf16_up(t) | (bf16_up(r) << 16)), (float)(0.5 * DISK_SHRINK) * inv);
 }
 
 // The disks of all slots, shared out as in k_refit_ranges: two passes over a
