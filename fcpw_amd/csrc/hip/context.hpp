@@ -42,6 +42,8 @@ struct fcpw_hip_ctx {
     unsigned long long *stats = nullptr; // internal nodes, primitive tests, queries (option "stats")
     // silhouettes (fcpw_hip_upload_silhouettes): cones per child slot and root, leaf ranges, records
     float4 *cones = nullptr, *sils = nullptr;
+    float4 *sil_faces = nullptr; // facing entries per child slot, valid while by_range
+    int sil_unit = 0;            // no record has a normal longer than one
     uint2 *sil_leaf = nullptr;
     bool has_silhouettes = false;
     int n_sil_refs = 0;
@@ -87,6 +89,7 @@ struct fcpw_hip_ctx {
     int ray_sort_dir = 1; // rays ordered by direction octant, then origin
     int ray_stack = 4, ray_hold_min = 8; // the cooperative ray kernels' LDS stack entries and leaf-pass threshold
     int sil_stack = 4, inst_stack = 12;  // LDS stack entries of the 3D cooperative silhouette and instance kernels
+    bool sil_stack_auto = true;          // sil_stack not set by the caller: eight (launch_silhouettes)
     int layout = 0;                      // record order in memory: 0 DFS, 1 treelets of three levels
     int sil_hold_min = 3;                // the cooperative silhouette kernel's leaf-pass threshold
     int sil_xcds = 8;                    // the silhouette kernels' XCD grouping
@@ -125,11 +128,12 @@ static std::string g_create_error;
 
 static void free_silhouettes(fcpw_hip_ctx *c)
 {
-    void *bufs[] = {c->cones, c->sils, c->sil_leaf};
+    void *bufs[] = {c->cones, c->sils, c->sil_leaf, c->sil_faces};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     c->cones = c->sils = nullptr;
     c->sil_leaf = nullptr;
+    c->sil_faces = nullptr;
     c->has_silhouettes = false;
     c->n_sil_refs = 0;
     c->sil_leaf_max = 0;

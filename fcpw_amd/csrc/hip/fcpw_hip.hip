@@ -82,6 +82,20 @@ static int launch_disks(fcpw_hip_ctx *c, hipStream_t s)
     return FCPW_HIP_OK;
 }
 
+// the facing entries of the silhouette queries, from the boxes, ranges and silhouette records
+static int launch_faces(fcpw_hip_ctx *c, hipStream_t s)
+{
+    if (!c->by_range || !c->sil_faces) return FCPW_HIP_OK;
+    if (c->dim == 3)
+        hipLaunchKernelGGL(k_build_faces<3>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->ranges,
+                           2 * c->n_records, c->big, c->n_big, slot_own_blocks(c), c->sil_leaf, c->sils, c->sil_faces);
+    else
+        hipLaunchKernelGGL(k_build_faces<2>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->ranges,
+                           2 * c->n_records, c->big, c->n_big, slot_own_blocks(c), c->sil_leaf, c->sils, c->sil_faces);
+    HIPCHECK(c, hipGetLastError());
+    return FCPW_HIP_OK;
+}
+
 // ranges, slot lists and disks of a tree whose slots were (re)numbered
 template <int DIM>
 static int compute_ranges(fcpw_hip_ctx *c)
@@ -675,7 +689,8 @@ static int relayout_records(fcpw_hip_ctx *c, int layout)
         HIPCHECK(c, hipMemcpy(c->cones, cones2.data(), cones2.size() * sizeof(float4), hipMemcpyHostToDevice));
     }
     if (c->range_mem) {
-        const int st = compute_ranges(c);
+        int st = compute_ranges(c);
+        if (!st) st = launch_faces(c, 0);
         if (st) return st;
     }
     HIPCHECK(c, hipDeviceSynchronize());
@@ -842,18 +857,22 @@ int fcpw_hip_upload_silhouettes(fcpw_hip_ctx *c, int n_nodes, const fcpw_hip_bou
     }
     const int RW = c->dim == 3 ? 4 : 2;
     std::vector<float4> rec_buf((size_t)std::max(n_refs, 1) * RW, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+    bool unit = true;
+    const auto at_most_one = [](const fcpw_hip_float3 &n) { return n.x * n.x + n.y * n.y + n.z * n.z < 1.0002f; };
     for (int r = 0; r < n_refs; r++) {
         if (c->dim == 2) {
             const fcpw_hip_vertex &v = ((const fcpw_hip_vertex *)silhouettes)[r];
             rec_buf[(size_t)r * 2] = make_float4(v.p.x, v.p.y, v.n0.x, v.n0.y);
             rec_buf[(size_t)r * 2 + 1] =
                 make_float4(v.n1.x, v.n1.y, bits_as_float(v.index), bits_as_float(v.has_one_adjacent_face));
+            unit = unit && at_most_one(v.n0) && at_most_one(v.n1);
         } else {
             const fcpw_hip_edge &e = ((const fcpw_hip_edge *)silhouettes)[r];
             rec_buf[(size_t)r * 4] = make_float4(e.pa.x, e.pa.y, e.pa.z, bits_as_float(e.index));
             rec_buf[(size_t)r * 4 + 1] = make_float4(e.pb.x, e.pb.y, e.pb.z, bits_as_float(e.has_one_adjacent_face));
             rec_buf[(size_t)r * 4 + 2] = make_float4(e.n0.x, e.n0.y, e.n0.z, 0.0f);
             rec_buf[(size_t)r * 4 + 3] = make_float4(e.n1.x, e.n1.y, e.n1.z, 0.0f);
+            unit = unit && at_most_one(e.n0) && at_most_one(e.n1);
         }
     }
     HIPCHECK(c, hipSetDevice(c->device));
@@ -867,6 +886,12 @@ int fcpw_hip_upload_silhouettes(fcpw_hip_ctx *c, int n_nodes, const fcpw_hip_bou
     HIPCHECK(c, hipMemcpy(c->sils, rec_buf.data(), rec_buf.size() * sizeof(float4), hipMemcpyHostToDevice));
     c->n_sil_refs = n_refs;
     c->sil_leaf_max = leaf_max;
+    c->sil_unit = unit ? 1 : 0;
+    if (c->by_range) {
+        HIPCHECK(c, hipMalloc((void **)&c->sil_faces, (size_t)2 * c->n_records * sizeof(float4)));
+        if ((st = launch_faces(c, 0))) return st;
+        HIPCHECK(c, hipDeviceSynchronize());
+    }
     c->has_silhouettes = true;
     return FCPW_HIP_OK;
 }
@@ -947,6 +972,7 @@ int fcpw_hip_refit(fcpw_hip_ctx *c, void *stream)
     HIPCHECK(c, hipGetLastError());
     if ((st = launch_disks(c, s))) return st;
     if (c->has_silhouettes) {
+        if ((st = launch_faces(c, s))) return st;
         if (c->dim == 3)
             hipLaunchKernelGGL(k_refit_cones<3>, dim3(blocks), dim3(threads), 0, s, c->records, c->root, c->cones,
                                c->sil_leaf, c->sils, c->leaf_refs, c->leaf_links, c->rec_parent, c->counters,
@@ -1439,7 +1465,7 @@ static int launch_silhouettes(fcpw_hip_ctx *c, const void *spheres, const uint32
                               float prec, void *out, hipStream_t s)
 {
     DevScene S = dev_scene(c);
-    SilScene T = {c->cones, c->sil_leaf, c->sils};
+    SilScene T = {c->cones, c->sil_leaf, c->sils, c->by_range ? c->sil_faces : nullptr, c->sil_unit};
     const uint32_t *order = nullptr;
     int st = morton_order(c, (const float *)spheres, 4, n, s, &order);
     if (st) return st;
@@ -1450,12 +1476,18 @@ static int launch_silhouettes(fcpw_hip_ctx *c, const void *spheres, const uint32
         // record indices within a leaf travel in 10 bits of a leaf-pass item
         const int wq = wave_queries(c, n);
         const dim3 g = grid_for(c, n, wq);
+        // Eight LDS entries unless the caller set the option.  Four, which keep eight
+        // waves a SIMD, were the faster before subtrees were dropped by their facing
+        // entries; now the spills of four cost more: 262,144 queries on 131,072
+        // triangles 13.0 ms with four and 11.0 with eight, 1M 21.6 and 17.9, 4.2M on
+        // a million triangles 164 and 133, 30,000 on 20,000 triangles 3.2 and 2.8.
+        const int k = c->sil_stack_auto ? 8 : c->sil_stack;
 #define FCPW_SIL3(K)                                                                                          \
     hipLaunchKernelGGL((k_closest_silhouettes_coop<3, K>), g, dim3(64), 0, s, S, T, (const float4 *)spheres, flip, n, \
                        r2min, prec, (float2 *)out, order, sil_xcd_arg(c), c->sil_hold_min, wq)
         if (c->dim == 3) {
-            if (c->sil_stack == 8) FCPW_SIL3(8);
-            else if (c->sil_stack == 12) FCPW_SIL3(12);
+            if (k == 8) FCPW_SIL3(8);
+            else if (k == 12) FCPW_SIL3(12);
             else FCPW_SIL3(SIL_COOP_K3);
         } else
 #undef FCPW_SIL3
@@ -1595,6 +1627,7 @@ int fcpw_hip_set_option(fcpw_hip_ctx *c, const char *key, int value)
         if (k == "sil_stack" ? (value != 4 && value != 8 && value != 12) : (value != 8 && value != 12))
             FAIL(c, FCPW_HIP_ERR_INVALID_ARGUMENT, "%s must be %s", key, k == "sil_stack" ? "4, 8 or 12" : "8 or 12");
         (k == "sil_stack" ? c->sil_stack : c->inst_stack) = value;
+        if (k == "sil_stack") c->sil_stack_auto = false;
     } else if (k == "bwd_order" || k == "bwd_reduce") {
         if (value != 0 && value != 1 && !(k == "bwd_reduce" && value == 2))
             FAIL(c, FCPW_HIP_ERR_INVALID_ARGUMENT, "%s must be 0 or 1%s", key, k == "bwd_reduce" ? " or 2" : "");

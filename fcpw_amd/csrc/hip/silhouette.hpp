@@ -26,6 +26,8 @@ struct SilScene {
     const float4 *cones;
     const uint2 *sil_leaf;
     const float4 *sils;
+    const float4 *faces; // facing entries of the child slots (faces_away), or null
+    int unit;            // no record has a normal longer than one (certainly_off needs it)
 };
 
 constexpr float PI_F = 3.14159265358979323846f;   // M_PI (math-constants.slang)
@@ -259,6 +261,60 @@ __device__ __forceinline__ bool silhouette_test(const SilRecord &s, v3 x, float 
     return process && d * d <= r2;
 }
 
+// ---------------------------------------------------------------------------
+// Facing entries.  A record is off the silhouette when x lies in front of both
+// of its faces, or behind both.  The cone test decides that for a subtree with
+// the subtree's whole radius as the play of its faces' planes; on a surface that
+// is flat but for noise the planes pass within a fraction of it.  So each child
+// slot of at most DISK_MAX_PRIMS primitives also carries, about its box centre c,
+// an axis a, the tangent T of the angle that holds all its face normals n, and
+// the extreme plane offsets n.(p - c) over both ends p of its records, divided by
+// that angle's cosine: F in front, B behind (both >= 0).  With w = x - c, h = a.w,
+// l^2 = w.w - h^2, every record's n.(x - p) is beyond the margin m when
+//   |h| - l T - m > (h >= 0 ? F : B),
+// and such a subtree is dropped before its cone test: its records accept nothing,
+// and the order of the remaining visits is the reference's.  m covers
+//   - the classification's own precision: it wants |n.(x - p)| > prec |x - p| and
+//     |x - p| > prec (an edge closer than that goes by its dihedral angle);
+//     |x - p| <= |h| + l + R with R the largest |p - c|, and 1 + T >= 1 / cosine;
+//   - rounding, here and in the reference's evaluation: 1e-5 of the lengths, and
+//     4e-6 of the coordinates, which F and B hold already.
+// Subtrees with boundary edges, faces without a normal or angles above 60 degrees
+// have none (T infinite).  Visits on the 131,072-triangle torus, 262,144 queries:
+// 281 expanded records and 638 record tests a query without, 176 and 332 with.
+//
+// 16 bytes a slot: {a.x, a.y (f16)} {a.z (f16), T (bf16)} {B, F (bf16)}
+// {1 / |a| - 1, R (bf16)}
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ bool faces_away(float4 D, v3 x, v3 lo, v3 hi, float prec)
+{
+    const v3 w = {x.x - 0.5f * (lo.x + hi.x), x.y - 0.5f * (lo.y + hi.y), x.z - 0.5f * (lo.z + hi.z)};
+    const float hw = __builtin_fmaf(w.z, half_lo(D.y), __builtin_fmaf(w.y, half_hi(D.x), w.x * half_lo(D.x)));
+    const float ww = __builtin_fmaf(w.z, w.z, __builtin_fmaf(w.y, w.y, w.x * w.x));
+    const float h = __builtin_fmaf(hw, bf16_lo(D.w), hw), T = bf16_hi(D.y);
+    const float l = __builtin_amdgcn_sqrtf(fmaxf(__builtin_fmaf(-h, h, ww * (1.0f + 1.2e-5f)), 0.0f));
+    const float reach = fabsf(h) + l + bf16_hi(D.w);
+    const float m = __builtin_fmaf((1.0f + T) * prec, fmaxf(1.0f, reach), 1e-5f * reach);
+    return fabsf(h) - __builtin_fmaf(l, T, m) > (h >= 0.0f ? bf16_hi(D.z) : bf16_lo(D.z));
+}
+
+// The same for one record: x beyond the margin on one side of both face planes at
+// both ends, hence all along the edge (4 dot products; the classification with its
+// closest point takes four divisions and two square roots).
+template <int DIM>
+__device__ __forceinline__ bool certainly_off(const SilRecord &s, v3 x, float prec)
+{
+    const v3 va = sub(x, s.pa), vb = DIM == 3 ? sub(x, s.pb) : va;
+    const float a0 = dot(s.n0, va), a1 = dot(s.n1, va);
+    const float b0 = DIM == 3 ? dot(s.n0, vb) : a0, b1 = DIM == 3 ? dot(s.n1, vb) : a1;
+    const float mn = fminf(fminf(a0, a1), fminf(b0, b1)), mx = fmaxf(fmaxf(a0, a1), fmaxf(b0, b1));
+    const float dm = __builtin_amdgcn_sqrtf(DIM == 3 ? fmaxf(dot(va, va), dot(vb, vb)) : dot(va, va)) * 1.00001f;
+    float c = fmaxf(fmaxf(fabsf(s.pa.x), fabsf(s.pa.y)), fabsf(s.pa.z));
+    if (DIM == 3) c = fmaxf(c, fmaxf(fmaxf(fabsf(s.pb.x), fabsf(s.pb.y)), fabsf(s.pb.z)));
+    const float m = prec * fmaxf(1.0f, dm) * 1.0001f + 4e-6f * (c + dm);
+    return s.one != 1u && (mn > m || mx < -m);
+}
+
 // The distance of a silhouette record to x when the record is on the silhouette
 // seen from x, NaN otherwise: silhouette_test without its radius checks, which
 // a NaN fails as the test's own rejection does.
@@ -280,7 +336,8 @@ __device__ __forceinline__ float silhouette_distance(const SilRecord &s, v3 x, b
 template <int DIM, bool BOUNDED>
 __device__ __forceinline__ void silhouette_children(const DevScene &S, const SilScene &T, uint32_t cur, v3 x,
                                                     typename Geo<DIM>::vec xb, float r2, bool &oA, bool &oB,
-                                                    float &a0, float &b0, uint32_t &lA, uint32_t &lB)
+                                                    float &a0, float &b0, uint32_t &lA, uint32_t &lB,
+                                                    float face_prec = 0.0f)
 {
     using G = Geo<DIM>;
     using vec = typename G::vec;
@@ -288,6 +345,12 @@ __device__ __forceinline__ void silhouette_children(const DevScene &S, const Sil
     G::record(S, cur, loA, hiA, lA, loB, hiB, lB);
     const float4 *cp = T.cones + (size_t)cur * 4;
     const float4 cA = cp[0], rA = cp[1], cB = cp[2], rB = cp[3];
+    const float none = __builtin_inff();
+    float4 fA = make_float4(0.0f, none, 0.0f, 0.0f), fB = fA;
+    if (BOUNDED && T.faces) {
+        fA = T.faces[(size_t)cur * 2];
+        fB = T.faces[(size_t)cur * 2 + 1];
+    }
     float unused;
     a0 = 0.0f;
     b0 = 0.0f;
@@ -295,6 +358,7 @@ __device__ __forceinline__ void silhouette_children(const DevScene &S, const Sil
     if (oA) {
         box_sqdist(loA, hiA, xb, a0, unused);
         oA = a0 <= r2;
+        if (BOUNDED && oA) oA = !faces_away(fA, x, to3(loA), to3(hiA), face_prec);
         if (oA) oA = BOUNDED ? cone_overlap_bounded(cA, rA, x, to3(loA), to3(hiA), a0)
                              : cone_overlap(cA, rA.x, x, to3(loA), to3(hiA), a0);
     }
@@ -302,6 +366,7 @@ __device__ __forceinline__ void silhouette_children(const DevScene &S, const Sil
     if (oB) {
         box_sqdist(loB, hiB, xb, b0, unused);
         oB = b0 <= r2;
+        if (BOUNDED && oB) oB = !faces_away(fB, x, to3(loB), to3(hiB), face_prec);
         if (oB) oB = BOUNDED ? cone_overlap_bounded(cB, rB, x, to3(loB), to3(hiB), b0)
                              : cone_overlap(cB, rB.x, x, to3(loB), to3(hiB), b0);
     }
@@ -409,6 +474,7 @@ struct SilShared {
     uint16_t item[256];
     float d[256];
     uint32_t index[256];
+    uint8_t left[256]; // the pairs that certainly_off does not decide
 };
 
 template <int DIM, int K>
@@ -445,6 +511,7 @@ __global__ __launch_bounds__(64) FCPW_EIGHT_WAVES void k_closest_silhouettes_coo
         box_sqdist(lo, hi, xb, cur_d2, unused);
     }
     bool active = valid && !(r2min >= r2) && cur_d2 <= r2, live = active, holding = false, overflow = false;
+    const float face_prec = fmaxf(prec, 0.0f); // 0 for a NaN, with which every comparison fails
     FCPW_STACK_DECL(BLOCK, K);
     __syncthreads();
     while (true) {
@@ -469,7 +536,7 @@ __global__ __launch_bounds__(64) FCPW_EIGHT_WAVES void k_closest_silhouettes_coo
                 uint32_t lA, lB;
                 float a0, b0;
                 bool oA, oB;
-                silhouette_children<DIM, true>(S, T, cur, x, xb, r2, oA, oB, a0, b0, lA, lB);
+                silhouette_children<DIM, true>(S, T, cur, x, xb, r2, oA, oB, a0, b0, lA, lB, face_prec);
                 live = oA || oB;
                 if (oA && oB) {
                     uint32_t nearL = lA, farL = lB;
@@ -506,19 +573,38 @@ __global__ __launch_bounds__(64) FCPW_EIGHT_WAVES void k_closest_silhouettes_coo
             if (h2) sh.item[i2] = (uint16_t)((lane << 10) | (j0 + 2));
             if (h3) sh.item[i3] = (uint16_t)((lane << 10) | (j0 + 3));
             __syncthreads();
+            uint32_t n_left = 0;
             for (uint32_t pass = 0; pass < total; pass += 64) {
                 const uint32_t kk = pass + (uint32_t)lane;
                 // every lane takes part in the permutes; lanes past the end read item 0
                 const uint32_t it = sh.item[kk < total ? kk : 0u];
                 const int src = (int)(it >> 10);
                 const v3 xo = {__shfl(x.x, src, 64), __shfl(x.y, src, 64), DIM == 3 ? __shfl(x.z, src, 64) : 0.0f};
+                const uint32_t off = __shfl(loff, src, 64);
+                bool maybe = kk < total;
+                if (maybe) {
+                    const SilRecord rec = load_silhouette<DIM>(T.sils, off + (it & 1023u));
+                    sh.index[kk] = rec.index;
+                    if (T.unit && certainly_off<DIM>(rec, xo, face_prec)) {
+                        sh.d[kk] = __builtin_nanf("");
+                        maybe = false;
+                    }
+                }
+                const uint64_t mb = __ballot(maybe);
+                if (maybe) sh.left[n_left + lanes_below(mb)] = (uint8_t)kk;
+                n_left += __popcll(mb);
+            }
+            __syncthreads();
+            // what certainly_off leaves: about one record in five
+            for (uint32_t pass = 0; pass < n_left; pass += 64) {
+                const bool on = pass + (uint32_t)lane < n_left;
+                const uint32_t kk = sh.left[on ? pass + (uint32_t)lane : 0u], it = sh.item[kk];
+                const int src = (int)(it >> 10);
+                const v3 xo = {__shfl(x.x, src, 64), __shfl(x.y, src, 64), DIM == 3 ? __shfl(x.z, src, 64) : 0.0f};
                 const bool fo = __shfl(flu, src, 64) != 0u;
                 const uint32_t off = __shfl(loff, src, 64);
-                if (kk < total) {
-                    const SilRecord rec = load_silhouette<DIM>(T.sils, off + (it & 1023u));
-                    sh.d[kk] = silhouette_distance<DIM>(rec, xo, fo, prec);
-                    sh.index[kk] = rec.index;
-                }
+                if (on)
+                    sh.d[kk] = silhouette_distance<DIM>(load_silhouette<DIM>(T.sils, off + (it & 1023u)), xo, fo, prec);
             }
             __syncthreads();
             if (holding) {
@@ -555,6 +641,101 @@ __global__ __launch_bounds__(64) FCPW_EIGHT_WAVES void k_closest_silhouettes_coo
         uv[0] = t;
     }
     write_interaction(out + i * 5, p3, nz, uv, d, best);
+}
+
+// The facing entries of all slots (faces_away), from the records of the leaves
+// below each: slots shared out as in k_build_disks, a leaf's records listed at
+// its first primitive.
+template <int DIM>
+__global__ __launch_bounds__(DISK_BLOCK) void k_build_faces(const float4 *records, const int2 *ranges, int n_slots,
+                                                            const int *big, int n_big, int own_blocks,
+                                                            const uint2 *sil_leaf, const float4 *sils, float4 *faces)
+{
+    const bool own = (int)blockIdx.x < own_blocks;
+    int slot, step = 1, first = 0;
+    if (own) {
+        slot = (int)blockIdx.x * DISK_BLOCK + (int)threadIdx.x;
+        if (slot >= n_slots) return;
+    } else {
+        const int w = ((int)blockIdx.x - own_blocks) * (DISK_BLOCK / 64) + (int)(threadIdx.x >> 6);
+        if (w >= n_big) return;
+        slot = big[w];
+        first = (int)(threadIdx.x & 63u);
+        step = 64;
+    }
+    const int2 rg = ranges[slot];
+    const float4 none = make_float4(0.0f, INFINITY, 0.0f, 0.0f);
+    if (own && rg.y > DISK_OWN) {
+        if (rg.y > DISK_MAX_PRIMS) faces[slot] = none;
+        return;
+    }
+    v3 lo, hi;
+    load_slot_box<DIM>(records, slot, lo, hi);
+    const v3 c = {0.5f * (lo.x + hi.x), 0.5f * (lo.y + hi.y), 0.5f * (lo.z + hi.z)};
+    v3 sum = {0.0f, 0.0f, 0.0f};
+    bool bad = false;
+    for (int k = first; k < rg.y; k += step) {
+        const uint2 leaf = sil_leaf[rg.x + k];
+        for (uint32_t j = 0; j < leaf.y; j++) {
+            const SilRecord r = load_silhouette<DIM>(sils, leaf.x + j);
+            sum = {sum.x + r.n0.x + r.n1.x, sum.y + r.n0.y + r.n1.y, sum.z + r.n0.z + r.n1.z};
+            bad = bad || r.one == 1u;
+        }
+    }
+    if (!own)
+        for (int off = 32; off > 0; off >>= 1) {
+            sum.x += __shfl_xor(sum.x, off, 64);
+            sum.y += __shfl_xor(sum.y, off, 64);
+            sum.z += __shfl_xor(sum.z, off, 64);
+        }
+    v3 a;
+    uint32_t axy, az;
+    float inv;
+    disk_round_normal(sum, a, axy, az, inv);
+    float cosine = 1.0f, front = 0.0f, back = 0.0f, far2 = 0.0f, coord = 0.0f;
+    for (int k = first; k < rg.y; k += step) {
+        const uint2 leaf = sil_leaf[rg.x + k];
+        for (uint32_t j = 0; j < leaf.y; j++) {
+            const SilRecord r = load_silhouette<DIM>(sils, leaf.x + j);
+            for (int f = 0; f < 2; f++) {
+                const v3 n = f ? r.n1 : r.n0;
+                const float nn = dot(n, n);
+                bad = bad || !(nn > 0.99999f && nn < 1.00001f);
+                cosine = fminf(cosine, dot(n, a));
+                for (int e = 0; e < (DIM == 3 ? 2 : 1); e++) {
+                    const v3 p = e ? r.pb : r.pa, w = sub(p, c);
+                    const float o = dot(n, w);
+                    bad = bad || !(fabsf(o) < 1e18f);
+                    front = fmaxf(front, o);
+                    back = fmaxf(back, -o);
+                    far2 = fmaxf(far2, dot(w, w));
+                    coord = fmaxf(coord, fmaxf(fmaxf(fabsf(p.x), fabsf(p.y)), fabsf(p.z)));
+                }
+            }
+        }
+    }
+    if (!own) {
+        for (int off = 32; off > 0; off >>= 1) {
+            cosine = fminf(cosine, __shfl_xor(cosine, off, 64));
+            front = fmaxf(front, __shfl_xor(front, off, 64));
+            back = fmaxf(back, __shfl_xor(back, off, 64));
+            far2 = fmaxf(far2, __shfl_xor(far2, off, 64));
+            coord = fmaxf(coord, __shfl_xor(coord, off, 64));
+        }
+        bad = __ballot(bad) != 0;
+        if (first != 0) return;
+    }
+    cosine -= 2e-5f; // the axis and the normals are unit to 5e-6
+    if (bad || !(cosine >= 0.5f)) {
+        faces[slot] = none;
+        return;
+    }
+    const float tangent = sqrtf(fmaxf(1.0f - cosine * cosine, 0.0f)) / cosine * (1.0f + 1e-5f);
+    const float R = sqrtf(far2) * (1.0f + 1e-5f), pad = 8e-6f * (coord + R);
+    const float delta = inv - 1.0f;
+    faces[slot] = make_float4(__uint_as_float(axy), __uint_as_float(az | (bf16_up(tangent) << 16)),
+                              __uint_as_float(bf16_up(back / cosine + pad) | (bf16_up(front / cosine + pad) << 16)),
+                              __uint_as_float((__float_as_uint(delta) >> 16) | (bf16_up(R) << 16)));
 }
 
 // ---------------------------------------------------------------------------
