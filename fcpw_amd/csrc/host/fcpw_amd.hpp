@@ -12,6 +12,9 @@
 //    shader source is compiled at run time.
 #pragma once
 
+#include <sched.h>
+
+#include <algorithm>
 #include <chrono>
 #include <cstdio>
 #include <cstdlib>
@@ -87,19 +90,40 @@ inline CostHeuristic heuristic_of(AggregateType t)
     }
 }
 
-// static partition over hardware threads, as the reference's batched helpers
-// (fcpw.inl:1547-1559)
-template <typename F>
-inline void parallel_rows(int64_t n, F &&f)
+// threads of the row-parallel helpers: the CPUs this process may run on, at most
+// 16 (a container's share can be far below the machine's count)
+inline int row_threads()
 {
-    int nt = (int)std::thread::hardware_concurrency();
-    if (nt < 1 || n < 65536) { f((int64_t)0, n); return; }
+    static const int n = [] {
+        int k = 0;
+        cpu_set_t set;
+        if (sched_getaffinity(0, sizeof(set), &set) == 0) k = CPU_COUNT(&set);
+        if (k < 1) k = (int)std::thread::hardware_concurrency();
+        return std::max(1, std::min(k, 16));
+    }();
+    return n;
+}
+
+// static partition over threads, as the reference's batched helpers
+// (fcpw.inl:1547-1559); the caller takes the first share, and any share that
+// finds no thread.  At least `grain` rows a thread: starting one costs about as
+// much as copying 32,768 records.
+template <typename F>
+inline void parallel_rows(int64_t n, F &&f, int64_t grain = 32768)
+{
+    const int nt = (int)std::min<int64_t>(row_threads(), n / grain);
+    if (nt < 2) { f((int64_t)0, n); return; }
     std::vector<std::thread> th;
-    int64_t per = n / nt;
-    for (int i = 0; i < nt; i++) {
-        int64_t s = i * per, e = (i == nt - 1) ? n : (i + 1) * per;
-        th.emplace_back([&f, s, e]() { f(s, e); });
+    const int64_t per = n / nt;
+    const auto share = [&f, per, n, nt](int i) { f(i * per, i == nt - 1 ? n : (i + 1) * per); };
+    int started = 1;
+    try {
+        th.reserve((size_t)nt);
+        for (; started < nt; started++) th.emplace_back(share, started);
+    } catch (...) {
     }
+    for (int i = started; i < nt; i++) share(i);
+    share(0);
     for (auto &t : th) t.join();
 }
 

@@ -370,7 +370,7 @@ SnchData<DIM> build_snch(const FlatBvh<DIM> &bvh, const float *positions, int n_
                 }
             }
         }
-    });
+    }, 4096); // a row walks its whole subtree
     return S;
 }
 

@@ -472,8 +472,11 @@ static py::array_t<float> gather(const InteractionList &v, size_t field_offset)
     py::array_t<float> out(W == 1 ? std::vector<py::ssize_t>{(py::ssize_t)v.size()}
                                   : std::vector<py::ssize_t>{(py::ssize_t)v.size(), (py::ssize_t)W});
     float *o = out.mutable_data();
-    for (size_t i = 0; i < v.size(); i++)
-        std::memcpy(o + i * W, reinterpret_cast<const char *>(&v[i]) + field_offset, W * sizeof(float));
+    // bound by the page faults of the new array: 1M records 1.0-1.25 ms a field on one thread
+    parallel_rows((int64_t)v.size(), [&](int64_t s, int64_t e) {
+        for (int64_t i = s; i < e; i++)
+            std::memcpy(o + i * W, reinterpret_cast<const char *>(&v[i]) + field_offset, W * sizeof(float));
+    });
     return out;
 }
 
@@ -545,7 +548,9 @@ PYBIND11_MODULE(_fcpw_amd, m)
         [](const InteractionList &v) {
             py::array_t<uint32_t> out((py::ssize_t)v.size());
             uint32_t *o = out.mutable_data();
-            for (size_t i = 0; i < v.size(); i++) o[i] = v[i].index;
+            parallel_rows((int64_t)v.size(), [&](int64_t s, int64_t e) {
+                for (int64_t i = s; i < e; i++) o[i] = v[i].index;
+            });
             return out;
         },
         "Extract all primitive indices as a NumPy array");
