@@ -87,6 +87,7 @@ struct fcpw_hip_ctx {
     int xcd_chunk = 0; // log2 tiles per XCD chunk of the tile mapping (0: one range per XCD)
     int ray_coop = 1; // wave-cooperative leaves for ray queries
     int ray_sort_dir = 1; // rays ordered by direction octant, then origin
+    bool stack_auto = true; // stack not set by the caller: by the batch size (launch_closest_kernel)
     int ray_stack = 4, ray_hold_min = 8; // the cooperative ray kernels' LDS stack entries and leaf-pass threshold
     int sil_stack = 4, inst_stack = 12;  // LDS stack entries of the 3D cooperative silhouette and instance kernels
     bool sil_stack_auto = true;          // sil_stack not set by the caller: eight (launch_silhouettes)
