@@ -396,7 +396,9 @@ int fcpw_hip_batch_get_option(const fcpw_hip_batch *batch, const char *key, int 
                  distance between the two queries, with margins), which never
                  changes a record; B = 1024 by default, 64..2^20, 0 = one launch
                  Until the option is set, batches below 2^21 queries run as one
-                 launch, which is then the faster form
+                 launch, which is then the faster form.  Likewise
+                 "stack" and "sil_stack": until set, closest points in batches of at
+                 most 16 waves a CU take twelve entries, and silhouettes eight
      "bwd_order" 1 = the adjoint walks the queries in the Morton order the latest
                  query call on this context computed, when that batch had the same
                  size (default); 0 = in the caller's order
