@@ -1664,10 +1664,91 @@ __device__ __forceinline__ int subtree_edge(const float4 *records, uint32_t link
 }
 
 template <int DIM>
-__global__ void k_slot_ranges(const float4 *records, int n_records, int2 *ranges, int *info)
+__device__ __forceinline__ void load_slot_box(const float4 *records, int slot, v3 &lo, v3 &hi)
+{
+    if (DIM == 3) {
+        const float4 *p = records + (size_t)(slot >> 1) * 4 + (slot & 1) * 2;
+        const float4 a = p[0], b = p[1];
+        lo = {a.x, a.y, a.z};
+        hi = {b.x, b.y, b.z};
+    } else {
+        const float4 p = records[(size_t)(slot >> 1) * 3 + (slot & 1)];
+        lo = {p.x, p.y, 0.0f};
+        hi = {p.z, p.w, 0.0f};
+    }
+}
+
+template <int DIM>
+__device__ __forceinline__ void load_root_box(const float4 *root, v3 &lo, v3 &hi)
+{
+    const float4 a = root[0], b = root[1];
+    lo = {a.x, a.y, DIM == 3 ? a.z : 0.0f};
+    hi = {DIM == 3 ? b.x : a.z, DIM == 3 ? b.y : a.w, DIM == 3 ? b.z : 0.0f};
+}
+
+// vertices of a primitive as 3D points (2D: two vertices, z = 0)
+template <int DIM>
+__device__ __forceinline__ void disk_verts(const float4 *prims, int slot, v3 p[3])
+{
+    if (DIM == 3) {
+        const float4 *t = prims + (size_t)slot * 3;
+        const float4 a = t[0], b = t[1], c = t[2];
+        p[0] = {a.x, a.y, a.z};
+        p[1] = {b.x, b.y, b.z};
+        p[2] = {c.x, c.y, c.z};
+    } else {
+        const float4 s4 = prims[slot];
+        p[0] = p[2] = {s4.x, s4.y, 0.0f};
+        p[1] = {s4.z, s4.w, 0.0f};
+    }
+}
+
+// (lo, hi) contains (l, h); false for a NaN
+__device__ __forceinline__ bool box_contains(v3 lo, v3 hi, v3 l, v3 h)
+{
+    return lo.x <= l.x && lo.y <= l.y && lo.z <= l.z && hi.x >= h.x && hi.y >= h.y && hi.z >= h.z;
+}
+
+// the box (lo, hi) contains the boxes of the record, or the primitives of the leaf, that link names
+template <int DIM>
+__device__ __forceinline__ bool box_holds(const float4 *records, const float4 *prims, uint32_t link, v3 lo, v3 hi)
+{
+    if (!(link & LEAF_BIT)) {
+        v3 l0, h0, l1, h1;
+        load_slot_box<DIM>(records, (int)link * 2, l0, h0);
+        load_slot_box<DIM>(records, (int)link * 2 + 1, l1, h1);
+        return box_contains(lo, hi, l0, h0) && box_contains(lo, hi, l1, h1);
+    }
+    const int first = (int)(link & OFF_MASK), last = first + (int)((link >> CNT_SHIFT) & CNT_MASK);
+    bool in = true;
+    for (int s = first; s <= last; s++) {
+        v3 p[3];
+        disk_verts<DIM>(prims, s, p);
+        for (int k = 0; k < DIM; k++) in = in && box_contains(lo, hi, p[k], p[k]);
+    }
+    return in;
+}
+
+// info[3] is set where a box does not hold what lies below it: a caller's boxes,
+// or boxes from before a vertex update.  The reference shrinks r^2 by such boxes
+// too, so dropping a subtree could change a record, and the disks stay off until
+// a refit (k_build_disks).
+template <int DIM>
+__global__ void k_slot_ranges(const float4 *records, const float4 *root, const float4 *prims, int n_records,
+                              int2 *ranges, int *info)
 {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n_records) return;
+    for (int side = 0; side < 2; side++) {
+        v3 lo, hi;
+        load_slot_box<DIM>(records, 2 * r + side, lo, hi);
+        if (!box_holds<DIM>(records, prims, slot_link<DIM>(records, (uint32_t)r, side), lo, hi)) info[3] = 1;
+    }
+    if (r == 0) {
+        v3 lo, hi;
+        load_root_box<DIM>(root, lo, hi);
+        if (!box_holds<DIM>(records, prims, link_of(DIM == 3 ? root[0].w : root[1].x), lo, hi)) info[3] = 1;
+    }
     const uint32_t a = slot_link<DIM>(records, (uint32_t)r, 0), b = slot_link<DIM>(records, (uint32_t)r, 1);
     const int a0 = subtree_edge<DIM>(records, a, 0), a1 = subtree_edge<DIM>(records, a, 1);
     const int b0 = subtree_edge<DIM>(records, b, 0), b1 = subtree_edge<DIM>(records, b, 1);
@@ -1713,21 +1794,6 @@ __global__ void k_slot_frontier(const int2 *ranges, const float4 *root, int n_sl
     const int2 rg = ranges[s];
     if (rg.y <= DISK_MAX_PRIMS && (rg.y + ranges[s ^ 1].y > DISK_MAX_PRIMS || (uint32_t)(s >> 1) == root_rec))
         frontier[pos[rg.x]] = s;
-}
-
-template <int DIM>
-__device__ __forceinline__ void load_slot_box(const float4 *records, int slot, v3 &lo, v3 &hi)
-{
-    if (DIM == 3) {
-        const float4 *p = records + (size_t)(slot >> 1) * 4 + (slot & 1) * 2;
-        const float4 a = p[0], b = p[1];
-        lo = {a.x, a.y, a.z};
-        hi = {b.x, b.y, b.z};
-    } else {
-        const float4 p = records[(size_t)(slot >> 1) * 3 + (slot & 1)];
-        lo = {p.x, p.y, 0.0f};
-        hi = {p.z, p.w, 0.0f};
-    }
 }
 
 template <int DIM>
@@ -1845,23 +1911,6 @@ struct DiskSums {
     float mt, mr;         // allowance for points off their primitive, along and across n
 };
 
-// vertices of a primitive as 3D points (2D: two vertices, z = 0)
-template <int DIM>
-__device__ __forceinline__ void disk_verts(const float4 *prims, int slot, v3 p[3])
-{
-    if (DIM == 3) {
-        const float4 *t = prims + (size_t)slot * 3;
-        const float4 a = t[0], b = t[1], c = t[2];
-        p[0] = {a.x, a.y, a.z};
-        p[1] = {b.x, b.y, b.z};
-        p[2] = {c.x, c.y, c.z};
-    } else {
-        const float4 s4 = prims[slot];
-        p[0] = p[2] = {s4.x, s4.y, 0.0f};
-        p[1] = {s4.z, s4.w, 0.0f};
-    }
-}
-
 template <int DIM>
 __device__ __forceinline__ void disk_normal_add(const float4 *prims, int slot, DiskSums &D)
 {
@@ -1959,30 +2008,24 @@ __device__ __forceinline__ float4 disk_pack(const DiskSums &D, v3 half, v3 n, ui
 // The disks of all slots, shared out as in k_refit_ranges: two passes over a
 // slot's primitives (normal, extents), which lie together in leaf order.
 // Slots above DISK_MAX_PRIMS have none.  Queries whose root box's farthest
-// corner lies beyond disk_limit go without.
+// corner lies beyond disk_limit go without, and all queries where the boxes do
+// not hold their primitives (info[3], k_slot_ranges; null after a refit).
 template <int DIM>
 __global__ __launch_bounds__(DISK_BLOCK) void k_build_disks(const float4 *records, const float4 *root,
                                                             const float4 *prims, const int2 *ranges, int n_slots,
                                                             const int *big, int n_big, int own_blocks, float4 *disks,
-                                                            float *disk_limit)
+                                                            float *disk_limit, const int *info)
 {
     v3 rlo, rhi;
-    if (DIM == 3) {
-        const float4 a = root[0], b = root[1];
-        rlo = {a.x, a.y, a.z};
-        rhi = {b.x, b.y, b.z};
-    } else {
-        const float4 a = root[0];
-        rlo = {a.x, a.y, 0.0f};
-        rhi = {a.z, a.w, 0.0f};
-    }
+    load_root_box<DIM>(root, rlo, rhi);
     const v3 ext = sub(rhi, rlo);
     const float reach = 1.5f * sqrtf(dot(ext, ext)); // queries in 1.5 times the box and beyond
     const float scale = fmaxf(fmaxf(fmaxf(fabsf(rlo.x), fabsf(rhi.x)), fmaxf(fabsf(rlo.y), fabsf(rhi.y))),
                               fmaxf(fabsf(rlo.z), fabsf(rhi.z)));
     // the bound's squares neither overflow (1e37) nor leave the normal range
     // (1e-6: a disk excludes no distance below 1e-6 of the coordinates)
-    if (blockIdx.x == 0 && threadIdx.x == 0) *disk_limit = reach >= 1e-6f ? fminf(reach * reach, 1e37f) : -1.0f;
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        *disk_limit = reach >= 1e-6f && !(info && info[3]) ? fminf(reach * reach, 1e37f) : -1.0f;
     const bool own = (int)blockIdx.x < own_blocks;
     int slot, step, first;
     if (own) {

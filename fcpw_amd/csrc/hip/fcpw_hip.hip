@@ -67,17 +67,20 @@ static dim3 slot_grid(const fcpw_hip_ctx *c)
     return dim3((unsigned)(slot_own_blocks(c) + (c->n_big + DISK_BLOCK / 64 - 1) / (DISK_BLOCK / 64)));
 }
 
-// the disks of a single object's tree, from its records, primitives and ranges
-static int launch_disks(fcpw_hip_ctx *c, hipStream_t s)
+// the disks of a single object's tree, from its records, primitives and ranges; info = what
+// k_slot_ranges found, null where the boxes have just been refitted
+static int launch_disks(fcpw_hip_ctx *c, hipStream_t s, const int *info = nullptr)
 {
     if (!c->by_range) return FCPW_HIP_OK;
     const int n_slots = 2 * c->n_records;
     if (c->dim == 3)
         hipLaunchKernelGGL(k_build_disks<3>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->root, c->prims,
-                           c->ranges, n_slots, c->big, c->n_big, slot_own_blocks(c), c->disks, c->disk_limit);
+                           c->ranges, n_slots, c->big, c->n_big, slot_own_blocks(c), c->disks, c->disk_limit,
+                           info);
     else
         hipLaunchKernelGGL(k_build_disks<2>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->root, c->prims,
-                           c->ranges, n_slots, c->big, c->n_big, slot_own_blocks(c), c->disks, c->disk_limit);
+                           c->ranges, n_slots, c->big, c->n_big, slot_own_blocks(c), c->disks, c->disk_limit,
+                           info);
     HIPCHECK(c, hipGetLastError());
     return FCPW_HIP_OK;
 }
@@ -110,7 +113,7 @@ static int compute_ranges(fcpw_hip_ctx *c)
     HIPCHECK(c, hipMemset(c->range_info, 0, 4 * sizeof(int)));
     HIPCHECK(c, hipMemset(c->range_mark, 0, ((size_t)c->n_prims + 1) * sizeof(uint32_t)));
     hipLaunchKernelGGL(k_slot_ranges<DIM>, dim3((unsigned)((c->n_records + t - 1) / t)), dim3(t), 0, 0, c->records,
-                       c->n_records, c->ranges, c->range_info);
+                       c->root, c->prims, c->n_records, c->ranges, c->range_info);
     HIPCHECK(c, hipGetLastError());
     int info[4];
     HIPCHECK(c, hipMemcpy(info, c->range_info, sizeof(info), hipMemcpyDeviceToHost));
@@ -129,7 +132,7 @@ static int compute_ranges(fcpw_hip_ctx *c)
     c->n_top = info[2];
     c->n_frontier = (int)n_frontier;
     c->by_range = true;
-    return launch_disks(c, 0);
+    return launch_disks(c, 0, c->range_info);
 }
 
 static int compute_ranges(fcpw_hip_ctx *c) { return c->dim == 3 ? compute_ranges<3>(c) : compute_ranges<2>(c); }

@@ -139,3 +139,35 @@ def test_batch_members_use_their_own_disks(gpu):
         ref = oracle.Bvh(V, F).closest_points_gpuorder(qk, np.full(len(qk), np.inf, np.float32))
         assert_bit_equal(rec[at:at + len(qk)], ref)
         at += len(qk)
+
+
+def torn(V, k):
+    """one half moved far away: the boxes it leaves behind shrink the reference's
+    r^2 for queries near them, so that the other half is out of reach"""
+    V2 = V.copy()
+    V2[(V[:, 0] < 0.0) == (k == 0), -1] += np.float32(10.0)
+    return V2
+
+
+@pytest.mark.parametrize("mesh", ["torus", "star2d"])
+def test_stale_boxes_stay_without_disks(gpu, mesh):
+    """boxes that do not hold their primitives shrink the reference's r^2 too, so
+    no subtree may be dropped: after a vertex update, also when the records are
+    reordered before the refit, and for a tree uploaded with boxes from before one"""
+    import torch
+    V, F = meshes.small_torus(64, 32) if mesh == "torus" else meshes.small_star(5000)
+    _, g = make_scene(V, F)
+    q = queries(V, 6000, 41)
+    b = oracle.Bvh(V, F)
+    for k, layout in enumerate((1, 0)):
+        V2 = torn(V, k)
+        st = torch.cuda.current_stream().cuda_stream
+        dv = torch.from_numpy(V2).cuda()
+        g._update_positions_device(dv.data_ptr(), len(V2), st)
+        torch.cuda.synchronize()
+        b.update_vertices(V2)
+        g.set_option("layout", layout)
+        check(g, V2, F, q, bvh=b)
+        g._refit_device(st)
+        b.refit()
+        check(g, V2, F, q, bvh=b)

@@ -1,0 +1,104 @@
+"""Trees a caller uploads through the C ABI, which need not be those of a build:
+boxes from before a vertex update, leaves whose primitives lie in another
+order than the leaves do.  The records are the oracle's bit for bit, whose
+traversal knows neither."""
+import ctypes
+import os
+
+import numpy as np
+import pytest
+
+import oracle
+from fcpw_amd import synth
+from tests import meshes
+from tests.test_gpu_disks import queries, torn
+from tests.test_gpu_parity import assert_bit_equal
+
+pytestmark = pytest.mark.gpu
+fcpw = pytest.importorskip("fcpw_amd")
+
+LIB = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "fcpw_amd", "lib", "libfcpw_hip.so")
+VP, I64 = ctypes.c_void_p, ctypes.c_int64
+MESHES = {"torus": lambda: meshes.small_torus(64, 32), "star2d": lambda: meshes.small_star(5000)}
+
+
+class Tree:
+    """the arrays fcpw_hip_upload_bvh takes"""
+
+    def __init__(self, b, F):
+        self.pmin, self.pmax, self.nrefs, self.offset = (np.ascontiguousarray(a) for a in b.nodes())
+        self.index = np.ascontiguousarray(b.prim_order(), np.int32)
+        self.prims = np.ascontiguousarray(F[self.index], np.int32)
+
+
+class Context:
+    def __init__(self, dim):
+        L = self.lib = ctypes.CDLL(LIB)
+        L.fcpw_hip_create.argtypes = [ctypes.c_int, ctypes.POINTER(VP)]
+        L.fcpw_hip_last_error.restype = ctypes.c_char_p
+        L.fcpw_hip_last_error.argtypes = [VP]
+        L.fcpw_hip_destroy.argtypes = [VP]
+        L.fcpw_hip_upload_bvh.argtypes = [VP, ctypes.c_int, ctypes.c_int] + [VP] * 4 + [ctypes.c_int, VP, VP,
+                                                                                       ctypes.c_int, VP]
+        L.fcpw_hip_refit.argtypes = [VP, VP]
+        L.fcpw_hip_set_option.argtypes = [VP, ctypes.c_char_p, ctypes.c_int]
+        L.fcpw_hip_update_positions.argtypes = [VP, VP, ctypes.c_int]
+        L.fcpw_hip_closest_points.argtypes = [VP, VP, I64, ctypes.c_int, VP]
+        L.fcpw_hip_upload_silhouettes.argtypes = [VP, ctypes.c_int, VP, VP, VP, ctypes.c_int, VP]
+        L.fcpw_hip_closest_silhouette_points.argtypes = [VP, VP, VP, I64, ctypes.c_float, ctypes.c_float, VP]
+        self.dim, self.h = dim, VP()
+        self.ok(L.fcpw_hip_create(0, ctypes.byref(self.h)))
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *unused):
+        self.lib.fcpw_hip_destroy(self.h)
+
+    def ok(self, st):
+        assert st == 0, self.lib.fcpw_hip_last_error(self.h)
+
+    def upload(self, t, V):
+        V = np.ascontiguousarray(V, np.float32)
+        self.ok(self.lib.fcpw_hip_upload_bvh(
+            self.h, self.dim, len(t.nrefs), t.pmin.ctypes.data, t.pmax.ctypes.data, t.nrefs.ctypes.data,
+            t.offset.ctypes.data, len(t.prims), t.prims.ctypes.data, t.index.ctypes.data, len(V), V.ctypes.data))
+
+    def update(self, V):
+        V = np.ascontiguousarray(V, np.float32)
+        self.ok(self.lib.fcpw_hip_update_positions(self.h, V.ctypes.data, len(V)))
+
+    def refit(self):
+        self.ok(self.lib.fcpw_hip_refit(self.h, None))
+
+    def option(self, key, value):
+        self.ok(self.lib.fcpw_hip_set_option(self.h, key.encode(), value))
+
+    def closest(self, q):
+        s = np.full((len(q), 4), np.inf, np.float32)
+        s[:, :3] = 0.0
+        s[:, :self.dim] = q
+        out = np.zeros(len(q), fcpw.INTERACTION_DTYPE)
+        self.ok(self.lib.fcpw_hip_closest_points(self.h, s.ctypes.data, len(q), 1, out.ctypes.data))
+        return out
+
+    def check(self, b, q):
+        ref = b.closest_points_gpuorder(q, record_normal=True)
+        assert_bit_equal(self.closest(q), ref)
+
+
+@pytest.mark.parametrize("mesh", sorted(MESHES))
+def test_boxes_from_before_a_vertex_update(gpu, mesh):
+    """they shrink the reference's r^2 although they hold nothing, so no subtree may be dropped"""
+    V, F = MESHES[mesh]()
+    b = oracle.Bvh(V, F)
+    t = Tree(b, F)
+    V2 = torn(V, 0)
+    q = queries(V, 6000, 46)
+    b.update_vertices(V2)
+    with Context(V.shape[1]) as c:
+        c.upload(t, V2)
+        c.check(b, q)
+        c.refit()
+        b.refit()
+        c.check(b, q)
