@@ -28,7 +28,8 @@ struct fcpw_hip_ctx {
     // the leaf-slot range below every child slot, the slots sorted by its size,
     // and the disks with the distance they hold up to: parts of range_mem, which
     // is null for a tree over instances.  by_range: the leaves lie in order, so
-    // the ranges are valid
+    // the ranges are valid; one_tree: every node but the root has one parent (a
+    // caller's arrays may say otherwise)
     void *range_mem = nullptr;
     float4 *disks = nullptr;
     int4 *top = nullptr;
@@ -36,7 +37,7 @@ struct fcpw_hip_ctx {
     int *big = nullptr, *frontier = nullptr, *range_info = nullptr;
     uint32_t *range_mark = nullptr, *range_sums = nullptr;
     float *disk_limit = nullptr;
-    bool by_range = false;
+    bool by_range = false, one_tree = false;
     int n_big = 0, n_top = 0, n_frontier = 0;
     int *flags = nullptr;
     unsigned long long *stats = nullptr; // internal nodes, primitive tests, queries (option "stats")

@@ -107,7 +107,9 @@ static int compute_ranges(fcpw_hip_ctx *c)
     c->n_big = c->n_top = c->n_frontier = 0;
     const float none = -1.0f;
     HIPCHECK(c, hipMemcpy(c->disk_limit, &none, sizeof(float), hipMemcpyHostToDevice));
-    if (c->n_records <= 0) return FCPW_HIP_OK; // a root leaf has no slots
+    // a root leaf has no slots; and where nodes have no or two parents the lists
+    // below would hold more slots than a tree has (upload_ranges)
+    if (c->n_records <= 0 || !c->one_tree) return FCPW_HIP_OK;
     const int n_slots = 2 * c->n_records, t = 256;
     const dim3 gs((unsigned)((n_slots + t - 1) / t));
     HIPCHECK(c, hipMemset(c->range_info, 0, 4 * sizeof(int)));
@@ -142,8 +144,8 @@ static int compute_ranges(fcpw_hip_ctx *c) { return c->dim == 3 ? compute_ranges
 static int upload_ranges(fcpw_hip_ctx *c)
 {
     const size_t n_slots = (size_t)2 * c->n_records, n_prims = (size_t)c->n_prims;
-    // slots above DISK_MAX_PRIMS are disjoint at each of at most STACK_TOTAL - 1 levels,
-    // and every marked slot is a child of one of their records or of the root
+    // in one tree (compute_ranges) slots above DISK_MAX_PRIMS are disjoint at each of
+    // at most STACK_TOTAL - 1 levels, and every marked slot is a child of one of their records or of the root
     const size_t cap_top = std::min(n_slots, (size_t)STACK_TOTAL * (n_prims / DISK_MAX_PRIMS + 1));
     const size_t cap_front = std::min(n_slots, 2 * cap_top + 2);
     const size_t segs = (n_prims + 1 + SCAN_SEG - 1) / SCAN_SEG;
@@ -376,6 +378,7 @@ static int gpu_build(fcpw_hip_ctx *c, const float *positions, int n_vertices, co
     c->n_prims = n;
     c->n_vertices = n_vertices;
     c->max_depth = status[1];
+    c->one_tree = true;
     c->node_slot = std::move(node_slot);
     c->node_leaf_off = std::move(node_leaf_off);
     const int st_disks = upload_ranges(c);
@@ -496,6 +499,7 @@ struct TreeRecords {
     std::vector<uint32_t> leaf_links;
     std::vector<int32_t> node_slot, node_leaf_off;
     int n_rec = 0, n_leaf = 0, max_depth = 0;
+    bool one_tree = true; // every node but the root is the child of exactly one
 };
 
 static int tree_records(fcpw_hip_ctx *c, const char *fn, int dim, int n_nodes, const float *pmin, const float *pmax,
@@ -555,6 +559,7 @@ static int tree_records(fcpw_hip_ctx *c, const char *fn, int dim, int n_nodes, c
         int kids[2] = {i + 1, i + offset[i]};
         for (int sd = 0; sd < 2; sd++) {
             int k = kids[sd];
+            if (T.node_slot[k] != 2 * n_rec) T.one_tree = false;
             T.node_slot[k] = r * 2 + sd;
             depth[k] = depth[i] + 1;
             max_depth = std::max(max_depth, depth[k]);
@@ -791,6 +796,7 @@ int fcpw_hip_upload_bvh(fcpw_hip_ctx *c, int dim, int n_nodes, const float *pmin
     c->n_prims = n_prims;
     c->n_vertices = n_vertices;
     c->max_depth = T.max_depth;
+    c->one_tree = T.one_tree;
     c->node_slot = std::move(T.node_slot);
     c->node_leaf_off = std::move(T.node_leaf_off);
     if ((st = upload_ranges(c))) return st;

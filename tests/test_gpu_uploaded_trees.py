@@ -102,3 +102,40 @@ def test_boxes_from_before_a_vertex_update(gpu, mesh):
         c.refit()
         b.refit()
         c.check(b, q)
+
+
+def test_nodes_without_a_parent(gpu):
+    """Arrays in which many nodes no other names all have the same second child:
+    they pass the upload's checks, queries never reach them, and the slots of the
+    ranges' lists would outnumber those of a tree."""
+    V, F = meshes.small_torus(64, 32)  # 4,096 triangles, as the root's second child
+    b = oracle.Bvh(V, F)
+    t = Tree(b, F)
+    E = np.array([[3.0, 0.0, 0.0], [3.0, 0.1, 0.0], [3.0, 0.0, 0.1]], np.float32)  # the first: one triangle
+    extra = 5000
+    pad = 2 + 2 * extra  # the root, its first child, pairs of an unnamed node and its leaf
+    at = np.arange(extra) * 2 + 2
+    nrefs, offset = np.zeros(pad, np.int32), np.zeros(pad, np.int32)
+    nrefs[1], offset[0] = 1, pad
+    nrefs[at + 1], offset[at] = 1, pad - at
+    t.nrefs, t.offset = np.concatenate([nrefs, t.nrefs]), np.concatenate([offset, t.offset + (t.nrefs > 0)])
+    t.offset = t.offset.astype(np.int32)
+    t.pmin = np.concatenate([np.full((pad, 3), -4.0, np.float32), t.pmin])
+    t.pmax = np.concatenate([np.full((pad, 3), 4.0, np.float32), t.pmax])
+    t.pmin[1], t.pmax[1] = E.min(0), E.max(0)
+    t.prims = np.concatenate([np.arange(3, dtype=np.int32)[None] + len(V), t.prims])
+    t.index = np.concatenate([np.array([len(F)], np.int32), t.index])
+    W = np.concatenate([V, E])
+    q = queries(W, 3000, 51)
+    ref = np.minimum(b.closest_points_gpuorder(q)["d"],
+                     oracle.Bvh(E, np.array([[0, 1, 2]], np.int32)).closest_points_gpuorder(q)["d"])
+    with Context(3) as c:
+        c.upload(t, W)
+        for refitted in (False, True):
+            rec = c.closest(q)
+            np.testing.assert_array_equal(rec["d"], ref)
+            assert (rec["index"] == len(F)).any() and (rec["index"] < len(F)).any()
+            c.option("coop", 0)
+            assert c.closest(q).tobytes() == rec.tobytes()
+            c.option("coop", 1)
+            c.refit()
