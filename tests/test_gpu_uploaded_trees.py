@@ -13,6 +13,7 @@ from fcpw_amd import synth
 from tests import meshes
 from tests.test_gpu_disks import queries, torn
 from tests.test_gpu_parity import assert_bit_equal
+from tests.test_gpu_silhouettes import MAX_ULP_FLIPS
 
 pytestmark = pytest.mark.gpu
 fcpw = pytest.importorskip("fcpw_amd")
@@ -139,3 +140,70 @@ def test_nodes_without_a_parent(gpu):
             assert c.closest(q).tobytes() == rec.tobytes()
             c.option("coop", 1)
             c.refit()
+
+
+def leaves_reversed(t):
+    """the same tree, its leaves' primitives laid out from the last leaf to the first"""
+    n = len(t.prims)
+    old = np.empty(n, np.int64)
+    for i in np.nonzero(t.nrefs > 0)[0]:
+        a, k = int(t.offset[i]), int(t.nrefs[i])
+        new = n - a - k
+        old[new:new + k] = np.arange(a, a + k)
+        t.offset[i] = new
+    t.prims, t.index = np.ascontiguousarray(t.prims[old]), np.ascontiguousarray(t.index[old])
+    return t
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("mesh", sorted(MESHES))
+def test_leaves_out_of_order(gpu, mesh, layout):
+    """such a tree has no ranges: boxes alone, refitted by climbing from the leaves"""
+    V, F = MESHES[mesh]()
+    b = oracle.Bvh(V, F)
+    q = queries(V, 6000, 61)
+    with Context(V.shape[1]) as c:
+        c.option("layout", layout)
+        c.upload(leaves_reversed(Tree(b, F)), V)
+        c.check(b, q)
+        for k in range(2):
+            V = (V + synth.Rng(62 + k).uniform(V.size, -0.02, 0.02).reshape(V.shape)).astype(np.float32)
+            c.update(V)
+            c.refit()
+            b.update_vertices(V)
+            b.refit()
+            c.check(b, q)
+
+
+@pytest.mark.parametrize("mesh", sorted(MESHES))
+def test_silhouettes_with_leaves_out_of_order(gpu, mesh):
+    """such a tree has no facing entries: the cooperative kernel against the
+    per-lane one bit for bit, and the oracle's traversal, which may round a cone
+    test the other way in MAX_ULP_FLIPS queries"""
+    V, F = MESHES[mesh]()
+    b = oracle.Bvh(V, F)
+    b.build_silhouettes()
+    cones, count, offset, rec = b.silhouettes()
+    if V.shape[1] == 2:  # fcpw_hip_vertex has one point
+        rec = np.ascontiguousarray(rec[["pa", "n0", "n1", "index", "has_one_adjacent_face"]].astype(
+            [("pa", "<f4", (3,)), ("n0", "<f4", (3,)), ("n1", "<f4", (3,)), ("index", "<u4"), ("one", "<u4")]))
+    q = queries(V, 4000, 63)
+    s = np.full((len(q), 4), np.finfo(np.float32).max, np.float32)
+    s[:, :3] = 0.0
+    s[:, :V.shape[1]] = q
+    flip = (np.arange(len(q)) % 2).astype(np.uint32)
+    with Context(V.shape[1]) as c:
+        c.upload(leaves_reversed(Tree(b, F)), V)
+        c.ok(c.lib.fcpw_hip_upload_silhouettes(c.h, len(count), cones.ctypes.data, count.ctypes.data,
+                                               offset.ctypes.data, len(rec), rec.ctypes.data))
+        out = []
+        for coop in (1, 0):
+            c.option("coop", coop)
+            o = np.zeros(len(q), fcpw.INTERACTION_DTYPE)
+            c.ok(c.lib.fcpw_hip_closest_silhouette_points(c.h, s.ctypes.data, flip.ctypes.data, len(q), 0.0, 1e-3,
+                                                          o.ctypes.data))
+            out.append(o)
+        assert out[0].tobytes() == out[1].tobytes()
+        ref = b.closest_silhouettes(q, flip=flip)
+        same = (out[0]["index"].view(np.int32) == ref["index"]) & (out[0]["d"] == ref["d"])
+        assert (~same).sum() <= MAX_ULP_FLIPS
