@@ -11,6 +11,8 @@ static float bits_as_float(uint32_t u)
     return f;
 }
 
+constexpr int RAY_HOLD_DEFAULT = 8;
+
 struct fcpw_hip_ctx {
     int device = 0;
     int dim = 0;
@@ -89,7 +91,9 @@ struct fcpw_hip_ctx {
     int ray_coop = 1; // wave-cooperative leaves for ray queries
     int ray_sort_dir = 1; // rays ordered by direction octant, then origin
     bool stack_auto = true; // stack not set by the caller: by the batch size (launch_closest_kernel)
-    int ray_stack = 4, ray_hold_min = 8; // the cooperative ray kernels' LDS stack entries and leaf-pass threshold
+    // the cooperative ray kernels' LDS stack entries and leaf-pass threshold (the
+    // default: by the batch size, launch_intersect)
+    int ray_stack = 4, ray_hold_min = RAY_HOLD_DEFAULT;
     int sil_stack = 4, inst_stack = 12;  // LDS stack entries of the 3D cooperative silhouette and instance kernels
     bool sil_stack_auto = true;          // sil_stack not set by the caller: eight (launch_silhouettes)
     int layout = 0;                      // record order in memory: 0 DFS, 1 treelets of three levels
@@ -97,6 +101,8 @@ struct fcpw_hip_ctx {
     int sil_xcds = 8;                    // the silhouette kernels' XCD grouping
     int inst_seed = 1024;                // instanced closest points: ordered queries per representative wave (0: off)
     bool inst_seed_auto = true;          // not set by the caller: only batches that gain from it (launch_instances_closest)
+    // what the latest cooperative launch took of the options and size rules
+    struct { int stack, hold_min, wave_queries; } launch = {0, 0, 0};
     int stats_on = 0, timing = 0;
     int n_cus = 256;
     // device scratch of fcpw_hip_build_bvh, kept (grow-only) for the next build

@@ -1175,6 +1175,7 @@ static int launch_closest_kernel(fcpw_hip_ctx *c, const CpIO &io, hipStream_t s,
         // the caller set the option it takes twelve and spills less (100,003 queries
         // 165 -> 160 us, 30,000 in 2D 317 -> 306, 12,000 on 300,000 triangles 851 -> 820).
         const int k = c->stack_auto && (int64_t)g.x <= (int64_t)16 * c->n_cus ? 12 : c->stack;
+        c->launch = {k, c->hold_min, wq};
         if (c->dim == 3) {
             if (k == 0) FCPW_COOP(3, 0);
             else if (k == 4) FCPW_COOP(3, 4);
@@ -1264,11 +1265,13 @@ static int launch_intersect(fcpw_hip_ctx *c, const void *rays, int64_t n, int oc
     if ((st = timing_begin(c, s))) return st;
     if (c->ray_coop) {
         const int wq = c->stats_on ? 64 : wave_queries(c, n);
-        // a part-filled wave has lanes free for every leaf: it waits for no others
-        // (65,537 occlusion rays, 32 a wave: 250 us waiting for 8, 238 for 1)
-        const int hold = wq < 64 ? 1 : c->ray_hold_min;
+        // a part-filled wave has lanes free for every leaf: unless the caller chose a
+        // threshold it waits for no others (65,537 occlusion rays, 32 a wave: 250 us
+        // waiting for 8, 238 for 1)
+        const int hold = wq < 64 && c->ray_hold_min == RAY_HOLD_DEFAULT ? 1 : c->ray_hold_min;
         const dim3 g = grid_for(c, n, wq);
         const int k = c->ray_stack;
+        c->launch = {k, hold, wq};
 #define FCPW_RCOOP(D, K, ST)                                                                                  \
     hipLaunchKernelGGL((k_intersect_coop<D, K, ST>), g, dim3(64), 0, s, S, (const float2 *)rays, n, occlusion, \
                        (float2 *)out, order, xcd_arg(c), hold, wq)
@@ -1495,6 +1498,7 @@ static int launch_silhouettes(fcpw_hip_ctx *c, const void *spheres, const uint32
         // triangles 13.0 ms with four and 11.0 with eight, 1M 21.6 and 17.9, 4.2M on
         // a million triangles 164 and 133, 30,000 on 20,000 triangles 3.2 and 2.8.
         const int k = c->sil_stack_auto ? 8 : c->sil_stack;
+        c->launch = {c->dim == 3 ? k : 8, c->sil_hold_min, wq};
 #define FCPW_SIL3(K)                                                                                          \
     hipLaunchKernelGGL((k_closest_silhouettes_coop<3, K>), g, dim3(64), 0, s, S, T, (const float4 *)spheres, flip, n, \
                        r2min, prec, (float2 *)out, order, sil_xcd_arg(c), c->sil_hold_min, wq)
@@ -1752,6 +1756,9 @@ int fcpw_hip_get_info(const fcpw_hip_ctx *c, const char *key, int64_t *value)
     else if (k == "generation") *value = (int64_t)c->generation;
     else if (k == "positions_version") *value = (int64_t)c->positions_version;
     else if (k == "device") *value = c->device;
+    else if (k == "launch_stack") *value = c->launch.stack;
+    else if (k == "launch_hold_min") *value = c->launch.hold_min;
+    else if (k == "launch_wave_queries") *value = c->launch.wave_queries;
     else if (k == "n_instances") *value = c->instanced ? c->n_instances : 0;
     else if (k == "n_objects") *value = c->instanced ? (int64_t)c->inst_objects.size() : (c->uploaded ? 1 : 0);
     else if (k.rfind("stat_", 0) == 0) {

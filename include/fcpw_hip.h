@@ -362,7 +362,8 @@ int fcpw_hip_batch_get_option(const fcpw_hip_batch *batch, const char *key, int 
                  instanced scenes, and closest silhouette points)
      "ray_coop"  the same choice for ray queries (default 1)
      "ray_stack", "ray_hold_min"  the cooperative ray kernels' LDS stack entries (4, 8
-                 or 16, default 4) and leaf-pass threshold (1..64, default 8)
+                 or 16, default 4) and leaf-pass threshold (1..64; the default 8 means 8
+                 in full waves of 64 rays and 1 in the part-filled ones of small batches)
      "sil_hold_min"  the cooperative silhouette kernel's leaf-pass threshold (default 3)
      "layout"    the order of the tree's records in HBM: 0 = DFS order of the internal
                  nodes (default), 1 = treelets (a node, its internal children and
@@ -425,6 +426,9 @@ int fcpw_hip_get_option(const fcpw_hip_ctx *ctx, const char *key, int *value);
    n_vertices = 0).  The instanced kernels run with fixed shapes (128 threads, 8
    LDS stack entries per object traversal, 4 for the instance tree); of the
    tuning knobs below only "sort", "morton_bits" and "xcds" apply to them.
+   launch_stack, launch_hold_min and launch_wave_queries: the LDS stack entries,
+   leaf-pass threshold and queries per wave that the latest launch of a cooperative
+   single-object kernel took (0 before the first).
    Measurement: stat_internal_nodes, stat_prim_tests,
    stat_queries and, for closest-point launches, stat_waves, stat_wave_iterations,
    stat_leaf_passes, stat_leaf_groups (cooperative leaf passes and their 64-item

@@ -33,3 +33,23 @@ def test_batch_sizes(gpu, mesh, n):
         hits = fcpw.GPUInteractionList()
         g.intersect(q, d, tmax, hits, check_for_occlusion=occlusion)
         assert_bit_equal(as_records(hits), b.intersect_gpuorder(q, d, tmax, occlusion))
+
+
+def cast(g, n):
+    hits = fcpw.GPUInteractionList()
+    o = np.zeros((n, 3), np.float32)
+    d = np.tile(np.array([[0.6, 0.8, 0.0]], np.float32), (n, 1))
+    g.intersect(o, d, np.full(n, np.inf, np.float32), hits)
+
+
+def test_a_chosen_leaf_pass_threshold_is_kept(gpu):
+    """the size rule stands in for the default of ray_hold_min only"""
+    _, g = make_scene(*meshes.small_torus(48, 24))
+    full = 512 * g.info("n_cus")
+    for value, part_filled in ((8, 1), (64, 64), (2, 2), (8, 1)):
+        g.set_option("ray_hold_min", value)
+        assert g.get_option("ray_hold_min") == value
+        cast(g, 1000)
+        assert g.info("launch_wave_queries") < 64 and g.info("launch_hold_min") == part_filled
+        cast(g, full)
+        assert g.info("launch_wave_queries") == 64 and g.info("launch_hold_min") == value
