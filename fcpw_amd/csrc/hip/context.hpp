@@ -11,7 +11,8 @@ static float bits_as_float(uint32_t u)
     return f;
 }
 
-constexpr int RAY_HOLD_DEFAULT = 8;
+// defaults that stand for a rule on sizes or on the mesh
+constexpr int RAY_HOLD_DEFAULT = 8, SIL_STACK_DEFAULT = 4;
 
 struct fcpw_hip_ctx {
     int device = 0;
@@ -45,8 +46,9 @@ struct fcpw_hip_ctx {
     unsigned long long *stats = nullptr; // internal nodes, primitive tests, queries (option "stats")
     // silhouettes (fcpw_hip_upload_silhouettes): cones per child slot and root, leaf ranges, records
     float4 *cones = nullptr, *sils = nullptr;
-    float4 *sil_faces = nullptr; // facing entries per child slot, valid while by_range
+    float4 *sil_faces = nullptr; // facing entries per child slot (3D trees with ranges, where they pay)
     int sil_unit = 0;            // no record has a normal longer than one
+    float sil_open = 1.0f;       // mean of (1 - n0.n1) / 2 over the records
     uint2 *sil_leaf = nullptr;
     bool has_silhouettes = false;
     int n_sil_refs = 0;
@@ -94,8 +96,9 @@ struct fcpw_hip_ctx {
     // the cooperative ray kernels' LDS stack entries and leaf-pass threshold (the
     // default: by the batch size, launch_intersect)
     int ray_stack = 4, ray_hold_min = RAY_HOLD_DEFAULT;
-    int sil_stack = 4, inst_stack = 12;  // LDS stack entries of the 3D cooperative silhouette and instance kernels
-    bool sil_stack_auto = true;          // sil_stack not set by the caller: eight (launch_silhouettes)
+    // LDS stack entries of the 3D cooperative silhouette (the default: by the mesh,
+    // launch_silhouettes) and instance kernels
+    int sil_stack = SIL_STACK_DEFAULT, inst_stack = 12;
     int layout = 0;                      // record order in memory: 0 DFS, 1 treelets of three levels
     int sil_hold_min = 3;                // the cooperative silhouette kernel's leaf-pass threshold
     int sil_xcds = 8;                    // the silhouette kernels' XCD grouping

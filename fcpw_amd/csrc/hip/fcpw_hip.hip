@@ -86,15 +86,11 @@ static int launch_disks(fcpw_hip_ctx *c, hipStream_t s, const int *info = nullpt
 }
 
 // the facing entries of the silhouette queries, from the boxes, ranges and silhouette records
-static int launch_faces(fcpw_hip_ctx *c, hipStream_t s)
+static int launch_faces(fcpw_hip_ctx *c, hipStream_t s, int *kept = nullptr)
 {
-    if (!c->by_range || !c->sil_faces) return FCPW_HIP_OK;
-    if (c->dim == 3)
-        hipLaunchKernelGGL(k_build_faces<3>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->ranges,
-                           2 * c->n_records, c->big, c->n_big, slot_own_blocks(c), c->sil_leaf, c->sils, c->sil_faces);
-    else
-        hipLaunchKernelGGL(k_build_faces<2>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->ranges,
-                           2 * c->n_records, c->big, c->n_big, slot_own_blocks(c), c->sil_leaf, c->sils, c->sil_faces);
+    if (!c->sil_faces) return FCPW_HIP_OK;
+    hipLaunchKernelGGL(k_build_faces, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->ranges, 2 * c->n_records,
+                       c->big, c->n_big, slot_own_blocks(c), c->sil_leaf, c->sils, c->sil_faces, kept);
     HIPCHECK(c, hipGetLastError());
     return FCPW_HIP_OK;
 }
@@ -867,6 +863,7 @@ int fcpw_hip_upload_silhouettes(fcpw_hip_ctx *c, int n_nodes, const fcpw_hip_bou
     const int RW = c->dim == 3 ? 4 : 2;
     std::vector<float4> rec_buf((size_t)std::max(n_refs, 1) * RW, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
     bool unit = true;
+    double open_sum = 0.0; // (1 - n0.n1) / 2 of the records, 1 of a boundary's
     const auto at_most_one = [](const fcpw_hip_float3 &n) { return n.x * n.x + n.y * n.y + n.z * n.z < 1.0002f; };
     for (int r = 0; r < n_refs; r++) {
         if (c->dim == 2) {
@@ -874,7 +871,6 @@ int fcpw_hip_upload_silhouettes(fcpw_hip_ctx *c, int n_nodes, const fcpw_hip_bou
             rec_buf[(size_t)r * 2] = make_float4(v.p.x, v.p.y, v.n0.x, v.n0.y);
             rec_buf[(size_t)r * 2 + 1] =
                 make_float4(v.n1.x, v.n1.y, bits_as_float(v.index), bits_as_float(v.has_one_adjacent_face));
-            unit = unit && at_most_one(v.n0) && at_most_one(v.n1);
         } else {
             const fcpw_hip_edge &e = ((const fcpw_hip_edge *)silhouettes)[r];
             rec_buf[(size_t)r * 4] = make_float4(e.pa.x, e.pa.y, e.pa.z, bits_as_float(e.index));
@@ -882,6 +878,9 @@ int fcpw_hip_upload_silhouettes(fcpw_hip_ctx *c, int n_nodes, const fcpw_hip_bou
             rec_buf[(size_t)r * 4 + 2] = make_float4(e.n0.x, e.n0.y, e.n0.z, 0.0f);
             rec_buf[(size_t)r * 4 + 3] = make_float4(e.n1.x, e.n1.y, e.n1.z, 0.0f);
             unit = unit && at_most_one(e.n0) && at_most_one(e.n1);
+            open_sum += e.has_one_adjacent_face == 1u
+                            ? 1.0
+                            : 0.5 * (1.0 - (double)(e.n0.x * e.n1.x + e.n0.y * e.n1.y + e.n0.z * e.n1.z));
         }
     }
     HIPCHECK(c, hipSetDevice(c->device));
@@ -896,10 +895,18 @@ int fcpw_hip_upload_silhouettes(fcpw_hip_ctx *c, int n_nodes, const fcpw_hip_bou
     c->n_sil_refs = n_refs;
     c->sil_leaf_max = leaf_max;
     c->sil_unit = unit ? 1 : 0;
-    if (c->by_range) {
+    c->sil_open = n_refs > 0 ? (float)(open_sum / n_refs) : 1.0f;
+    if (c->by_range && c->dim == 3) {
         HIPCHECK(c, hipMalloc((void **)&c->sil_faces, (size_t)2 * c->n_records * sizeof(float4)));
-        if ((st = launch_faces(c, 0))) return st;
-        HIPCHECK(c, hipDeviceSynchronize());
+        int *const kept = c->range_info; // [0] is zero where there are ranges
+        int n_kept = 0;
+        if ((st = launch_faces(c, 0, kept))) return st;
+        HIPCHECK(c, hipMemcpy(&n_kept, kept, sizeof(int), hipMemcpyDeviceToHost));
+        HIPCHECK(c, hipMemset(kept, 0, sizeof(int)));
+        if (n_kept < (2 * c->n_records - c->n_big - c->n_top) / 2) { // see launch_silhouettes
+            HIPCHECK(c, hipFree(c->sil_faces));
+            c->sil_faces = nullptr;
+        }
     }
     c->has_silhouettes = true;
     return FCPW_HIP_OK;
@@ -1473,15 +1480,11 @@ int fcpw_hip_intersect_spheres(fcpw_hip_ctx *c, const fcpw_hip_bounding_sphere *
     return FCPW_HIP_OK;
 }
 
-// LDS stack entries of the 3D cooperative silhouette kernel (4M queries on the
-// torus: 118.7 ms with 4, 120.1 with 0, 129.4 with 8, 132.0 with 12)
-constexpr int SIL_COOP_K3 = 4;
-
 static int launch_silhouettes(fcpw_hip_ctx *c, const void *spheres, const uint32_t *flip, int64_t n, float r2min,
                               float prec, void *out, hipStream_t s)
 {
     DevScene S = dev_scene(c);
-    SilScene T = {c->cones, c->sil_leaf, c->sils, c->by_range ? c->sil_faces : nullptr, c->sil_unit};
+    SilScene T = {c->cones, c->sil_leaf, c->sils, c->sil_faces, c->sil_unit};
     const uint32_t *order = nullptr;
     int st = morton_order(c, (const float *)spheres, 4, n, s, &order);
     if (st) return st;
@@ -1492,24 +1495,41 @@ static int launch_silhouettes(fcpw_hip_ctx *c, const void *spheres, const uint32
         // record indices within a leaf travel in 10 bits of a leaf-pass item
         const int wq = wave_queries(c, n);
         const dim3 g = grid_for(c, n, wq);
-        // Eight LDS entries unless the caller set the option.  Four, which keep eight
-        // waves a SIMD, were the faster before subtrees were dropped by their facing
-        // entries; now the spills of four cost more: 262,144 queries on 131,072
-        // triangles 13.0 ms with four and 11.0 with eight, 1M 21.6 and 17.9, 4.2M on
-        // a million triangles 164 and 133, 30,000 on 20,000 triangles 3.2 and 2.8.
-        const int k = c->sil_stack_auto ? 8 : c->sil_stack;
-        c->launch = {c->dim == 3 ? k : 8, c->sil_hold_min, wq};
+        // Which kernel, by the mesh as it was uploaded (262,144 queries, half of them near):
+        //  - facing entries and prepass where at least half of the small slots have an
+        //    entry: 131,072-triangle torus (all have) 17.0 ms without either, 16.2 with
+        //    the prepass alone, 11.5 with both; a box of 19,200 flat triangles (0.91)
+        //    30.0, 30.7, 23.3; a noisy sphere with 0.39 of them 11.4, 10.1, 10.5;
+        //  - the prepass alone where the faces of a record still mostly face the same
+        //    way (the mean of (1 - n0.n1) / 2 below 0.315): noisy spheres of 0.19
+        //    3.27 -> 2.77 ms, of 0.29 200 -> 181, of 0.31 29.5 -> 27.0 (but 0.80 -> 0.90
+        //    if all queries are near); of 0.33 1.00 -> 1.11, a soup (all boundary, 1)
+        //    0.33 -> 0.39;
+        //  - neither otherwise, and in 2D, whose records are cheap: 262,144 queries on
+        //    a star of 200,000 segments 0.96 ms with both, 0.93 with facing entries, 0.85
+        //    with neither; on a ring of 30,000 0.97, 0.89, 0.97.
+        // Four LDS entries, which keep eight waves a SIMD, for the last kind (1M queries on
+        // the sphere of 0.33: 1.82 ms, eight entries 1.97), eight with the others,
+        // whose spills cost more (131,072-triangle torus 11.0 ms, four 13.0).
+        const bool faces = c->sil_faces, pre = c->dim == 3 && (faces || c->sil_open < 0.315f);
+        const int k = c->dim == 2 ? 8 : c->sil_stack != SIL_STACK_DEFAULT ? c->sil_stack : pre ? 8 : 4;
+        c->launch = {k, c->sil_hold_min, wq};
+#define FCPW_SIL(DIM, K, FACES, PREPASS)                                                                      \
+    hipLaunchKernelGGL((k_closest_silhouettes_coop<DIM, K, FACES, PREPASS>), g, dim3(64), 0, s, S, T,         \
+                       (const float4 *)spheres, flip, n, r2min, prec, (float2 *)out, order, sil_xcd_arg(c),   \
+                       c->sil_hold_min, wq)
 #define FCPW_SIL3(K)                                                                                          \
-    hipLaunchKernelGGL((k_closest_silhouettes_coop<3, K>), g, dim3(64), 0, s, S, T, (const float4 *)spheres, flip, n, \
-                       r2min, prec, (float2 *)out, order, sil_xcd_arg(c), c->sil_hold_min, wq)
-        if (c->dim == 3) {
-            if (k == 8) FCPW_SIL3(8);
-            else if (k == 12) FCPW_SIL3(12);
-            else FCPW_SIL3(SIL_COOP_K3);
-        } else
+    do {                                                                                                      \
+        if (faces) FCPW_SIL(3, K, true, true);                                                                \
+        else if (pre) FCPW_SIL(3, K, false, true);                                                            \
+        else FCPW_SIL(3, K, false, false);                                                                    \
+    } while (0)
+        if (c->dim == 2) FCPW_SIL(2, 8, false, false);
+        else if (k == 4) FCPW_SIL(3, 4, false, false);
+        else if (k == 8) FCPW_SIL3(8);
+        else FCPW_SIL3(12);
 #undef FCPW_SIL3
-            hipLaunchKernelGGL((k_closest_silhouettes_coop<2, 8>), g, dim3(64), 0, s, S, T, (const float4 *)spheres,
-                               flip, n, r2min, prec, (float2 *)out, order, sil_xcd_arg(c), c->sil_hold_min, wq);
+#undef FCPW_SIL
     } else if (c->dim == 3)
         hipLaunchKernelGGL((k_closest_silhouettes<3, 128, 8>), dim3(blocks), dim3(128), 0, s, S, T,
                            (const float4 *)spheres, flip, n, r2min, prec, (float2 *)out, order, sil_xcd_arg(c));
@@ -1644,7 +1664,6 @@ int fcpw_hip_set_option(fcpw_hip_ctx *c, const char *key, int value)
         if (k == "sil_stack" ? (value != 4 && value != 8 && value != 12) : (value != 8 && value != 12))
             FAIL(c, FCPW_HIP_ERR_INVALID_ARGUMENT, "%s must be %s", key, k == "sil_stack" ? "4, 8 or 12" : "8 or 12");
         (k == "sil_stack" ? c->sil_stack : c->inst_stack) = value;
-        if (k == "sil_stack") c->sil_stack_auto = false;
     } else if (k == "bwd_order" || k == "bwd_reduce") {
         if (value != 0 && value != 1 && !(k == "bwd_reduce" && value == 2))
             FAIL(c, FCPW_HIP_ERR_INVALID_ARGUMENT, "%s must be 0 or 1%s", key, k == "bwd_reduce" ? " or 2" : "");

@@ -26,7 +26,7 @@ struct SilScene {
     const float4 *cones;
     const uint2 *sil_leaf;
     const float4 *sils;
-    const float4 *faces; // facing entries of the child slots (faces_away), or null
+    const float4 *faces; // facing entries of the child slots (faces_away)
     int unit;            // no record has a normal longer than one (certainly_off needs it)
 };
 
@@ -280,7 +280,7 @@ __device__ __forceinline__ bool silhouette_test(const SilRecord &s, v3 x, float 
 //   - rounding, here and in the reference's evaluation: 1e-5 of the lengths, and
 //     4e-6 of the coordinates, which F and B hold already.
 // Subtrees with boundary edges, faces without a normal or angles above 60 degrees
-// have none (T infinite).  Visits on the 131,072-triangle torus, 262,144 queries:
+// have none (T infinite), and 2D scenes (launch_silhouettes).  Visits on the 131,072-triangle torus, 262,144 queries:
 // 281 expanded records and 638 record tests a query without, 176 and 332 with.
 //
 // 16 bytes a slot: {a.x, a.y (f16)} {a.z (f16), T (bf16)} {B, F (bf16)}
@@ -301,16 +301,14 @@ __device__ __forceinline__ bool faces_away(float4 D, v3 x, v3 lo, v3 hi, float p
 // The same for one record: x beyond the margin on one side of both face planes at
 // both ends, hence all along the edge (4 dot products; the classification with its
 // closest point takes four divisions and two square roots).
-template <int DIM>
 __device__ __forceinline__ bool certainly_off(const SilRecord &s, v3 x, float prec)
 {
-    const v3 va = sub(x, s.pa), vb = DIM == 3 ? sub(x, s.pb) : va;
-    const float a0 = dot(s.n0, va), a1 = dot(s.n1, va);
-    const float b0 = DIM == 3 ? dot(s.n0, vb) : a0, b1 = DIM == 3 ? dot(s.n1, vb) : a1;
+    const v3 va = sub(x, s.pa), vb = sub(x, s.pb);
+    const float a0 = dot(s.n0, va), a1 = dot(s.n1, va), b0 = dot(s.n0, vb), b1 = dot(s.n1, vb);
     const float mn = fminf(fminf(a0, a1), fminf(b0, b1)), mx = fmaxf(fmaxf(a0, a1), fmaxf(b0, b1));
-    const float dm = __builtin_amdgcn_sqrtf(DIM == 3 ? fmaxf(dot(va, va), dot(vb, vb)) : dot(va, va)) * 1.00001f;
-    float c = fmaxf(fmaxf(fabsf(s.pa.x), fabsf(s.pa.y)), fabsf(s.pa.z));
-    if (DIM == 3) c = fmaxf(c, fmaxf(fmaxf(fabsf(s.pb.x), fabsf(s.pb.y)), fabsf(s.pb.z)));
+    const float dm = __builtin_amdgcn_sqrtf(fmaxf(dot(va, va), dot(vb, vb))) * 1.00001f;
+    const float ca = fmaxf(fmaxf(fabsf(s.pa.x), fabsf(s.pa.y)), fabsf(s.pa.z));
+    const float c = fmaxf(ca, fmaxf(fmaxf(fabsf(s.pb.x), fabsf(s.pb.y)), fabsf(s.pb.z)));
     const float m = prec * fmaxf(1.0f, dm) * 1.0001f + 4e-6f * (c + dm);
     return s.one != 1u && (mn > m || mx < -m);
 }
@@ -333,7 +331,7 @@ __device__ __forceinline__ float silhouette_distance(const SilRecord &s, v3 x, b
 // a child with a valid cone whose box overlaps the sphere and whose cone passes
 // BoundingCone.overlap (the reference's form, or cone_overlap_bounded, which
 // decides the same); a0, b0 are the children's squared box distances.
-template <int DIM, bool BOUNDED>
+template <int DIM, bool BOUNDED, bool FACES = false>
 __device__ __forceinline__ void silhouette_children(const DevScene &S, const SilScene &T, uint32_t cur, v3 x,
                                                     typename Geo<DIM>::vec xb, float r2, bool &oA, bool &oB,
                                                     float &a0, float &b0, uint32_t &lA, uint32_t &lB,
@@ -345,9 +343,8 @@ __device__ __forceinline__ void silhouette_children(const DevScene &S, const Sil
     G::record(S, cur, loA, hiA, lA, loB, hiB, lB);
     const float4 *cp = T.cones + (size_t)cur * 4;
     const float4 cA = cp[0], rA = cp[1], cB = cp[2], rB = cp[3];
-    const float none = __builtin_inff();
-    float4 fA = make_float4(0.0f, none, 0.0f, 0.0f), fB = fA;
-    if (BOUNDED && T.faces) {
+    float4 fA = make_float4(0.0f, 0.0f, 0.0f, 0.0f), fB = fA;
+    if (FACES) {
         fA = T.faces[(size_t)cur * 2];
         fB = T.faces[(size_t)cur * 2 + 1];
     }
@@ -358,7 +355,7 @@ __device__ __forceinline__ void silhouette_children(const DevScene &S, const Sil
     if (oA) {
         box_sqdist(loA, hiA, xb, a0, unused);
         oA = a0 <= r2;
-        if (BOUNDED && oA) oA = !faces_away(fA, x, to3(loA), to3(hiA), face_prec);
+        if (FACES && oA) oA = !faces_away(fA, x, to3(loA), to3(hiA), face_prec);
         if (oA) oA = BOUNDED ? cone_overlap_bounded(cA, rA, x, to3(loA), to3(hiA), a0)
                              : cone_overlap(cA, rA.x, x, to3(loA), to3(hiA), a0);
     }
@@ -366,7 +363,7 @@ __device__ __forceinline__ void silhouette_children(const DevScene &S, const Sil
     if (oB) {
         box_sqdist(loB, hiB, xb, b0, unused);
         oB = b0 <= r2;
-        if (BOUNDED && oB) oB = !faces_away(fB, x, to3(loB), to3(hiB), face_prec);
+        if (FACES && oB) oB = !faces_away(fB, x, to3(loB), to3(hiB), face_prec);
         if (oB) oB = BOUNDED ? cone_overlap_bounded(cB, rB, x, to3(loB), to3(hiB), b0)
                              : cone_overlap(cB, rB.x, x, to3(loB), to3(hiB), b0);
     }
@@ -477,7 +474,9 @@ struct SilShared {
     uint8_t left[256]; // the pairs that certainly_off does not decide
 };
 
-template <int DIM, int K>
+// FACES: subtrees dropped by their facing entries; PREPASS: records by
+// certainly_off (launch_silhouettes says when).
+template <int DIM, int K, bool FACES, bool PREPASS>
 __global__ __launch_bounds__(64) FCPW_EIGHT_WAVES void k_closest_silhouettes_coop(DevScene S, SilScene T, const float4 *spheres,
                                                                  const uint32_t *flip, int64_t n, float r2min,
                                                                  float prec, float2 *out, const uint32_t *order,
@@ -536,7 +535,7 @@ __global__ __launch_bounds__(64) FCPW_EIGHT_WAVES void k_closest_silhouettes_coo
                 uint32_t lA, lB;
                 float a0, b0;
                 bool oA, oB;
-                silhouette_children<DIM, true>(S, T, cur, x, xb, r2, oA, oB, a0, b0, lA, lB, face_prec);
+                silhouette_children<DIM, true, FACES>(S, T, cur, x, xb, r2, oA, oB, a0, b0, lA, lB, face_prec);
                 live = oA || oB;
                 if (oA && oB) {
                     uint32_t nearL = lA, farL = lB;
@@ -573,38 +572,56 @@ __global__ __launch_bounds__(64) FCPW_EIGHT_WAVES void k_closest_silhouettes_coo
             if (h2) sh.item[i2] = (uint16_t)((lane << 10) | (j0 + 2));
             if (h3) sh.item[i3] = (uint16_t)((lane << 10) | (j0 + 3));
             __syncthreads();
-            uint32_t n_left = 0;
-            for (uint32_t pass = 0; pass < total; pass += 64) {
-                const uint32_t kk = pass + (uint32_t)lane;
-                // every lane takes part in the permutes; lanes past the end read item 0
-                const uint32_t it = sh.item[kk < total ? kk : 0u];
-                const int src = (int)(it >> 10);
-                const v3 xo = {__shfl(x.x, src, 64), __shfl(x.y, src, 64), DIM == 3 ? __shfl(x.z, src, 64) : 0.0f};
-                const uint32_t off = __shfl(loff, src, 64);
-                bool maybe = kk < total;
-                if (maybe) {
-                    const SilRecord rec = load_silhouette<DIM>(T.sils, off + (it & 1023u));
-                    sh.index[kk] = rec.index;
-                    if (T.unit && certainly_off<DIM>(rec, xo, face_prec)) {
-                        sh.d[kk] = __builtin_nanf("");
-                        maybe = false;
+            if (PREPASS && T.unit) {
+                uint32_t n_left = 0;
+                for (uint32_t pass = 0; pass < total; pass += 64) {
+                    const uint32_t kk = pass + (uint32_t)lane;
+                    // every lane takes part in the permutes; lanes past the end read item 0
+                    const uint32_t it = sh.item[kk < total ? kk : 0u];
+                    const int src = (int)(it >> 10);
+                    const v3 xo = {__shfl(x.x, src, 64), __shfl(x.y, src, 64), __shfl(x.z, src, 64)};
+                    const uint32_t off = __shfl(loff, src, 64);
+                    bool maybe = kk < total;
+                    if (maybe) {
+                        const SilRecord rec = load_silhouette<DIM>(T.sils, off + (it & 1023u));
+                        sh.index[kk] = rec.index;
+                        if (certainly_off(rec, xo, face_prec)) {
+                            sh.d[kk] = __builtin_nanf("");
+                            maybe = false;
+                        }
+                    }
+                    const uint64_t mb = __ballot(maybe);
+                    if (maybe) sh.left[n_left + lanes_below(mb)] = (uint8_t)kk;
+                    n_left += __popcll(mb);
+                }
+                __syncthreads();
+                // what certainly_off leaves: about one record in five
+                for (uint32_t pass = 0; pass < n_left; pass += 64) {
+                    const bool on = pass + (uint32_t)lane < n_left;
+                    const uint32_t kk = sh.left[on ? pass + (uint32_t)lane : 0u], it = sh.item[kk];
+                    const int src = (int)(it >> 10);
+                    const v3 xo = {__shfl(x.x, src, 64), __shfl(x.y, src, 64), __shfl(x.z, src, 64)};
+                    const bool fo = __shfl(flu, src, 64) != 0u;
+                    const uint32_t off = __shfl(loff, src, 64);
+                    if (on)
+                        sh.d[kk] = silhouette_distance<DIM>(load_silhouette<DIM>(T.sils, off + (it & 1023u)), xo, fo,
+                                                            prec);
+                }
+            } else {
+                for (uint32_t pass = 0; pass < total; pass += 64) {
+                    const uint32_t kk = pass + (uint32_t)lane;
+                    // every lane takes part in the permutes; lanes past the end read item 0
+                    const uint32_t it = sh.item[kk < total ? kk : 0u];
+                    const int src = (int)(it >> 10);
+                    const v3 xo = {__shfl(x.x, src, 64), __shfl(x.y, src, 64), DIM == 3 ? __shfl(x.z, src, 64) : 0.0f};
+                    const bool fo = __shfl(flu, src, 64) != 0u;
+                    const uint32_t off = __shfl(loff, src, 64);
+                    if (kk < total) {
+                        const SilRecord rec = load_silhouette<DIM>(T.sils, off + (it & 1023u));
+                        sh.d[kk] = silhouette_distance<DIM>(rec, xo, fo, prec);
+                        sh.index[kk] = rec.index;
                     }
                 }
-                const uint64_t mb = __ballot(maybe);
-                if (maybe) sh.left[n_left + lanes_below(mb)] = (uint8_t)kk;
-                n_left += __popcll(mb);
-            }
-            __syncthreads();
-            // what certainly_off leaves: about one record in five
-            for (uint32_t pass = 0; pass < n_left; pass += 64) {
-                const bool on = pass + (uint32_t)lane < n_left;
-                const uint32_t kk = sh.left[on ? pass + (uint32_t)lane : 0u], it = sh.item[kk];
-                const int src = (int)(it >> 10);
-                const v3 xo = {__shfl(x.x, src, 64), __shfl(x.y, src, 64), DIM == 3 ? __shfl(x.z, src, 64) : 0.0f};
-                const bool fo = __shfl(flu, src, 64) != 0u;
-                const uint32_t off = __shfl(loff, src, 64);
-                if (on)
-                    sh.d[kk] = silhouette_distance<DIM>(load_silhouette<DIM>(T.sils, off + (it & 1023u)), xo, fo, prec);
             }
             __syncthreads();
             if (holding) {
@@ -645,11 +662,12 @@ __global__ __launch_bounds__(64) FCPW_EIGHT_WAVES void k_closest_silhouettes_coo
 
 // The facing entries of all slots (faces_away), from the records of the leaves
 // below each: slots shared out as in k_build_disks, a leaf's records listed at
-// its first primitive.
-template <int DIM>
+// its first primitive.  kept (when not null) counts those of at most DISK_OWN
+// primitives that have one.
 __global__ __launch_bounds__(DISK_BLOCK) void k_build_faces(const float4 *records, const int2 *ranges, int n_slots,
                                                             const int *big, int n_big, int own_blocks,
-                                                            const uint2 *sil_leaf, const float4 *sils, float4 *faces)
+                                                            const uint2 *sil_leaf, const float4 *sils, float4 *faces,
+                                                            int *kept)
 {
     const bool own = (int)blockIdx.x < own_blocks;
     int slot, step = 1, first = 0;
@@ -670,14 +688,14 @@ __global__ __launch_bounds__(DISK_BLOCK) void k_build_faces(const float4 *record
         return;
     }
     v3 lo, hi;
-    load_slot_box<DIM>(records, slot, lo, hi);
+    load_slot_box<3>(records, slot, lo, hi);
     const v3 c = {0.5f * (lo.x + hi.x), 0.5f * (lo.y + hi.y), 0.5f * (lo.z + hi.z)};
     v3 sum = {0.0f, 0.0f, 0.0f};
     bool bad = false;
     for (int k = first; k < rg.y; k += step) {
         const uint2 leaf = sil_leaf[rg.x + k];
         for (uint32_t j = 0; j < leaf.y; j++) {
-            const SilRecord r = load_silhouette<DIM>(sils, leaf.x + j);
+            const SilRecord r = load_silhouette<3>(sils, leaf.x + j);
             sum = {sum.x + r.n0.x + r.n1.x, sum.y + r.n0.y + r.n1.y, sum.z + r.n0.z + r.n1.z};
             bad = bad || r.one == 1u;
         }
@@ -696,13 +714,13 @@ __global__ __launch_bounds__(DISK_BLOCK) void k_build_faces(const float4 *record
     for (int k = first; k < rg.y; k += step) {
         const uint2 leaf = sil_leaf[rg.x + k];
         for (uint32_t j = 0; j < leaf.y; j++) {
-            const SilRecord r = load_silhouette<DIM>(sils, leaf.x + j);
+            const SilRecord r = load_silhouette<3>(sils, leaf.x + j);
             for (int f = 0; f < 2; f++) {
                 const v3 n = f ? r.n1 : r.n0;
                 const float nn = dot(n, n);
                 bad = bad || !(nn > 0.99999f && nn < 1.00001f);
                 cosine = fminf(cosine, dot(n, a));
-                for (int e = 0; e < (DIM == 3 ? 2 : 1); e++) {
+                for (int e = 0; e < 2; e++) {
                     const v3 p = e ? r.pb : r.pa, w = sub(p, c);
                     const float o = dot(n, w);
                     bad = bad || !(fabsf(o) < 1e18f);
@@ -730,6 +748,7 @@ __global__ __launch_bounds__(DISK_BLOCK) void k_build_faces(const float4 *record
         faces[slot] = none;
         return;
     }
+    if (kept && own) atomicAdd(kept, 1);
     const float tangent = sqrtf(fmaxf(1.0f - cosine * cosine, 0.0f)) / cosine * (1.0f + 1e-5f);
     const float R = sqrtf(far2) * (1.0f + 1e-5f), pad = 8e-6f * (coord + R);
     const float delta = inv - 1.0f;

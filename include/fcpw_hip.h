@@ -371,7 +371,7 @@ int fcpw_hip_batch_get_option(const fcpw_hip_batch *batch, const char *key, int 
                  uploaded single-object scene reorders the records in place, and later
                  uploads and device builds of the context use it
      "sil_stack", "inst_stack"  LDS stack entries of the 3D cooperative silhouette kernel
-                 (4, 8 or 12, default 4) and of the 3D cooperative instanced closest-point
+                 (8 or 12; the default 4 means 4 or 8, by the uploaded silhouettes) and of the 3D cooperative instanced closest-point
                  kernel (8 or 12, default 12)
      "ray_sort_dir"  1 = rays ordered by direction octant (quadrant), then by origin
                  along the Morton curve (default); 0 = by origin only
@@ -398,8 +398,8 @@ int fcpw_hip_batch_get_option(const fcpw_hip_batch *batch, const char *key, int 
                  changes a record; B = 1024 by default, 64..2^20, 0 = one launch
                  Until the option is set, batches below 2^21 queries run as one
                  launch, which is then the faster form.  Likewise
-                 "stack" and "sil_stack": until set, closest points in batches of at
-                 most 16 waves a CU take twelve entries, and silhouettes eight
+                 "stack": until set, closest points in batches of at most 16 waves a
+                 CU take twelve entries
      "bwd_order" 1 = the adjoint walks the queries in the Morton order the latest
                  query call on this context computed, when that batch had the same
                  size (default); 0 = in the caller's order

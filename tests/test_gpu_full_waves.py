@@ -1,0 +1,62 @@
+"""The cooperative kernels with 64 queries in every wave (batches of at least
+eight waves a CU), where leaf passes take several groups of 64: the same records
+as the one-query-per-lane kernels, bit for bit, for the knobs they read."""
+import numpy as np
+import pytest
+
+from fcpw_amd import synth
+from tests import meshes
+from tests.test_gpu_disks import CASES, queries
+from tests.test_gpu_silhouettes import gpu_scene, records
+from tests.test_oracle_silhouettes import product_scene
+
+pytestmark = pytest.mark.gpu
+fcpw = pytest.importorskip("fcpw_amd")
+
+
+def full(g):
+    """a batch of full waves, the last one ragged"""
+    return 512 * g.info("n_cus") + 77
+
+
+def noisy_sphere(amplitude):
+    v, f = synth.geodesic_sphere(12)
+    return synth.f32(synth.radial_noise(v, amplitude, synth.Rng(9))), f.astype(np.int32)
+
+
+# with facing entries and prepass, with the prepass alone, and with neither
+SILHOUETTES = {
+    "torus": (lambda: meshes.small_torus(64, 32), 8),
+    "noisy": (lambda: noisy_sphere(0.05), 8),
+    "spiky": (lambda: noisy_sphere(0.6), 4),
+    "soup": (CASES["soup"], 4),
+    "open_plate": (CASES["plate_tilted"], 8),
+    "star2d": (CASES["star2d"], 8),
+}
+
+
+@pytest.mark.parametrize("name", sorted(SILHOUETTES))
+def test_silhouettes(gpu, name):
+    make, entries = SILHOUETTES[name]
+    V, F = make()
+    g = gpu_scene(product_scene(V, F), V.shape[1])
+    n = full(g)
+    q = queries(V, n, 71)[:n]
+    flip = (np.arange(n) % 2).astype(np.int32)
+    r2 = np.full(n, np.inf, np.float32)
+    r2[1::3] = np.float32((0.3 * float((V.max(0) - V.min(0)).max())) ** 2)
+
+    def run(**opts):
+        for key, value in opts.items():
+            g.set_option(key, value)
+        hits = fcpw.GPUInteractionList()
+        g.find_closest_silhouette_points(q, r2, flip, hits)
+        return records(hits).tobytes()
+
+    ref = run(coop=0)
+    for hold in (3, 1, 64):
+        assert run(coop=1, sil_hold_min=hold) == ref, hold
+        assert g.info("launch_wave_queries") == 64 and g.info("launch_hold_min") == hold
+        assert g.info("launch_stack") == entries
+    for k in (8, 12):
+        assert run(sil_stack=k, sil_hold_min=3) == ref, k
