@@ -5,8 +5,10 @@ import numpy as np
 import pytest
 
 from fcpw_amd import synth
-from tests import meshes
+from tests import meshes, scenes
 from tests.test_gpu_disks import CASES, queries
+from tests.test_gpu_instances import setup
+from tests.test_gpu_parity import as_records, make_scene
 from tests.test_gpu_silhouettes import gpu_scene, records
 from tests.test_oracle_silhouettes import product_scene
 
@@ -60,3 +62,73 @@ def test_silhouettes(gpu, name):
         assert g.info("launch_stack") == entries
     for k in (8, 12):
         assert run(sil_stack=k, sil_hold_min=3) == ref, k
+
+
+@pytest.mark.parametrize("mesh", ["torus", "star2d"])
+@pytest.mark.parametrize("occlusion", [False, True])
+def test_rays(gpu, mesh, occlusion):
+    V, F = meshes.small_torus(48, 24) if mesh == "torus" else meshes.small_star(3000)
+    _, g = make_scene(V, F)
+    n = full(g)
+    o, d = meshes.rays_from(V, n, seed=72)
+    tmax = np.full(n, np.inf, np.float32)
+    tmax[::7] = 0.3
+
+    def run(**opts):
+        for key, value in opts.items():
+            g.set_option(key, value)
+        hits = fcpw.GPUInteractionList()
+        g.intersect(o, d, tmax, hits, check_for_occlusion=occlusion)
+        return as_records(hits).tobytes()
+
+    ref = run(ray_coop=0)
+    for hold in (1, 8, 64):
+        assert run(ray_coop=1, ray_hold_min=hold) == ref, hold
+        assert g.info("launch_wave_queries") == 64 and g.info("launch_hold_min") == hold
+
+
+@pytest.mark.parametrize("mesh", ["torus", "soup", "star2d"])
+def test_closest_points(gpu, mesh):
+    V, F = meshes.small_torus(64, 32) if mesh == "torus" else CASES[mesh]()
+    _, g = make_scene(V, F)
+    n = full(g)
+    q = queries(V, n, 73)[:n]
+    r2 = np.full(n, np.inf, np.float32)
+    r2[1::3] = np.float32((0.05 * float((V.max(0) - V.min(0)).max())) ** 2)
+
+    def run(**opts):
+        for key, value in opts.items():
+            g.set_option(key, value)
+        hits = fcpw.GPUInteractionList()
+        g.find_closest_points(q, r2, hits, record_normals=True)
+        return as_records(hits).tobytes()
+
+    ref = run(coop=0)
+    for hold in (1, 8, 64):
+        for k in (6, 12):
+            assert run(coop=1, hold_min=hold, stack=k) == ref, (hold, k)
+            assert g.info("launch_wave_queries") == 64 and g.info("launch_hold_min") == hold
+
+
+@pytest.mark.parametrize("name", scenes.NAMES + ["crowd3d"])
+def test_instances(gpu, name):
+    objs, tr, s, g, bv, I = setup(name)
+    n = full(g)
+    q = scenes.queries(objs, tr, n, seed=74)
+    r2 = np.full(n, np.inf, np.float32)
+    r2[1::3] = np.float32(0.04)
+
+    def run(**opts):
+        for key, value in opts.items():
+            g.set_option(key, value)
+        hits = fcpw.GPUInteractionList()
+        obj = np.full(n, -7, np.int32)
+        g.find_closest_points(q, r2, hits, record_normals=True, object_indices=obj)
+        return records(hits).tobytes() + obj.tobytes()
+
+    try:
+        ref = run(coop=0)
+        for hold in (1, 8, 64):
+            assert run(coop=1, hold_min=hold) == ref, hold
+    finally:
+        run(coop=1, hold_min=1)
