@@ -12,7 +12,7 @@ static float bits_as_float(uint32_t u)
 }
 
 // defaults that stand for a rule on sizes or on the mesh
-constexpr int RAY_HOLD_DEFAULT = 8, SIL_STACK_DEFAULT = 4;
+constexpr int STACK_DEFAULT = 6, RAY_HOLD_DEFAULT = 8, SIL_STACK_DEFAULT = 4, INST_SEED_DEFAULT = 1024;
 
 struct fcpw_hip_ctx {
     int device = 0;
@@ -88,11 +88,10 @@ struct fcpw_hip_ctx {
     // facts
     int n_records = 0, n_leaves = 0, n_prims = 0, n_vertices = 0, max_depth = 0;
     // options
-    int block = 128, stack = 6, sort = 1, xcds = 4, coop = 1, hold_min = 1, morton_bits = 24;
+    int block = 128, stack = STACK_DEFAULT, sort = 1, xcds = 4, coop = 1, hold_min = 1, morton_bits = 24;
     int xcd_chunk = 0; // log2 tiles per XCD chunk of the tile mapping (0: one range per XCD)
     int ray_coop = 1; // wave-cooperative leaves for ray queries
     int ray_sort_dir = 1; // rays ordered by direction octant, then origin
-    bool stack_auto = true; // stack not set by the caller: by the batch size (launch_closest_kernel)
     // the cooperative ray kernels' LDS stack entries and leaf-pass threshold (the
     // default: by the batch size, launch_intersect)
     int ray_stack = 4, ray_hold_min = RAY_HOLD_DEFAULT;
@@ -102,10 +101,9 @@ struct fcpw_hip_ctx {
     int layout = 0;                      // record order in memory: 0 DFS, 1 treelets of three levels
     int sil_hold_min = 3;                // the cooperative silhouette kernel's leaf-pass threshold
     int sil_xcds = 8;                    // the silhouette kernels' XCD grouping
-    int inst_seed = 1024;                // instanced closest points: ordered queries per representative wave (0: off)
-    bool inst_seed_auto = true;          // not set by the caller: only batches that gain from it (launch_instances_closest)
+    int inst_seed = INST_SEED_DEFAULT;   // instanced closest points: ordered queries per representative wave (0: off)
     // what the latest cooperative launch took of the options and size rules
-    struct { int stack, hold_min, wave_queries; } launch = {0, 0, 0};
+    struct { int stack, hold_min, wave_queries, block; } launch = {0, 0, 0, 0};
     int stats_on = 0, timing = 0;
     int n_cus = 256;
     // device scratch of fcpw_hip_build_bvh, kept (grow-only) for the next build

@@ -1179,10 +1179,10 @@ static int launch_closest_kernel(fcpw_hip_ctx *c, const CpIO &io, hipStream_t s,
                        wq)
         // 0, 4, 6, 8, 12, 16 or 24 LDS entries (2D: 24 runs as 16).  Six keep eight
         // waves a SIMD, which a batch of at most 16 waves a CU does not make: unless
-        // the caller set the option it takes twelve and spills less (100,003 queries
+        // the caller chose another number it takes twelve and spills less (100,003 queries
         // 165 -> 160 us, 30,000 in 2D 317 -> 306, 12,000 on 300,000 triangles 851 -> 820).
-        const int k = c->stack_auto && (int64_t)g.x <= (int64_t)16 * c->n_cus ? 12 : c->stack;
-        c->launch = {k, c->hold_min, wq};
+        const int k = c->stack == STACK_DEFAULT && (int64_t)g.x <= (int64_t)16 * c->n_cus ? 12 : c->stack;
+        c->launch = {k, c->hold_min, wq, 0};
         if (c->dim == 3) {
             if (k == 0) FCPW_COOP(3, 0);
             else if (k == 4) FCPW_COOP(3, 4);
@@ -1278,7 +1278,7 @@ static int launch_intersect(fcpw_hip_ctx *c, const void *rays, int64_t n, int oc
         const int hold = wq < 64 && c->ray_hold_min == RAY_HOLD_DEFAULT ? 1 : c->ray_hold_min;
         const dim3 g = grid_for(c, n, wq);
         const int k = c->ray_stack;
-        c->launch = {k, hold, wq};
+        c->launch = {k, hold, wq, 0};
 #define FCPW_RCOOP(D, K, ST)                                                                                  \
     hipLaunchKernelGGL((k_intersect_coop<D, K, ST>), g, dim3(64), 0, s, S, (const float2 *)rays, n, occlusion, \
                        (float2 *)out, order, xcd_arg(c), hold, wq)
@@ -1513,7 +1513,7 @@ static int launch_silhouettes(fcpw_hip_ctx *c, const void *spheres, const uint32
         // whose spills cost more (131,072-triangle torus 11.0 ms, four 13.0).
         const bool faces = c->sil_faces, pre = c->dim == 3 && (faces || c->sil_open < 0.315f);
         const int k = c->dim == 2 ? 8 : c->sil_stack != SIL_STACK_DEFAULT ? c->sil_stack : pre ? 8 : 4;
-        c->launch = {k, c->sil_hold_min, wq};
+        c->launch = {k, c->sil_hold_min, wq, 0};
 #define FCPW_SIL(DIM, K, FACES, PREPASS)                                                                      \
     hipLaunchKernelGGL((k_closest_silhouettes_coop<DIM, K, FACES, PREPASS>), g, dim3(64), 0, s, S, T,         \
                        (const float4 *)spheres, flip, n, r2min, prec, (float2 *)out, order, sil_xcd_arg(c),   \
@@ -1672,7 +1672,6 @@ int fcpw_hip_set_option(fcpw_hip_ctx *c, const char *key, int value)
         if (value != 0 && value != 4 && value != 6 && value != 8 && value != 12 && value != 16 && value != 24)
             FAIL(c, FCPW_HIP_ERR_INVALID_ARGUMENT, "stack must be 0, 4, 6, 8, 12, 16 or 24");
         c->stack = value;
-        c->stack_auto = false;
     } else if (k == "sort") {
         if (value != 0 && value != 1) FAIL(c, FCPW_HIP_ERR_INVALID_ARGUMENT, "sort must be 0 or 1");
         c->sort = value;
@@ -1704,7 +1703,6 @@ int fcpw_hip_set_option(fcpw_hip_ctx *c, const char *key, int value)
         if (value != 0 && (value < 64 || value > (1 << 20)))
             FAIL(c, FCPW_HIP_ERR_INVALID_ARGUMENT, "inst_seed must be 0 or in [64, 2^20]");
         c->inst_seed = value;
-        c->inst_seed_auto = false;
     } else if (k == "xcd_chunk") {
         if (value < 0 || value > 16) FAIL(c, FCPW_HIP_ERR_INVALID_ARGUMENT, "xcd_chunk must be in [0, 16]");
         c->xcd_chunk = value;
@@ -1778,6 +1776,7 @@ int fcpw_hip_get_info(const fcpw_hip_ctx *c, const char *key, int64_t *value)
     else if (k == "launch_stack") *value = c->launch.stack;
     else if (k == "launch_hold_min") *value = c->launch.hold_min;
     else if (k == "launch_wave_queries") *value = c->launch.wave_queries;
+    else if (k == "launch_block") *value = c->launch.block;
     else if (k == "n_instances") *value = c->instanced ? c->n_instances : 0;
     else if (k == "n_objects") *value = c->instanced ? (int64_t)c->inst_objects.size() : (c->uploaded ? 1 : 0);
     else if (k.rfind("stat_", 0) == 0) {

@@ -1303,10 +1303,11 @@ static int launch_instances_closest(fcpw_hip_ctx *c, const void *spheres, int64_
     // the rest with radii lowered from them (seeded_r2); otherwise one launch.
     // Two launches end twice with their longest walks (2.4 ms with 256 instances
     // of 20,480 triangles, where one launch of 16,384 queries takes all of that),
-    // so unless the caller asked for it the batch has to be large: 1M queries
+    // so unless the caller chose a block the batch has to be large: 1M queries
     // there 8.6 ms in one launch against 9.8 in two, 4M 24.0 against 20.5.
-    const bool seed = c->inst_seed > 0 && (!c->inst_seed_auto || n >= ((int64_t)1 << 21));
+    const bool seed = c->inst_seed > 0 && (c->inst_seed != INST_SEED_DEFAULT || n >= ((int64_t)1 << 21));
     const int block = order && seed ? c->inst_seed : 0;
+    c->launch.block = block;
     const bool coop = c->coop && c->max_depth + c->inst_obj_depth < STACK_TOTAL;
     for (int pass = block ? 0 : 1; pass < 2; pass++) {
         const int64_t m = pass == 0 ? (n + block - 1) / block * 64 : n;

@@ -357,6 +357,7 @@ int fcpw_hip_batch_get_option(const fcpw_hip_batch *batch, const char *key, int 
 
 /* Tuning knobs read by the kernels (values chosen by fcpw_amd.autotune).  None
    of them changes a result bit: every setting visits nodes in the same order.
+   Where a default stands for a rule, setting the default sets the rule again.
      "coop"      1 = wave-cooperative leaf processing (default), 0 = one query per
                  lane with the leaf loop inline (closest points, on single-object and
                  instanced scenes, and closest silhouette points)
@@ -377,7 +378,8 @@ int fcpw_hip_batch_get_option(const fcpw_hip_batch *batch, const char *key, int 
                  along the Morton curve (default); 0 = by origin only
      "hold_min"  coop: lanes that must hold a leaf before the wave processes
                  leaves together (1..64, default 1)
-     "stack"     traversal-stack entries per lane kept in LDS (default 6): the newest
+     "stack"     traversal-stack entries per lane kept in LDS (the default 6 means 6, and
+                 12 for closest points in batches of at most 16 waves a CU): the newest
                  entries, as a sliding window; older ones are spilled once to cached
                  scratch: 0, 4, 6, 8, 12, 16 or 24 (the 2D coop kernel uses 16 for 24,
                  the one-query-per-lane kernel 8 for 0, 4, 6 and 12)
@@ -395,11 +397,8 @@ int fcpw_hip_batch_get_option(const fcpw_hip_batch *batch, const char *key, int 
                  64 in its middle first, then the others with their radius lowered
                  to an upper bound from the nearest of those (its distance plus the
                  distance between the two queries, with margins), which never
-                 changes a record; B = 1024 by default, 64..2^20, 0 = one launch
-                 Until the option is set, batches below 2^21 queries run as one
-                 launch, which is then the faster form.  Likewise
-                 "stack": until set, closest points in batches of at most 16 waves a
-                 CU take twelve entries
+                 changes a record; 64..2^20, 0 = one launch; the default 1024 means
+                 two launches from 2^21 queries on and one, then the faster form, below
      "bwd_order" 1 = the adjoint walks the queries in the Morton order the latest
                  query call on this context computed, when that batch had the same
                  size (default); 0 = in the caller's order
@@ -428,7 +427,8 @@ int fcpw_hip_get_option(const fcpw_hip_ctx *ctx, const char *key, int *value);
    tuning knobs below only "sort", "morton_bits" and "xcds" apply to them.
    launch_stack, launch_hold_min and launch_wave_queries: the LDS stack entries,
    leaf-pass threshold and queries per wave that the latest launch of a cooperative
-   single-object kernel took (0 before the first).
+   single-object kernel took (0 before the first); launch_block: the block of the
+   latest instanced closest-point call (0 = one launch).
    Measurement: stat_internal_nodes, stat_prim_tests,
    stat_queries and, for closest-point launches, stat_waves, stat_wave_iterations,
    stat_leaf_passes, stat_leaf_groups (cooperative leaf passes and their 64-item

@@ -6,8 +6,9 @@ import numpy as np
 import pytest
 
 import oracle
-from tests import meshes
+from tests import meshes, scenes
 from tests.test_gpu_disks import check, queries
+from tests.test_gpu_instances import setup
 from tests.test_gpu_parity import as_records, assert_bit_equal, make_scene
 
 pytestmark = pytest.mark.gpu
@@ -53,3 +54,39 @@ def test_a_chosen_leaf_pass_threshold_is_kept(gpu):
         assert g.info("launch_wave_queries") < 64 and g.info("launch_hold_min") == part_filled
         cast(g, full)
         assert g.info("launch_wave_queries") == 64 and g.info("launch_hold_min") == value
+
+
+def test_a_default_written_back_is_the_size_rule_again(gpu):
+    """reading an option and setting it to what was read changes nothing"""
+    _, g = make_scene(*meshes.small_torus(48, 24))
+    n_small, n_full = 1000, 2048 * g.info("n_cus")
+    q = queries(meshes.small_torus(48, 24)[0], n_full, 3)[:n_full]
+
+    def entries(n):
+        g.find_closest_points(q[:n], np.full(n, np.inf, np.float32), fcpw.GPUInteractionList())
+        return g.info("launch_stack")
+
+    default = g.get_option("stack")
+    assert default == 6
+    for _ in range(2):
+        assert (entries(n_small), entries(n_full)) == (12, 6)
+        g.set_option("stack", 8)
+        assert (entries(n_small), entries(n_full)) == (8, 8)
+        g.set_option("stack", default)
+
+
+def test_a_default_block_written_back_is_the_size_rule_again(gpu):
+    objs, tr, s, g, bv, I = setup("crowd3d")
+    q = scenes.queries(objs, tr, 5000, seed=3)
+
+    def block():
+        g.find_closest_points(q, np.full(len(q), np.inf, np.float32), fcpw.GPUInteractionList())
+        return g.info("launch_block")
+
+    default = g.get_option("inst_seed")
+    assert default == 1024
+    for _ in range(2):
+        assert block() == 0
+        g.set_option("inst_seed", 512)
+        assert block() == 512
+        g.set_option("inst_seed", default)
