@@ -40,6 +40,8 @@ struct fcpw_hip_ctx {
     int *big = nullptr, *frontier = nullptr, *range_info = nullptr;
     uint32_t *range_mark = nullptr, *range_sums = nullptr;
     float *disk_limit = nullptr;
+    unsigned long long *disk_tally = nullptr;
+    bool disks_off = true; // known on the host: they are off until the next refit or upload
     bool by_range = false, one_tree = false;
     int n_big = 0, n_top = 0, n_frontier = 0;
     int *flags = nullptr;
@@ -162,6 +164,8 @@ static void free_scene(fcpw_hip_ctx *c)
     c->big = c->frontier = c->range_info = nullptr;
     c->range_mark = c->range_sums = nullptr;
     c->disk_limit = nullptr;
+    c->disk_tally = nullptr;
+    c->disks_off = true;
     c->by_range = false;
     c->inst = nullptr;
     c->obj_table = nullptr;

@@ -331,13 +331,15 @@ __device__ __forceinline__ void store_p(v2 p, float o[3]) { o[0] = p.x; o[1] = p
 // so r^2, the order of the remaining visits and the result are the
 // reference's bit for bit; only visits that accept nothing are left out.
 // Counts on the 1M-triangle torus (half uniform, half near): 162 expanded
-// records and 185 primitive tests a query with boxes alone, 60 and 35 with the
+// records and 185 primitive tests a query with boxes alone, 59 and 32 with the
 // disks.  The kernel is bound by VALU issue and a step costs half as much again
-// (two bounds of 28 instructions), so 16.8M queries there went from 53.9 to
+// (two bounds of 24 instructions), so 16.8M queries there went from 53.9 to
 // 14.6 ms, 8.4M on a 262,144-segment polygon from 11.3 to 5.8 ms, 1M inside a
-// noisy sphere from 8.2 to 1.0 ms; 4.2M within 0.1 of a sphere whose noise is as
-// large as its triangles, where disks exclude next to nothing, from 2.00 to
-// 2.09 ms.
+// noisy sphere from 8.2 to 1.0 ms.  Where the first leaf already holds the answer
+// the disks cost and exclude nothing: 2.1M queries within 0.001 of a smooth
+// surface 0.63 -> 0.65 ms, 4.2M within 0.1 of a sphere whose noise is as large as
+// its triangles 2.32 -> 2.39.  Testing only the farther of two children, or none
+// that holds the query, lost more (16.8M on the torus 21.1 ms; a rough sphere +10%).
 //
 // 16 bytes a slot: {n.x, n.y (f16)} {n.z (f16), o (bf16)} {t, rho (bf16)}
 // {0.5 / |n| (f32); 0: no disk}.  n is rounded first and o, t and rho are
@@ -985,7 +987,9 @@ __device__ __forceinline__ void wave_loop_stats_add(const DevScene &S, uint32_t 
     }
 }
 
-template <int DIM, int K, int OUT, bool STATS>
+// DISK false: for a tree whose disks are off (launch_closest_kernel), and for the
+// counting variant, which visits what the reference visits
+template <int DIM, int K, int OUT, bool STATS, bool DISK = !STATS>
 __global__ __launch_bounds__(64) void k_closest_points_coop(DevScene S, CpIO io, int xcds, int hold_min,
                                                             int wave_q)
 {
@@ -995,8 +999,7 @@ __global__ __launch_bounds__(64) void k_closest_points_coop(DevScene S, CpIO io,
     float q[3] = {0.0f, 0.0f, 0.0f}, r2 = -1.0f;
     if (valid) cp_load<DIM, OUT>(io, i, q, r2);
     CpResult r;
-    // the counting variant visits what the reference visits
-    closest_point_query_coop<DIM, K, !STATS>(S, Geo<DIM>::load_point(q), r2, valid, hold_min, r);
+    closest_point_query_coop<DIM, K, DISK>(S, Geo<DIM>::load_point(q), r2, valid, hold_min, r);
     if (valid) cp_store<DIM, OUT>(S, io, i, r);
     if (STATS) {
         wave_stats_add(S, r.n_internal, r.n_prims, valid ? 1u : 0u);
@@ -2010,11 +2013,22 @@ __device__ __forceinline__ float4 disk_pack(const DiskSums &D, v3 half, v3 n, ui
 // Slots above DISK_MAX_PRIMS have none.  Queries whose root box's farthest
 // corner lies beyond disk_limit go without, and all queries where the boxes do
 // not hold their primitives (info[3], k_slot_ranges; null after a refit).
+// Where fewer than DISK_KEPT_MIN of the slots of at most DISK_OWN primitives keep
+// a disk, the walk drops next to nothing by them and pays their loads: they then
+// stay off as a whole.  8.4M queries, half of them near, with disks and without:
+// triangle soups that keep 0.24 of them 4.19 ms and 3.95, 0.35 3.72 and 3.48, 0.39
+// 2.15 and 2.04, 0.46 4.45 and 4.34, 0.47 11.6 and 11.2; noisy spheres that keep 0.59
+// 5.71 and 6.04 (200,000 triangles) and 3.60 and 3.39 (20,000), 0.66 3.55 and 3.54, 0.75
+// 10.1 and 11.1.  tally counts the kept slots (upper half) and the blocks that have
+// added theirs; the last one decides.
+constexpr float DISK_KEPT_MIN = 0.5f;
+
 template <int DIM>
 __global__ __launch_bounds__(DISK_BLOCK) void k_build_disks(const float4 *records, const float4 *root,
                                                             const float4 *prims, const int2 *ranges, int n_slots,
-                                                            const int *big, int n_big, int own_blocks, float4 *disks,
-                                                            float *disk_limit, const int *info)
+                                                            const int *big, int n_big, int n_own, int own_blocks,
+                                                            float4 *disks, float *disk_limit, const int *info,
+                                                            unsigned long long *tally)
 {
     v3 rlo, rhi;
     load_root_box<DIM>(root, rlo, rhi);
@@ -2022,17 +2036,14 @@ __global__ __launch_bounds__(DISK_BLOCK) void k_build_disks(const float4 *record
     const float reach = 1.5f * sqrtf(dot(ext, ext)); // queries in 1.5 times the box and beyond
     const float scale = fmaxf(fmaxf(fmaxf(fabsf(rlo.x), fabsf(rhi.x)), fmaxf(fabsf(rlo.y), fabsf(rhi.y))),
                               fmaxf(fabsf(rlo.z), fabsf(rhi.z)));
-    // the bound's squares neither overflow (1e37) nor leave the normal range
-    // (1e-6: a disk excludes no distance below 1e-6 of the coordinates)
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-        *disk_limit = reach >= 1e-6f && !(info && info[3]) ? fminf(reach * reach, 1e37f) : -1.0f;
     const bool own = (int)blockIdx.x < own_blocks;
     int slot, step, first;
+    bool on = true;
     if (own) {
         slot = (int)blockIdx.x * DISK_BLOCK + (int)threadIdx.x;
         first = 0;
         step = 1;
-        if (slot >= n_slots) return;
+        on = slot < n_slots;
     } else {
         const int w = ((int)blockIdx.x - own_blocks) * (DISK_BLOCK / 64) + (int)(threadIdx.x >> 6);
         if (w >= n_big) return;
@@ -2040,39 +2051,52 @@ __global__ __launch_bounds__(DISK_BLOCK) void k_build_disks(const float4 *record
         first = (int)(threadIdx.x & 63u);
         step = 64;
     }
-    const int2 rg = ranges[slot];
+    int2 rg = make_int2(0, 0);
+    if (on) rg = ranges[slot];
     if (own && rg.y > DISK_OWN) {
         if (rg.y > DISK_MAX_PRIMS) disks[slot] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        return;
+        on = false;
     }
-    v3 lo, hi;
-    load_slot_box<DIM>(records, slot, lo, hi);
-    const v3 c2 = {lo.x + hi.x, lo.y + hi.y, lo.z + hi.z};
-    const v3 half = {0.5f * (hi.x - lo.x), 0.5f * (hi.y - lo.y), 0.5f * (hi.z - lo.z)};
-    DiskSums D = {{0, 0, 0}, INFINITY, -INFINITY, 0.0f, 0.0f, 0.0f};
-    for (int k = first; k < rg.y; k += step) disk_normal_add<DIM>(prims, rg.x + k, D);
-    if (!own)
-        for (int off = 32; off > 0; off >>= 1) {
-            D.n.x += __shfl_xor(D.n.x, off, 64);
-            D.n.y += __shfl_xor(D.n.y, off, 64);
-            D.n.z += __shfl_xor(D.n.z, off, 64);
-        }
-    v3 n;
-    uint32_t nxy, nz;
-    float inv;
-    disk_round_normal(D.n, n, nxy, nz, inv);
-    for (int k = first; k < rg.y; k += step) disk_extent_add<DIM>(prims, rg.x + k, c2, n, reach, D);
-    if (!own) {
-        for (int off = 32; off > 0; off >>= 1) {
-            D.lo = fminf(D.lo, __shfl_xor(D.lo, off, 64));
-            D.hi = fmaxf(D.hi, __shfl_xor(D.hi, off, 64));
-            D.l2 = fmaxf(D.l2, __shfl_xor(D.l2, off, 64));
-            D.mt = fmaxf(D.mt, __shfl_xor(D.mt, off, 64));
-            D.mr = fmaxf(D.mr, __shfl_xor(D.mr, off, 64));
-        }
-        if (first != 0) return;
+    float4 packed = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (on) {
+        v3 lo, hi;
+        load_slot_box<DIM>(records, slot, lo, hi);
+        const v3 c2 = {lo.x + hi.x, lo.y + hi.y, lo.z + hi.z};
+        const v3 half = {0.5f * (hi.x - lo.x), 0.5f * (hi.y - lo.y), 0.5f * (hi.z - lo.z)};
+        DiskSums D = {{0, 0, 0}, INFINITY, -INFINITY, 0.0f, 0.0f, 0.0f};
+        for (int k = first; k < rg.y; k += step) disk_normal_add<DIM>(prims, rg.x + k, D);
+        if (!own)
+            for (int off = 32; off > 0; off >>= 1) {
+                D.n.x += __shfl_xor(D.n.x, off, 64);
+                D.n.y += __shfl_xor(D.n.y, off, 64);
+                D.n.z += __shfl_xor(D.n.z, off, 64);
+            }
+        v3 n;
+        uint32_t nxy, nz;
+        float inv;
+        disk_round_normal(D.n, n, nxy, nz, inv);
+        for (int k = first; k < rg.y; k += step) disk_extent_add<DIM>(prims, rg.x + k, c2, n, reach, D);
+        if (!own)
+            for (int off = 32; off > 0; off >>= 1) {
+                D.lo = fminf(D.lo, __shfl_xor(D.lo, off, 64));
+                D.hi = fmaxf(D.hi, __shfl_xor(D.hi, off, 64));
+                D.l2 = fmaxf(D.l2, __shfl_xor(D.l2, off, 64));
+                D.mt = fmaxf(D.mt, __shfl_xor(D.mt, off, 64));
+                D.mr = fmaxf(D.mr, __shfl_xor(D.mr, off, 64));
+            }
+        packed = disk_pack(D, half, n, nxy, nz, inv, scale);
+        if (first == 0) disks[slot] = packed;
     }
-    disks[slot] = disk_pack(D, half, n, nxy, nz, inv, scale);
+    if (!own) return;
+    const int kept = __syncthreads_count(packed.w != 0.0f);
+    if (threadIdx.x != 0) return;
+    const unsigned long long before = atomicAdd(tally, ((unsigned long long)kept << 32) | 1ull);
+    if ((int)(before & 0xFFFFFFFFull) != own_blocks - 1) return;
+    *tally = 0;
+    // the bound's squares neither overflow (1e37) nor leave the normal range
+    // (1e-6: a disk excludes no distance below 1e-6 of the coordinates)
+    const bool pay = (float)((int)(before >> 32) + kept) >= DISK_KEPT_MIN * (float)n_own;
+    *disk_limit = pay && reach >= 1e-6f && !(info && info[3]) ? fminf(reach * reach, 1e37f) : -1.0f;
 }
 
 // Adjoint of d(x, mesh): recompute p and its barycentric weights from the saved

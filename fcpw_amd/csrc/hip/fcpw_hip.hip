@@ -75,12 +75,12 @@ static int launch_disks(fcpw_hip_ctx *c, hipStream_t s, const int *info = nullpt
     const int n_slots = 2 * c->n_records;
     if (c->dim == 3)
         hipLaunchKernelGGL(k_build_disks<3>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->root, c->prims,
-                           c->ranges, n_slots, c->big, c->n_big, slot_own_blocks(c), c->disks, c->disk_limit,
-                           info);
+                           c->ranges, n_slots, c->big, c->n_big, n_slots - c->n_big - c->n_top, slot_own_blocks(c),
+                           c->disks, c->disk_limit, info, c->disk_tally);
     else
         hipLaunchKernelGGL(k_build_disks<2>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->root, c->prims,
-                           c->ranges, n_slots, c->big, c->n_big, slot_own_blocks(c), c->disks, c->disk_limit,
-                           info);
+                           c->ranges, n_slots, c->big, c->n_big, n_slots - c->n_big - c->n_top, slot_own_blocks(c),
+                           c->disks, c->disk_limit, info, c->disk_tally);
     HIPCHECK(c, hipGetLastError());
     return FCPW_HIP_OK;
 }
@@ -100,6 +100,7 @@ template <int DIM>
 static int compute_ranges(fcpw_hip_ctx *c)
 {
     c->by_range = false;
+    c->disks_off = true;
     c->n_big = c->n_top = c->n_frontier = 0;
     const float none = -1.0f;
     HIPCHECK(c, hipMemcpy(c->disk_limit, &none, sizeof(float), hipMemcpyHostToDevice));
@@ -109,6 +110,7 @@ static int compute_ranges(fcpw_hip_ctx *c)
     const int n_slots = 2 * c->n_records, t = 256;
     const dim3 gs((unsigned)((n_slots + t - 1) / t));
     HIPCHECK(c, hipMemset(c->range_info, 0, 4 * sizeof(int)));
+    HIPCHECK(c, hipMemset(c->disk_tally, 0, sizeof(unsigned long long)));
     HIPCHECK(c, hipMemset(c->range_mark, 0, ((size_t)c->n_prims + 1) * sizeof(uint32_t)));
     hipLaunchKernelGGL(k_slot_ranges<DIM>, dim3((unsigned)((c->n_records + t - 1) / t)), dim3(t), 0, 0, c->records,
                        c->root, c->prims, c->n_records, c->ranges, c->range_info);
@@ -130,7 +132,12 @@ static int compute_ranges(fcpw_hip_ctx *c)
     c->n_top = info[2];
     c->n_frontier = (int)n_frontier;
     c->by_range = true;
-    return launch_disks(c, 0, c->range_info);
+    const int st_disks = launch_disks(c, 0, c->range_info);
+    if (st_disks) return st_disks;
+    float limit = 0.0f;
+    HIPCHECK(c, hipMemcpy(&limit, c->disk_limit, sizeof(float), hipMemcpyDeviceToHost));
+    c->disks_off = limit < 0.0f && !info[3]; // stale boxes: until a refit, which may be a graph's
+    return FCPW_HIP_OK;
 }
 
 static int compute_ranges(fcpw_hip_ctx *c) { return c->dim == 3 ? compute_ranges<3>(c) : compute_ranges<2>(c); }
@@ -154,7 +161,8 @@ static int upload_ranges(fcpw_hip_ctx *c)
     const size_t at_disks = take(n_slots * sizeof(float4)), at_top = take(cap_top * sizeof(int4)),
                  at_ranges = take(n_slots * sizeof(int2)), at_big = take(n_slots * sizeof(int)),
                  at_front = take(cap_front * sizeof(int)), at_mark = take((n_prims + 1) * sizeof(uint32_t)),
-                 at_sums = take(segs * sizeof(uint32_t)), at_info = take(4 * sizeof(int)), at_limit = take(sizeof(float));
+                 at_sums = take(segs * sizeof(uint32_t)), at_info = take(4 * sizeof(int)), at_limit = take(sizeof(float)),
+                 at_tally = take(sizeof(unsigned long long));
     HIPCHECK(c, hipMalloc((void **)&c->range_mem, bytes));
     char *m = (char *)c->range_mem;
     c->disks = (float4 *)(m + at_disks);
@@ -166,6 +174,7 @@ static int upload_ranges(fcpw_hip_ctx *c)
     c->range_sums = (uint32_t *)(m + at_sums);
     c->range_info = (int *)(m + at_info);
     c->disk_limit = (float *)(m + at_limit);
+    c->disk_tally = (unsigned long long *)(m + at_tally);
     const int st = compute_ranges(c);
     if (st) return st;
     HIPCHECK(c, hipDeviceSynchronize());
@@ -987,6 +996,7 @@ int fcpw_hip_refit(fcpw_hip_ctx *c, void *stream)
     }
     HIPCHECK(c, hipGetLastError());
     if ((st = launch_disks(c, s))) return st;
+    c->disks_off = !c->by_range; // where the new boxes' disks do not pay the kernels find them off
     if (c->has_silhouettes) {
         if ((st = launch_faces(c, s))) return st;
         if (c->dim == 3)
@@ -1174,16 +1184,25 @@ static int launch_closest_kernel(fcpw_hip_ctx *c, const CpIO &io, hipStream_t s,
     } else if (c->coop) {
         const int wq = wave_queries(c, n);
         dim3 g = grid_for(c, n, wq);
-#define FCPW_COOP(D, K)                                                                                       \
-    hipLaunchKernelGGL((k_closest_points_coop<D, K, OUT, false>), g, dim3(64), 0, s, S, io, xcd_arg(c), c->hold_min, \
-                       wq)
+#define FCPW_COOP_D(D, K, DISK)                                                                               \
+    hipLaunchKernelGGL((k_closest_points_coop<D, K, OUT, false, DISK>), g, dim3(64), 0, s, S, io, xcd_arg(c),  \
+                       c->hold_min, wq)
+#define FCPW_COOP(D, K) FCPW_COOP_D(D, K, true)
+        // A tree whose disks are known to be off walks without them, for the entries
+        // below (with the tests in the kernel, all failing, 8.4M queries on soups take
+        // 2 to 3% longer).
         // 0, 4, 6, 8, 12, 16 or 24 LDS entries (2D: 24 runs as 16).  Six keep eight
         // waves a SIMD, which a batch of at most 16 waves a CU does not make: unless
         // the caller chose another number it takes twelve and spills less (100,003 queries
         // 165 -> 160 us, 30,000 in 2D 317 -> 306, 12,000 on 300,000 triangles 851 -> 820).
         const int k = c->stack == STACK_DEFAULT && (int64_t)g.x <= (int64_t)16 * c->n_cus ? 12 : c->stack;
         c->launch = {k, c->hold_min, wq, 0};
-        if (c->dim == 3) {
+        if (c->disks_off && (k == 6 || k == 12)) {
+            if (c->dim == 3 && k == 6) FCPW_COOP_D(3, 6, false);
+            else if (c->dim == 3) FCPW_COOP_D(3, 12, false);
+            else if (k == 6) FCPW_COOP_D(2, 6, false);
+            else FCPW_COOP_D(2, 12, false);
+        } else if (c->dim == 3) {
             if (k == 0) FCPW_COOP(3, 0);
             else if (k == 4) FCPW_COOP(3, 4);
             else if (k == 6) FCPW_COOP(3, 6);

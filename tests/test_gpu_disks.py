@@ -171,3 +171,26 @@ def test_stale_boxes_stay_without_disks(gpu, mesh):
         g._refit_device(st)
         b.refit()
         check(g, V2, F, q, bvh=b)
+
+
+def test_disks_off_where_few_slots_keep_one(gpu):
+    """a soup's patches are no plates: the walk goes without disks, after a refit
+    that makes a smooth surface of it with them, and back; the records stay"""
+    import torch
+    V, F = meshes.small_torus(64, 32)
+    V = V[F].reshape(-1, 3).copy()  # triangles of their own
+    F = np.arange(len(V), dtype=np.int32).reshape(-1, 3)
+    soup = synth.f32(synth.Rng(71).uniform(V.size, -1.0, 1.0).reshape(V.shape))
+    _, g = make_scene(soup, F)
+    b = oracle.Bvh(soup, F)
+    q = queries(V, 6000, 72)
+    check(g, soup, F, q, bvh=b)
+    st = torch.cuda.current_stream().cuda_stream
+    for W in (V, soup, V):
+        dv = torch.from_numpy(W).cuda()
+        g._update_positions_device(dv.data_ptr(), len(W), st)
+        g._refit_device(st)
+        torch.cuda.synchronize()
+        b.update_vertices(W)
+        b.refit()
+        check(g, W, F, q, bvh=b)
