@@ -28,6 +28,9 @@ struct fcpw_hip_ctx {
     int32_t *rec_parent = nullptr, *leaf_refs = nullptr;
     uint32_t *leaf_links = nullptr;
     unsigned int *counters = nullptr;
+    // an upload's two allocations, of the tree and of the geometry (null after a
+    // device build, whose buffers are their own)
+    void *tree_mem = nullptr, *geom_mem = nullptr;
     // the leaf-slot range below every child slot, the slots sorted by its size,
     // and the disks with the distance they hold up to: parts of range_mem, which
     // is null for a tree over instances.  by_range: the leaves lie in order, so
@@ -37,13 +40,13 @@ struct fcpw_hip_ctx {
     float4 *disks = nullptr;
     int4 *top = nullptr;
     int2 *ranges = nullptr;
-    int *big = nullptr, *frontier = nullptr, *range_info = nullptr;
+    int *big = nullptr, *frontier = nullptr;
+    SlotInfo *slot_info = nullptr;
     uint32_t *range_mark = nullptr, *range_sums = nullptr;
-    float *disk_limit = nullptr;
-    unsigned long long *disk_tally = nullptr;
     bool disks_off = true; // known on the host: they are off until the next refit or upload
     bool by_range = false, one_tree = false;
     int n_big = 0, n_top = 0, n_frontier = 0;
+    int2 root_range = {0, 0}; // first primitive and the one past the last
     int *flags = nullptr;
     unsigned long long *stats = nullptr; // internal nodes, primitive tests, queries (option "stats")
     // silhouettes (fcpw_hip_upload_silhouettes): cones per child slot and root, leaf ranges, records
@@ -152,19 +155,24 @@ static void free_silhouettes(fcpw_hip_ctx *c)
 
 static void free_scene(fcpw_hip_ctx *c)
 {
-    void *bufs[] = {c->records, c->root, c->prims, c->prim_index, c->prim_vids, c->V,
-                    c->rec_parent, c->leaf_refs, c->leaf_links, c->counters, c->inst, c->obj_table, c->range_mem};
+    // an upload's buffers are parts of tree_mem and geom_mem, a device build's are their own
+    void *own[] = {c->records, c->root, c->prims, c->prim_index, c->prim_vids, c->V,
+                   c->rec_parent, c->leaf_refs, c->leaf_links, c->counters};
+    if (!c->tree_mem)
+        for (void *b : own)
+            if (b) (void)hipFree(b);
+    void *bufs[] = {c->tree_mem, c->geom_mem, c->inst, c->obj_table, c->range_mem};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
+    c->tree_mem = c->geom_mem = nullptr;
     free_silhouettes(c);
     c->range_mem = nullptr;
     c->disks = nullptr;
     c->top = nullptr;
     c->ranges = nullptr;
-    c->big = c->frontier = c->range_info = nullptr;
+    c->big = c->frontier = nullptr;
+    c->slot_info = nullptr;
     c->range_mark = c->range_sums = nullptr;
-    c->disk_limit = nullptr;
-    c->disk_tally = nullptr;
     c->disks_off = true;
     c->by_range = false;
     c->inst = nullptr;
@@ -188,7 +196,8 @@ static inline int sil_xcd_arg(const fcpw_hip_ctx *c) { return c->sil_xcds | (c->
 
 static DevScene dev_scene(fcpw_hip_ctx *c)
 {
-    return DevScene{c->records, c->root, c->prims, c->prim_index, c->disks, c->disk_limit, c->flags, c->stats};
+    return DevScene{c->records, c->root, c->prims, c->prim_index, c->disks,
+                    c->slot_info ? &c->slot_info->disk_limit : nullptr, c->flags, c->stats};
 }
 
 static int grow(fcpw_hip_ctx *c, void **buf, size_t *cap, size_t bytes)

@@ -1647,9 +1647,9 @@ __global__ void k_refit(float4 *records, float4 *root, const float4 *prims, cons
 // lie together, from its leftmost leaf to its rightmost: one thread a record
 // walks down the inner and outer edges of its two subtrees (a climb from the
 // leaves with a counter per record, as k_refit's, took 1.6 ms for a million
-// triangles; its fences reach all L2s).  info[0] is set where the two ranges of
-// a record do not join up -- a caller's tree may place its leaves in any
-// order -- and the tree then goes without ranges and disks.
+// triangles; its fences reach all L2s).  Where the two ranges of a record do not
+// join up -- a caller's tree may place its leaves in any order -- the tree goes
+// without ranges and disks.
 template <int DIM>
 __device__ __forceinline__ uint32_t slot_link(const float4 *records, uint32_t rec, int side)
 {
@@ -1732,63 +1732,95 @@ __device__ __forceinline__ bool box_holds(const float4 *records, const float4 *p
     return in;
 }
 
-// info[3] is set where a box does not hold what lies below it: a caller's boxes,
-// or boxes from before a vertex update.  The reference shrinks r^2 by such boxes
-// too, so dropping a subtree could change a record, and the disks stay off until
-// a refit (k_build_disks).
-template <int DIM>
-__global__ void k_slot_ranges(const float4 *records, const float4 *root, const float4 *prims, int n_records,
-                              int2 *ranges, int *info)
-{
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= n_records) return;
-    for (int side = 0; side < 2; side++) {
-        v3 lo, hi;
-        load_slot_box<DIM>(records, 2 * r + side, lo, hi);
-        if (!box_holds<DIM>(records, prims, slot_link<DIM>(records, (uint32_t)r, side), lo, hi)) info[3] = 1;
-    }
-    if (r == 0) {
-        v3 lo, hi;
-        load_root_box<DIM>(root, lo, hi);
-        if (!box_holds<DIM>(records, prims, link_of(DIM == 3 ? root[0].w : root[1].x), lo, hi)) info[3] = 1;
-    }
-    const uint32_t a = slot_link<DIM>(records, (uint32_t)r, 0), b = slot_link<DIM>(records, (uint32_t)r, 1);
-    const int a0 = subtree_edge<DIM>(records, a, 0), a1 = subtree_edge<DIM>(records, a, 1);
-    const int b0 = subtree_edge<DIM>(records, b, 0), b1 = subtree_edge<DIM>(records, b, 1);
-    if (a1 != b0 || a1 <= a0 || b1 <= b0) info[0] = 1;
-    ranges[2 * r] = make_int2(a0, a1 - a0);
-    ranges[2 * r + 1] = make_int2(b0, b1 - b0);
-}
-
 // Sorts the child slots by the size of their range: up to DISK_OWN primitives
 // one lane handles the slot, up to DISK_MAX_PRIMS one wave (list `big`), above
 // that (list `top`) its box is put together from the boxes of the largest
 // slots of at most DISK_MAX_PRIMS below it.  Those, the children of records
 // that hold more (and of the root record), are marked at their first primitive;
 // after a scan of the marks a subtree's share of them is a range of their list.
-// info: [1] big slots, [2] top slots
 constexpr int DISK_OWN = 16;
+
+// What the passes over a tree's slots leave for the host and for each other.
+struct SlotInfo {
+    int out_of_order;         // the leaves do not lie in order: no ranges
+    int n_big, n_top, n_frontier;
+    int stale;                // a box does not hold what lies below it (slot_range)
+    int faces;                // slots that have a facing entry, of at most DISK_OWN primitives
+    float disk_limit;         // DevScene::disk_limit
+    int root_first, root_end; // the root's range
+    int unused;
+    unsigned long long tally; // k_build_disks
+};
+
+// The ranges of record r's two slots; flags bit 0 where they do not join up, bit 1
+// where a box does not hold what lies below it: a caller's boxes, or boxes from
+// before a vertex update.  The reference shrinks r^2 by such boxes too, so
+// dropping a subtree could change a record, and the disks stay off until a refit.
+template <int DIM>
+__device__ __forceinline__ int slot_range(const float4 *records, const float4 *root, const float4 *prims, int r,
+                                          int2 &ra, int2 &rb)
+{
+    int flags = 0;
+    for (int side = 0; side < 2; side++) {
+        v3 lo, hi;
+        load_slot_box<DIM>(records, 2 * r + side, lo, hi);
+        if (!box_holds<DIM>(records, prims, slot_link<DIM>(records, (uint32_t)r, side), lo, hi)) flags |= 2;
+    }
+    if (r == 0) {
+        v3 lo, hi;
+        load_root_box<DIM>(root, lo, hi);
+        if (!box_holds<DIM>(records, prims, link_of(DIM == 3 ? root[0].w : root[1].x), lo, hi)) flags |= 2;
+    }
+    const uint32_t a = slot_link<DIM>(records, (uint32_t)r, 0), b = slot_link<DIM>(records, (uint32_t)r, 1);
+    const int a0 = subtree_edge<DIM>(records, a, 0), a1 = subtree_edge<DIM>(records, a, 1);
+    const int b0 = subtree_edge<DIM>(records, b, 0), b1 = subtree_edge<DIM>(records, b, 1);
+    if (a1 != b0 || a1 <= a0 || b1 <= b0) flags |= 1;
+    ra = make_int2(a0, a1 - a0);
+    rb = make_int2(b0, b1 - b0);
+    return flags;
+}
+
+template <int DIM>
+__global__ void k_slot_ranges(const float4 *records, const float4 *root, const float4 *prims, int n_records,
+                              int2 *ranges, SlotInfo *info)
+{
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r == 0) info->disk_limit = -1.0f;
+    if (r >= n_records) return;
+    int2 ra, rb;
+    const int flags = slot_range<DIM>(records, root, prims, r, ra, rb);
+    if (flags & 1) info->out_of_order = 1;
+    if (flags & 2) info->stale = 1;
+    if ((uint32_t)r == link_of(DIM == 3 ? root[0].w : root[1].x)) {
+        info->root_first = ra.x;
+        info->root_end = rb.x + rb.y;
+    }
+    ranges[2 * r] = ra;
+    ranges[2 * r + 1] = rb;
+}
 
 template <int DIM>
 __global__ void k_slot_lists(const int2 *ranges, const float4 *root, int n_slots, int *big, int4 *top, uint32_t *mark,
-                             int *info)
+                             SlotInfo *info)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n_slots) return;
+    if (s >= n_slots || info->out_of_order) return;
     const uint32_t root_rec = link_of(DIM == 3 ? root[0].w : root[1].x);
     const int2 rg = ranges[s];
-    if (rg.y > DISK_OWN && rg.y <= DISK_MAX_PRIMS) big[atomicAdd(&info[1], 1)] = s;
-    if (rg.y > DISK_MAX_PRIMS) top[atomicAdd(&info[2], 1)] = make_int4(s, rg.x, rg.x + rg.y, 0);
+    if (rg.y > DISK_OWN && rg.y <= DISK_MAX_PRIMS) big[atomicAdd(&info->n_big, 1)] = s;
+    if (rg.y > DISK_MAX_PRIMS) top[atomicAdd(&info->n_top, 1)] = make_int4(s, rg.x, rg.x + rg.y, 0);
     else if (rg.y + ranges[s ^ 1].y > DISK_MAX_PRIMS || (uint32_t)(s >> 1) == root_rec) mark[rg.x] = 1u;
 }
 
 // pos = exclusive scan of the marks (n_prims + 1 entries)
 template <int DIM>
 __global__ void k_slot_frontier(const int2 *ranges, const float4 *root, int n_slots, const uint32_t *pos, int4 *top,
-                                int *frontier, const int *info)
+                                int *frontier, int n_prims, SlotInfo *info)
 {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < info[2]) {
+    if (info->out_of_order) return;
+    if (s == 0) info->n_frontier = (int)pos[n_prims];
+    if (s < info->n_top) {
         const int4 t = top[s];
         top[s] = make_int4(t.x, (int)pos[t.y], (int)pos[t.z], 0);
     }
@@ -1811,14 +1843,26 @@ __device__ __forceinline__ void store_slot_box(float4 *records, int slot, v3 lo,
     }
 }
 
+template <int DIM>
+__device__ __forceinline__ void store_root_box(float4 *root, v3 lo, v3 hi)
+{
+    if (DIM == 3) {
+        root[0] = make_float4(lo.x, lo.y, lo.z, root[0].w); // the link stays
+        root[1] = make_float4(hi.x, hi.y, hi.z, 0.0f);
+    } else {
+        root[0] = make_float4(lo.x, lo.y, hi.x, hi.y);
+    }
+}
+
 __device__ __forceinline__ void box_merge(v3 &lo, v3 &hi, v3 l, v3 h)
 {
     lo = {fminf(lo.x, l.x), fminf(lo.y, l.y), fminf(lo.z, l.z)};
     hi = {fmaxf(hi.x, h.x), fmaxf(hi.y, h.y), fmaxf(hi.z, h.z)};
 }
-__device__ __forceinline__ void box_wave_merge(v3 &lo, v3 &hi)
+// over groups of `lanes` neighbouring lanes
+__device__ __forceinline__ void box_wave_merge(v3 &lo, v3 &hi, int lanes = 64)
 {
-    for (int off = 32; off > 0; off >>= 1) {
+    for (int off = lanes / 2; off > 0; off >>= 1) {
         const v3 l = {__shfl_xor(lo.x, off, 64), __shfl_xor(lo.y, off, 64), __shfl_xor(lo.z, off, 64)};
         const v3 h = {__shfl_xor(hi.x, off, 64), __shfl_xor(hi.y, off, 64), __shfl_xor(hi.z, off, 64)};
         box_merge(lo, hi, l, h);
@@ -1827,22 +1871,33 @@ __device__ __forceinline__ void box_wave_merge(v3 &lo, v3 &hi)
 
 // the inflated box of one primitive (Triangle / LineSegment.getBoundingBox)
 template <int DIM>
-__device__ __forceinline__ void prim_box_merge(const float4 *prims, int slot, v3 &lo, v3 &hi)
+__device__ __forceinline__ void prim_box_merge(const v3 p[3], v3 &lo, v3 &hi)
 {
-    v3 l, h;
+    // in 2D p[2] is p[0]
+    v3 l = {fminf(fminf(p[0].x, p[1].x), p[2].x) - FLT_EPSILON, fminf(fminf(p[0].y, p[1].y), p[2].y) - FLT_EPSILON,
+            0.0f};
+    v3 h = {fmaxf(fmaxf(p[0].x, p[1].x), p[2].x) + FLT_EPSILON, fmaxf(fmaxf(p[0].y, p[1].y), p[2].y) + FLT_EPSILON,
+            0.0f};
     if (DIM == 3) {
-        const float4 *t = prims + (size_t)slot * 3;
-        const float4 a = t[0], b = t[1], c = t[2];
-        l = {fminf(fminf(a.x, b.x), c.x) - FLT_EPSILON, fminf(fminf(a.y, b.y), c.y) - FLT_EPSILON,
-             fminf(fminf(a.z, b.z), c.z) - FLT_EPSILON};
-        h = {fmaxf(fmaxf(a.x, b.x), c.x) + FLT_EPSILON, fmaxf(fmaxf(a.y, b.y), c.y) + FLT_EPSILON,
-             fmaxf(fmaxf(a.z, b.z), c.z) + FLT_EPSILON};
-    } else {
-        const float4 s = prims[slot];
-        l = {fminf(s.x, s.z) - FLT_EPSILON, fminf(s.y, s.w) - FLT_EPSILON, 0.0f};
-        h = {fmaxf(s.x, s.z) + FLT_EPSILON, fmaxf(s.y, s.w) + FLT_EPSILON, 0.0f};
+        l.z = fminf(fminf(p[0].z, p[1].z), p[2].z) - FLT_EPSILON;
+        h.z = fmaxf(fmaxf(p[0].z, p[1].z), p[2].z) + FLT_EPSILON;
     }
     box_merge(lo, hi, l, h);
+}
+
+// the box of a slot from its primitives: of one lane (step 1), or of a group of
+// `step` neighbouring lanes (first = the lane's place in it; all return it)
+template <int DIM>
+__device__ __forceinline__ void slot_box(const float4 *prims, int2 rg, int first, int step, v3 &lo, v3 &hi)
+{
+    lo = {FLT_MAX, FLT_MAX, FLT_MAX};
+    hi = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+    for (int k = first; k < rg.y; k += step) {
+        v3 p[3];
+        disk_verts<DIM>(prims, rg.x + k, p);
+        prim_box_merge<DIM>(p, lo, hi);
+    }
+    box_wave_merge(lo, hi, step);
 }
 
 // Refit of the boxes by range, first part: the box of every slot of at most
@@ -1859,22 +1914,20 @@ template <int DIM>
 __global__ __launch_bounds__(DISK_BLOCK) void k_refit_ranges(float4 *records, const float4 *prims, const int2 *ranges,
                                                              int n_slots, const int *big, int n_big, int own_blocks)
 {
-    v3 lo = {FLT_MAX, FLT_MAX, FLT_MAX}, hi = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+    v3 lo, hi;
     if ((int)blockIdx.x < own_blocks) {
         const int slot = (int)blockIdx.x * DISK_BLOCK + (int)threadIdx.x;
         if (slot >= n_slots) return;
         const int2 rg = ranges[slot];
         if (rg.y > DISK_OWN) return;
-        for (int k = 0; k < rg.y; k++) prim_box_merge<DIM>(prims, rg.x + k, lo, hi);
+        slot_box<DIM>(prims, rg, 0, 1, lo, hi);
         store_slot_box<DIM>(records, slot, lo, hi);
         return;
     }
     const int w = ((int)blockIdx.x - own_blocks) * (DISK_BLOCK / 64) + (int)(threadIdx.x >> 6);
     if (w >= n_big) return;
     const int slot = big[w], lane = (int)(threadIdx.x & 63u);
-    const int2 rg = ranges[slot];
-    for (int k = lane; k < rg.y; k += 64) prim_box_merge<DIM>(prims, rg.x + k, lo, hi);
-    box_wave_merge(lo, hi);
+    slot_box<DIM>(prims, ranges[slot], lane, 64, lo, hi);
     if (lane == 0) store_slot_box<DIM>(records, slot, lo, hi);
 }
 
@@ -1896,14 +1949,8 @@ __global__ __launch_bounds__(DISK_BLOCK) void k_refit_top(float4 *records, float
     }
     box_wave_merge(lo, hi);
     if (lane != 0) return;
-    if (t.x >= 0) {
-        store_slot_box<DIM>(records, t.x, lo, hi);
-    } else if (DIM == 3) {
-        root[0] = make_float4(lo.x, lo.y, lo.z, root[0].w);
-        root[1] = make_float4(hi.x, hi.y, hi.z, 0.0f);
-    } else {
-        root[0] = make_float4(lo.x, lo.y, hi.x, hi.y);
-    }
+    if (t.x >= 0) store_slot_box<DIM>(records, t.x, lo, hi);
+    else store_root_box<DIM>(root, lo, hi);
 }
 
 // What k_build_disks gathers of a slot's primitives: first the sum of their
@@ -1915,10 +1962,8 @@ struct DiskSums {
 };
 
 template <int DIM>
-__device__ __forceinline__ void disk_normal_add(const float4 *prims, int slot, DiskSums &D)
+__device__ __forceinline__ void disk_normal_add(const v3 p[3], DiskSums &D)
 {
-    v3 p[3];
-    disk_verts<DIM>(prims, slot, p);
     const v3 e = sub(p[1], p[0]);
     const v3 m = DIM == 3 ? cross(e, sub(p[2], p[0])) : v3{e.y, -e.x, 0.0f};
     D.n = {D.n.x + m.x, D.n.y + m.y, D.n.z + m.z};
@@ -1927,10 +1972,8 @@ __device__ __forceinline__ void disk_normal_add(const float4 *prims, int slot, D
 // c2 = lo + hi of the box (twice its centre), n the unit normal as rounded;
 // reach = the largest distance of a query the disks serve
 template <int DIM>
-__device__ __forceinline__ void disk_extent_add(const float4 *prims, int slot, v3 c2, v3 n, float reach, DiskSums &D)
+__device__ __forceinline__ void disk_extent_add(const v3 p[3], v3 c2, v3 n, float reach, DiskSums &D)
 {
-    v3 p[3];
-    disk_verts<DIM>(prims, slot, p);
     for (int k = 0; k < DIM; k++) {
         const v3 w = {p[k].x - 0.5f * c2.x, p[k].y - 0.5f * c2.y, p[k].z - 0.5f * c2.z};
         const float h = dot(w, n);
@@ -2008,95 +2051,240 @@ __device__ __forceinline__ float4 disk_pack(const DiskSums &D, v3 half, v3 n, ui
                        __uint_as_float(bf16_up(t) | (bf16_up(r) << 16)), (float)(0.5 * DISK_SHRINK) * inv);
 }
 
-// The disks of all slots, shared out as in k_refit_ranges: two passes over a
-// slot's primitives (normal, extents), which lie together in leaf order.
-// Slots above DISK_MAX_PRIMS have none.  Queries whose root box's farthest
-// corner lies beyond disk_limit go without, and all queries where the boxes do
-// not hold their primitives (info[3], k_slot_ranges; null after a refit).
+// The queries a tree's disks serve, from its root box: in 1.5 times the box and
+// somewhat beyond, those whose farthest corner of it is within `reach`.  The others
+// go without: 1M queries on 131,072 triangles in 2 times the box 8.8 -> 2.0 ms, in 3
+// times 9.8 -> 2.9, in 6 times 9.5 -> 4.1.
+struct DiskScope {
+    float reach, scale; // scale: the largest coordinate magnitude
+};
+__device__ __forceinline__ DiskScope disk_scope(v3 rlo, v3 rhi)
+{
+    const v3 ext = sub(rhi, rlo);
+    return {1.5f * sqrtf(dot(ext, ext)),
+            fmaxf(fmaxf(fmaxf(fabsf(rlo.x), fabsf(rhi.x)), fmaxf(fabsf(rlo.y), fabsf(rhi.y))),
+                  fmaxf(fabsf(rlo.z), fabsf(rhi.z)))};
+}
+
+// The disk of a slot with box (lo, hi), in two passes over its primitives (normal,
+// extents), which lie together in leaf order; lanes as in slot_box
+template <int DIM>
+__device__ __forceinline__ float4 slot_disk(const float4 *prims, int2 rg, int first, int step, v3 lo, v3 hi, DiskScope q)
+{
+    const v3 c2 = {lo.x + hi.x, lo.y + hi.y, lo.z + hi.z};
+    const v3 half = {0.5f * (hi.x - lo.x), 0.5f * (hi.y - lo.y), 0.5f * (hi.z - lo.z)};
+    DiskSums D = {{0, 0, 0}, INFINITY, -INFINITY, 0.0f, 0.0f, 0.0f};
+    v3 p[3];
+    for (int k = first; k < rg.y; k += step) {
+        disk_verts<DIM>(prims, rg.x + k, p);
+        disk_normal_add<DIM>(p, D);
+    }
+    for (int off = step / 2; off > 0; off >>= 1) {
+        D.n.x += __shfl_xor(D.n.x, off, 64);
+        D.n.y += __shfl_xor(D.n.y, off, 64);
+        D.n.z += __shfl_xor(D.n.z, off, 64);
+    }
+    v3 n;
+    uint32_t nxy, nz;
+    float inv;
+    disk_round_normal(D.n, n, nxy, nz, inv);
+    for (int k = first; k < rg.y; k += step) {
+        disk_verts<DIM>(prims, rg.x + k, p);
+        disk_extent_add<DIM>(p, c2, n, q.reach, D);
+    }
+    for (int off = step / 2; off > 0; off >>= 1) {
+        D.lo = fminf(D.lo, __shfl_xor(D.lo, off, 64));
+        D.hi = fmaxf(D.hi, __shfl_xor(D.hi, off, 64));
+        D.l2 = fmaxf(D.l2, __shfl_xor(D.l2, off, 64));
+        D.mt = fmaxf(D.mt, __shfl_xor(D.mt, off, 64));
+        D.mr = fmaxf(D.mr, __shfl_xor(D.mr, off, 64));
+    }
+    return disk_pack(D, half, n, nxy, nz, inv, q.scale);
+}
+
 // Where fewer than DISK_KEPT_MIN of the slots of at most DISK_OWN primitives keep
 // a disk, the walk drops next to nothing by them and pays their loads: they then
 // stay off as a whole.  8.4M queries, half of them near, with disks and without:
 // triangle soups that keep 0.24 of them 4.19 ms and 3.95, 0.35 3.72 and 3.48, 0.39
 // 2.15 and 2.04, 0.46 4.45 and 4.34, 0.47 11.6 and 11.2; noisy spheres that keep 0.59
 // 5.71 and 6.04 (200,000 triangles) and 3.60 and 3.39 (20,000), 0.66 3.55 and 3.54, 0.75
-// 10.1 and 11.1.  tally counts the kept slots (upper half) and the blocks that have
-// added theirs; the last one decides.
+// 10.1 and 11.1.
 constexpr float DISK_KEPT_MIN = 0.5f;
+__device__ __forceinline__ float disk_limit_of(int n_kept, int n_own, bool stale, DiskScope q)
+{
+    // the bound's squares neither overflow (1e37) nor leave the normal range
+    // (1e-6: a disk excludes no distance below 1e-6 of the coordinates)
+    const bool on = (float)n_kept >= DISK_KEPT_MIN * (float)n_own && q.reach >= 1e-6f && !stale;
+    return on ? fminf(q.reach * q.reach, 1e37f) : -1.0f;
+}
 
+// The kept slots of one block (upper half of the tally) and the block itself
+// counted; the last one sets the limit.
+__device__ __forceinline__ void disk_tally(SlotInfo *info, int kept, int blocks, int n_own, bool stale, DiskScope q)
+{
+    const unsigned long long before = atomicAdd(&info->tally, ((unsigned long long)kept << 32) | 1ull);
+    if ((int)(before & 0xFFFFFFFFull) != blocks - 1) return;
+    info->tally = 0;
+    info->disk_limit = disk_limit_of((int)(before >> 32) + kept, n_own, stale, q);
+}
+
+// The disks of all slots, shared out as in k_refit_ranges.  Slots above
+// DISK_MAX_PRIMS have none.  refitted: the boxes have just been rebuilt, whatever
+// info->stale says.
 template <int DIM>
 __global__ __launch_bounds__(DISK_BLOCK) void k_build_disks(const float4 *records, const float4 *root,
                                                             const float4 *prims, const int2 *ranges, int n_slots,
                                                             const int *big, int n_big, int n_own, int own_blocks,
-                                                            float4 *disks, float *disk_limit, const int *info,
-                                                            unsigned long long *tally)
+                                                            float4 *disks, SlotInfo *info, int refitted)
 {
-    v3 rlo, rhi;
-    load_root_box<DIM>(root, rlo, rhi);
-    const v3 ext = sub(rhi, rlo);
-    const float reach = 1.5f * sqrtf(dot(ext, ext)); // queries in 1.5 times the box and beyond
-    const float scale = fmaxf(fmaxf(fmaxf(fabsf(rlo.x), fabsf(rhi.x)), fmaxf(fabsf(rlo.y), fabsf(rhi.y))),
-                              fmaxf(fabsf(rlo.z), fabsf(rhi.z)));
-    const bool own = (int)blockIdx.x < own_blocks;
-    int slot, step, first;
-    bool on = true;
-    if (own) {
-        slot = (int)blockIdx.x * DISK_BLOCK + (int)threadIdx.x;
-        first = 0;
-        step = 1;
-        on = slot < n_slots;
-    } else {
+    v3 lo, hi;
+    load_root_box<DIM>(root, lo, hi);
+    const DiskScope q = disk_scope(lo, hi);
+    if ((int)blockIdx.x >= own_blocks) {
         const int w = ((int)blockIdx.x - own_blocks) * (DISK_BLOCK / 64) + (int)(threadIdx.x >> 6);
         if (w >= n_big) return;
-        slot = big[w];
-        first = (int)(threadIdx.x & 63u);
-        step = 64;
-    }
-    int2 rg = make_int2(0, 0);
-    if (on) rg = ranges[slot];
-    if (own && rg.y > DISK_OWN) {
-        if (rg.y > DISK_MAX_PRIMS) disks[slot] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        on = false;
-    }
-    float4 packed = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (on) {
-        v3 lo, hi;
+        const int slot = big[w], lane = (int)(threadIdx.x & 63u);
         load_slot_box<DIM>(records, slot, lo, hi);
-        const v3 c2 = {lo.x + hi.x, lo.y + hi.y, lo.z + hi.z};
-        const v3 half = {0.5f * (hi.x - lo.x), 0.5f * (hi.y - lo.y), 0.5f * (hi.z - lo.z)};
-        DiskSums D = {{0, 0, 0}, INFINITY, -INFINITY, 0.0f, 0.0f, 0.0f};
-        for (int k = first; k < rg.y; k += step) disk_normal_add<DIM>(prims, rg.x + k, D);
-        if (!own)
-            for (int off = 32; off > 0; off >>= 1) {
-                D.n.x += __shfl_xor(D.n.x, off, 64);
-                D.n.y += __shfl_xor(D.n.y, off, 64);
-                D.n.z += __shfl_xor(D.n.z, off, 64);
-            }
-        v3 n;
-        uint32_t nxy, nz;
-        float inv;
-        disk_round_normal(D.n, n, nxy, nz, inv);
-        for (int k = first; k < rg.y; k += step) disk_extent_add<DIM>(prims, rg.x + k, c2, n, reach, D);
-        if (!own)
-            for (int off = 32; off > 0; off >>= 1) {
-                D.lo = fminf(D.lo, __shfl_xor(D.lo, off, 64));
-                D.hi = fmaxf(D.hi, __shfl_xor(D.hi, off, 64));
-                D.l2 = fmaxf(D.l2, __shfl_xor(D.l2, off, 64));
-                D.mt = fmaxf(D.mt, __shfl_xor(D.mt, off, 64));
-                D.mr = fmaxf(D.mr, __shfl_xor(D.mr, off, 64));
-            }
-        packed = disk_pack(D, half, n, nxy, nz, inv, scale);
-        if (first == 0) disks[slot] = packed;
+        const float4 d = slot_disk<DIM>(prims, ranges[slot], lane, 64, lo, hi, q);
+        if (lane == 0) disks[slot] = d;
+        return;
     }
-    if (!own) return;
-    const int kept = __syncthreads_count(packed.w != 0.0f);
-    if (threadIdx.x != 0) return;
-    const unsigned long long before = atomicAdd(tally, ((unsigned long long)kept << 32) | 1ull);
-    if ((int)(before & 0xFFFFFFFFull) != own_blocks - 1) return;
-    *tally = 0;
-    // the bound's squares neither overflow (1e37) nor leave the normal range
-    // (1e-6: a disk excludes no distance below 1e-6 of the coordinates)
-    const bool pay = (float)((int)(before >> 32) + kept) >= DISK_KEPT_MIN * (float)n_own;
-    *disk_limit = pay && reach >= 1e-6f && !(info && info[3]) ? fminf(reach * reach, 1e37f) : -1.0f;
+    const int slot = (int)blockIdx.x * DISK_BLOCK + (int)threadIdx.x;
+    float4 d = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (slot < n_slots) {
+        const int2 rg = ranges[slot];
+        if (rg.y <= DISK_OWN) {
+            load_slot_box<DIM>(records, slot, lo, hi);
+            d = slot_disk<DIM>(prims, rg, 0, 1, lo, hi, q);
+        }
+        if (rg.y <= DISK_OWN || rg.y > DISK_MAX_PRIMS) disks[slot] = d;
+    }
+    const int kept = __syncthreads_count(d.w != 0.0f);
+    if (threadIdx.x == 0) disk_tally(info, kept, own_blocks, n_own, !refitted && info->stale, q);
+}
+
+// Box and disk of a slot in one go, by a group of `step` lanes.
+template <int DIM>
+__device__ __forceinline__ bool refit_slot(float4 *records, const float4 *prims, int slot, int2 rg, int first,
+                                           int step, DiskScope q, float4 *disks)
+{
+    v3 lo, hi;
+    slot_box<DIM>(prims, rg, first, step, lo, hi);
+    const float4 d = slot_disk<DIM>(prims, rg, first, step, lo, hi, q);
+    if (first == 0) {
+        store_slot_box<DIM>(records, slot, lo, hi);
+        disks[slot] = d;
+    }
+    return d.w != 0.0f;
+}
+
+// The refit of a tree of at most DISK_MAX_PRIMS primitives in one launch, where the
+// three of larger trees (5 us each, one after another) are what it takes: every
+// block finds the root's box from all primitives by itself, so none waits for
+// another.  A slot of at most DISK_OWN primitives has as many lanes: the passes over
+// a slot are bound by their latency, some 200 instructions a primitive.  Twenty
+// refits one after another, in three launches, in this one with 4 lanes a slot, and
+// with 16: 20 triangles 307, 139 and 125 us, 320 393, 156 and 138, 980 497, 235
+// and 235.
+template <int DIM>
+__global__ __launch_bounds__(DISK_BLOCK) void k_refit_small(float4 *records, float4 *root, const float4 *prims,
+                                                            const int2 *ranges, int n_slots, const int *big, int n_big,
+                                                            int own_blocks, float4 *disks, SlotInfo *info,
+                                                            int2 root_range)
+{
+    __shared__ float part[6][DISK_BLOCK / 64];
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    v3 lo, hi;
+    lo = {FLT_MAX, FLT_MAX, FLT_MAX};
+    hi = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+    for (int k = root_range.x + tid; k < root_range.y; k += DISK_BLOCK) {
+        v3 p[3];
+        disk_verts<DIM>(prims, k, p);
+        prim_box_merge<DIM>(p, lo, hi);
+    }
+    box_wave_merge(lo, hi);
+    if (lane == 0) {
+        part[0][wave] = lo.x; part[1][wave] = lo.y; part[2][wave] = lo.z;
+        part[3][wave] = hi.x; part[4][wave] = hi.y; part[5][wave] = hi.z;
+    }
+    __syncthreads();
+    for (int w = 0; w < DISK_BLOCK / 64; w++)
+        box_merge(lo, hi, v3{part[0][w], part[1][w], part[2][w]}, v3{part[3][w], part[4][w], part[5][w]});
+    const DiskScope q = disk_scope(lo, hi);
+    if (blockIdx.x == 0 && tid == 0) store_root_box<DIM>(root, lo, hi);
+    if ((int)blockIdx.x >= own_blocks) {
+        const int w = ((int)blockIdx.x - own_blocks) * (DISK_BLOCK / 64) + wave;
+        if (w < n_big) refit_slot<DIM>(records, prims, big[w], ranges[big[w]], lane, 64, q, disks);
+        return;
+    }
+    const int slot = (int)blockIdx.x * (DISK_BLOCK / DISK_OWN) + tid / DISK_OWN;
+    bool kept = false;
+    if (slot < n_slots) {
+        const int2 rg = ranges[slot];
+        if (rg.y <= DISK_OWN) kept = refit_slot<DIM>(records, prims, slot, rg, tid % DISK_OWN, DISK_OWN, q, disks);
+    }
+    const int n = __syncthreads_count(kept && tid % DISK_OWN == 0);
+    if (tid == 0) disk_tally(info, n, own_blocks, n_slots - n_big, false, q);
+}
+
+// Ranges, lists and disks of a tree of at most SMALL_PRIMS primitives that was just
+// uploaded, by one block, DISK_OWN lanes a slot (info need not be cleared).
+constexpr int SMALL_PRIMS = 64, SMALL_BLOCK = 1024;
+
+template <int DIM>
+__global__ __launch_bounds__(SMALL_BLOCK) void k_small_tree(const float4 *records, const float4 *root,
+                                                            const float4 *prims, int n_records, int2 *ranges, int *big,
+                                                            float4 *disks, SlotInfo *info)
+{
+    __shared__ int flags, n_big, n_kept;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int n_slots = 2 * n_records;
+    if (tid == 0) flags = n_big = n_kept = 0;
+    __syncthreads();
+    for (int r = tid; r < n_records; r += SMALL_BLOCK) {
+        int2 rg[2];
+        const int f = slot_range<DIM>(records, root, prims, r, rg[0], rg[1]);
+        if (f) atomicOr(&flags, f);
+        for (int side = 0; side < 2; side++) {
+            ranges[2 * r + side] = rg[side];
+            if (rg[side].y > DISK_OWN) big[atomicAdd(&n_big, 1)] = 2 * r + side;
+        }
+    }
+    __syncthreads();
+    const uint32_t link = link_of(DIM == 3 ? root[0].w : root[1].x);
+    if (tid == 0) {
+        info->out_of_order = flags & 1;
+        info->stale = flags >> 1;
+        info->n_big = n_big;
+        info->n_top = info->n_frontier = info->faces = 0;
+        info->root_first = ranges[2 * link].x;
+        info->root_end = ranges[2 * link + 1].x + ranges[2 * link + 1].y;
+        info->disk_limit = -1.0f;
+        info->tally = 0;
+    }
+    if (flags & 1) return;
+    v3 lo, hi;
+    load_root_box<DIM>(root, lo, hi);
+    const DiskScope q = disk_scope(lo, hi);
+    int kept = 0;
+    for (int s = tid / DISK_OWN; s < n_slots; s += SMALL_BLOCK / DISK_OWN) {
+        const int2 rg = ranges[s];
+        if (rg.y > DISK_OWN) continue;
+        load_slot_box<DIM>(records, s, lo, hi);
+        const float4 d = slot_disk<DIM>(prims, rg, tid % DISK_OWN, DISK_OWN, lo, hi, q);
+        if (tid % DISK_OWN == 0) {
+            disks[s] = d;
+            kept += d.w != 0.0f ? 1 : 0;
+        }
+    }
+    for (int w = wave; w < n_big; w += SMALL_BLOCK / 64) {
+        load_slot_box<DIM>(records, big[w], lo, hi);
+        const float4 d = slot_disk<DIM>(prims, ranges[big[w]], lane, 64, lo, hi, q);
+        if (lane == 0) disks[big[w]] = d;
+    }
+    if (kept) atomicAdd(&n_kept, kept);
+    __syncthreads();
+    if (tid == 0) info->disk_limit = disk_limit_of(n_kept, n_slots - n_big, flags != 0, q);
 }
 
 // Adjoint of d(x, mesh): recompute p and its barycentric weights from the saved

@@ -19,6 +19,8 @@
 static void *noalloc_scratch_ptr(fcpw_hip_ctx *c);
 // the record layout of an uploaded tree (defined before upload_tree)
 static int relayout_records(fcpw_hip_ctx *c, int layout);
+// the primitives in leaf order, from the vertices (defined before update_positions)
+static int launch_rebuild(fcpw_hip_ctx *c, hipStream_t s);
 
 // scenes of several objects (instances.hpp)
 static int instances_refit(fcpw_hip_ctx *c, hipStream_t s);
@@ -34,6 +36,32 @@ static int exclusive_scan(fcpw_hip_ctx *c, uint32_t *v, int64_t n, uint32_t *sum
     HIPCHECK(c, hipGetLastError());
     return FCPW_HIP_OK;
 }
+
+// Copies of host arrays into one device region, as a single copy where it is small:
+// each takes 5 to 10 us whatever it holds.
+struct Upload {
+    static constexpr size_t STAGED_MAX = 1 << 18;
+    fcpw_hip_ctx *c;
+    char *base;
+    size_t bytes;
+    std::vector<char> staged;
+    Upload(fcpw_hip_ctx *ctx, void *region, size_t n) : c(ctx), base((char *)region), bytes(n)
+    {
+        if (n <= STAGED_MAX) staged.resize(n);
+    }
+    int put(void *dst, const void *src, size_t n)
+    {
+        if (n == 0) return FCPW_HIP_OK;
+        if (!staged.empty()) memcpy(staged.data() + ((char *)dst - base), src, n);
+        else HIPCHECK(c, hipMemcpy(dst, src, n, hipMemcpyHostToDevice));
+        return FCPW_HIP_OK;
+    }
+    int finish()
+    {
+        if (!staged.empty()) HIPCHECK(c, hipMemcpy(base, staged.data(), bytes, hipMemcpyHostToDevice));
+        return FCPW_HIP_OK;
+    }
+};
 
 // device scratch of the build: numbered slots kept in the context and grown on
 // demand, so a rebuild of a scene of the same size allocates nothing
@@ -67,20 +95,42 @@ static dim3 slot_grid(const fcpw_hip_ctx *c)
     return dim3((unsigned)(slot_own_blocks(c) + (c->n_big + DISK_BLOCK / 64 - 1) / (DISK_BLOCK / 64)));
 }
 
-// the disks of a single object's tree, from its records, primitives and ranges; info = what
-// k_slot_ranges found, null where the boxes have just been refitted
-static int launch_disks(fcpw_hip_ctx *c, hipStream_t s, const int *info = nullptr)
+static int launch_small_tree(fcpw_hip_ctx *c)
 {
-    if (!c->by_range) return FCPW_HIP_OK;
-    const int n_slots = 2 * c->n_records;
+    if (c->dim == 3)
+        hipLaunchKernelGGL(k_small_tree<3>, dim3(1), dim3(SMALL_BLOCK), 0, 0, c->records, c->root, c->prims,
+                           c->n_records, c->ranges, c->big, c->disks, c->slot_info);
+    else
+        hipLaunchKernelGGL(k_small_tree<2>, dim3(1), dim3(SMALL_BLOCK), 0, 0, c->records, c->root, c->prims,
+                           c->n_records, c->ranges, c->big, c->disks, c->slot_info);
+    HIPCHECK(c, hipGetLastError());
+    return FCPW_HIP_OK;
+}
+
+template <int DIM>
+static int launch_refit_small(fcpw_hip_ctx *c, hipStream_t s)
+{
+    const int n_slots = 2 * c->n_records, per = DISK_BLOCK / DISK_OWN, own = (n_slots + per - 1) / per;
+    const int waves = DISK_BLOCK / 64;
+    hipLaunchKernelGGL(k_refit_small<DIM>, dim3((unsigned)(own + (c->n_big + waves - 1) / waves)),
+                       dim3(DISK_BLOCK), 0, s, c->records, c->root, c->prims, c->ranges, n_slots, c->big, c->n_big,
+                       own, c->disks, c->slot_info, c->root_range);
+    HIPCHECK(c, hipGetLastError());
+    return FCPW_HIP_OK;
+}
+
+// the disks of a tree with ranges, from its records and primitives
+static int launch_disks(fcpw_hip_ctx *c, hipStream_t s, int refitted)
+{
+    const int n_slots = 2 * c->n_records, n_own = n_slots - c->n_big - c->n_top;
     if (c->dim == 3)
         hipLaunchKernelGGL(k_build_disks<3>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->root, c->prims,
-                           c->ranges, n_slots, c->big, c->n_big, n_slots - c->n_big - c->n_top, slot_own_blocks(c),
-                           c->disks, c->disk_limit, info, c->disk_tally);
+                           c->ranges, n_slots, c->big, c->n_big, n_own, slot_own_blocks(c), c->disks, c->slot_info,
+                           refitted);
     else
         hipLaunchKernelGGL(k_build_disks<2>, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->root, c->prims,
-                           c->ranges, n_slots, c->big, c->n_big, n_slots - c->n_big - c->n_top, slot_own_blocks(c),
-                           c->disks, c->disk_limit, info, c->disk_tally);
+                           c->ranges, n_slots, c->big, c->n_big, n_own, slot_own_blocks(c), c->disks, c->slot_info,
+                           refitted);
     HIPCHECK(c, hipGetLastError());
     return FCPW_HIP_OK;
 }
@@ -95,56 +145,62 @@ static int launch_faces(fcpw_hip_ctx *c, hipStream_t s, int *kept = nullptr)
     return FCPW_HIP_OK;
 }
 
-// ranges, slot lists and disks of a tree whose slots were (re)numbered
+// Ranges, slot lists and disks of a tree whose slots were (re)numbered.  The host
+// waits for what it has to know: once for a small tree, twice for others.
 template <int DIM>
 static int compute_ranges(fcpw_hip_ctx *c)
 {
     c->by_range = false;
     c->disks_off = true;
     c->n_big = c->n_top = c->n_frontier = 0;
-    const float none = -1.0f;
-    HIPCHECK(c, hipMemcpy(c->disk_limit, &none, sizeof(float), hipMemcpyHostToDevice));
+    SlotInfo info;
     // a root leaf has no slots; and where nodes have no or two parents the lists
     // below would hold more slots than a tree has (upload_ranges)
-    if (c->n_records <= 0 || !c->one_tree) return FCPW_HIP_OK;
+    if (c->n_records <= 0 || !c->one_tree) {
+        memset(&info, 0, sizeof(info));
+        info.disk_limit = -1.0f;
+        HIPCHECK(c, hipMemcpy(c->slot_info, &info, sizeof(info), hipMemcpyHostToDevice));
+        return FCPW_HIP_OK;
+    }
     const int n_slots = 2 * c->n_records, t = 256;
-    const dim3 gs((unsigned)((n_slots + t - 1) / t));
-    HIPCHECK(c, hipMemset(c->range_info, 0, 4 * sizeof(int)));
-    HIPCHECK(c, hipMemset(c->disk_tally, 0, sizeof(unsigned long long)));
-    HIPCHECK(c, hipMemset(c->range_mark, 0, ((size_t)c->n_prims + 1) * sizeof(uint32_t)));
-    hipLaunchKernelGGL(k_slot_ranges<DIM>, dim3((unsigned)((c->n_records + t - 1) / t)), dim3(t), 0, 0, c->records,
-                       c->root, c->prims, c->n_records, c->ranges, c->range_info);
-    HIPCHECK(c, hipGetLastError());
-    int info[4];
-    HIPCHECK(c, hipMemcpy(info, c->range_info, sizeof(info), hipMemcpyDeviceToHost));
-    if (info[0]) return FCPW_HIP_OK; // leaves out of order: boxes alone, refitted by climbing
-    hipLaunchKernelGGL(k_slot_lists<DIM>, gs, dim3(t), 0, 0, c->ranges, c->root, n_slots, c->big, c->top,
-                       c->range_mark, c->range_info);
-    const int st = exclusive_scan(c, c->range_mark, (int64_t)c->n_prims + 1, c->range_sums, 0);
-    if (st) return st;
-    hipLaunchKernelGGL(k_slot_frontier<DIM>, gs, dim3(t), 0, 0, c->ranges, c->root, n_slots, c->range_mark, c->top,
-                       c->frontier, c->range_info);
-    HIPCHECK(c, hipGetLastError());
-    uint32_t n_frontier = 0;
-    HIPCHECK(c, hipMemcpy(info, c->range_info, sizeof(info), hipMemcpyDeviceToHost));
-    HIPCHECK(c, hipMemcpy(&n_frontier, c->range_mark + c->n_prims, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    c->n_big = info[1];
-    c->n_top = info[2];
-    c->n_frontier = (int)n_frontier;
+    const bool small = c->n_prims <= SMALL_PRIMS;
+    int st;
+    if (small) {
+        if ((st = launch_small_tree(c))) return st;
+    } else {
+        const dim3 gs((unsigned)((n_slots + t - 1) / t));
+        HIPCHECK(c, hipMemsetAsync(c->slot_info, 0, sizeof(info), 0));
+        HIPCHECK(c, hipMemsetAsync(c->range_mark, 0, ((size_t)c->n_prims + 1) * sizeof(uint32_t), 0));
+        hipLaunchKernelGGL(k_slot_ranges<DIM>, dim3((unsigned)((c->n_records + t - 1) / t)), dim3(t), 0, 0,
+                           c->records, c->root, c->prims, c->n_records, c->ranges, c->slot_info);
+        hipLaunchKernelGGL(k_slot_lists<DIM>, gs, dim3(t), 0, 0, c->ranges, c->root, n_slots, c->big, c->top,
+                           c->range_mark, c->slot_info);
+        if ((st = exclusive_scan(c, c->range_mark, (int64_t)c->n_prims + 1, c->range_sums, 0))) return st;
+        hipLaunchKernelGGL(k_slot_frontier<DIM>, gs, dim3(t), 0, 0, c->ranges, c->root, n_slots, c->range_mark,
+                           c->top, c->frontier, c->n_prims, c->slot_info);
+        HIPCHECK(c, hipGetLastError());
+    }
+    HIPCHECK(c, hipMemcpy(&info, c->slot_info, sizeof(info), hipMemcpyDeviceToHost));
+    if (info.out_of_order) return FCPW_HIP_OK; // boxes alone, refitted by climbing
+    c->n_big = info.n_big;
+    c->n_top = info.n_top;
+    c->n_frontier = info.n_frontier;
+    c->root_range = make_int2(info.root_first, info.root_end);
     c->by_range = true;
-    const int st_disks = launch_disks(c, 0, c->range_info);
-    if (st_disks) return st_disks;
-    float limit = 0.0f;
-    HIPCHECK(c, hipMemcpy(&limit, c->disk_limit, sizeof(float), hipMemcpyDeviceToHost));
-    c->disks_off = limit < 0.0f && !info[3]; // stale boxes: until a refit, which may be a graph's
+    if (!small) {
+        if ((st = launch_disks(c, 0, 0))) return st;
+        HIPCHECK(c, hipMemcpy(&info.disk_limit, &c->slot_info->disk_limit, sizeof(float), hipMemcpyDeviceToHost));
+    }
+    c->disks_off = info.disk_limit < 0.0f && !info.stale; // stale boxes: until a refit, which may be a graph's
     return FCPW_HIP_OK;
 }
 
 static int compute_ranges(fcpw_hip_ctx *c) { return c->dim == 3 ? compute_ranges<3>(c) : compute_ranges<2>(c); }
 
 // allocates the ranges, lists and disks of a freshly uploaded or built tree (one
-// allocation) and computes them; c's counts, dimension and tree must be set
-static int upload_ranges(fcpw_hip_ctx *c)
+// allocation) and computes them; c's counts, dimension and tree must be set.
+// rebuild: the primitives are to be gathered first
+static int upload_ranges(fcpw_hip_ctx *c, bool rebuild)
 {
     const size_t n_slots = (size_t)2 * c->n_records, n_prims = (size_t)c->n_prims;
     // in one tree (compute_ranges) slots above DISK_MAX_PRIMS are disjoint at each of
@@ -161,8 +217,7 @@ static int upload_ranges(fcpw_hip_ctx *c)
     const size_t at_disks = take(n_slots * sizeof(float4)), at_top = take(cap_top * sizeof(int4)),
                  at_ranges = take(n_slots * sizeof(int2)), at_big = take(n_slots * sizeof(int)),
                  at_front = take(cap_front * sizeof(int)), at_mark = take((n_prims + 1) * sizeof(uint32_t)),
-                 at_sums = take(segs * sizeof(uint32_t)), at_info = take(4 * sizeof(int)), at_limit = take(sizeof(float)),
-                 at_tally = take(sizeof(unsigned long long));
+                 at_sums = take(segs * sizeof(uint32_t)), at_info = take(sizeof(SlotInfo));
     HIPCHECK(c, hipMalloc((void **)&c->range_mem, bytes));
     char *m = (char *)c->range_mem;
     c->disks = (float4 *)(m + at_disks);
@@ -172,13 +227,12 @@ static int upload_ranges(fcpw_hip_ctx *c)
     c->frontier = (int *)(m + at_front);
     c->range_mark = (uint32_t *)(m + at_mark);
     c->range_sums = (uint32_t *)(m + at_sums);
-    c->range_info = (int *)(m + at_info);
-    c->disk_limit = (float *)(m + at_limit);
-    c->disk_tally = (unsigned long long *)(m + at_tally);
-    const int st = compute_ranges(c);
-    if (st) return st;
-    HIPCHECK(c, hipDeviceSynchronize());
-    return FCPW_HIP_OK;
+    c->slot_info = (SlotInfo *)(m + at_info);
+    if (rebuild) {
+        const int st = launch_rebuild(c, 0);
+        if (st) return st;
+    }
+    return compute_ranges(c);
 }
 
 static unsigned blocks_for(int64_t n, int t) { return (unsigned)std::max<int64_t>(1, (n + t - 1) / t); }
@@ -386,7 +440,7 @@ static int gpu_build(fcpw_hip_ctx *c, const float *positions, int n_vertices, co
     c->one_tree = true;
     c->node_slot = std::move(node_slot);
     c->node_leaf_off = std::move(node_leaf_off);
-    const int st_disks = upload_ranges(c);
+    const int st_disks = upload_ranges(c, false);
     if (st_disks) return st_disks;
     c->uploaded = true;
     c->generation++;
@@ -712,26 +766,40 @@ static int relayout_records(fcpw_hip_ctx *c, int layout)
 }
 
 // allocates and fills the tree buffers of c (records, root, leaf-slot index,
-// refit schedule); the scene's previous buffers must have been freed
+// refit schedule; one allocation); the scene's previous buffers must have been freed
 static int upload_tree(fcpw_hip_ctx *c, const TreeRecords &T, const int32_t *slot_index, int n_slots)
 {
-    size_t rec_bytes = T.rec.size() * sizeof(float4);
-    HIPCHECK(c, hipMalloc((void **)&c->records, rec_bytes));
-    HIPCHECK(c, hipMalloc((void **)&c->root, 2 * sizeof(float4)));
-    HIPCHECK(c, hipMalloc((void **)&c->prim_index, (size_t)n_slots * sizeof(int32_t)));
-    HIPCHECK(c, hipMalloc((void **)&c->rec_parent, T.parent.size() * sizeof(int32_t)));
-    HIPCHECK(c, hipMalloc((void **)&c->leaf_refs, T.leaf_refs.size() * sizeof(int32_t)));
-    HIPCHECK(c, hipMalloc((void **)&c->leaf_links, T.leaf_links.size() * sizeof(uint32_t)));
-    HIPCHECK(c, hipMalloc((void **)&c->counters, T.parent.size() * sizeof(unsigned int)));
-    HIPCHECK(c, hipMemcpy(c->records, T.rec.data(), rec_bytes, hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->root, T.root, sizeof(T.root), hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->prim_index, slot_index, (size_t)n_slots * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->rec_parent, T.parent.data(), T.parent.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->leaf_refs, T.leaf_refs.data(), T.leaf_refs.size() * sizeof(int32_t),
-                          hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->leaf_links, T.leaf_links.data(), T.leaf_links.size() * sizeof(uint32_t),
-                          hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemset(c->counters, 0, T.parent.size() * sizeof(unsigned int)));
+    size_t bytes = 0;
+    auto take = [&bytes](size_t b) {
+        const size_t at = bytes;
+        bytes += (b + 255) / 256 * 256;
+        return at;
+    };
+    const size_t rec_bytes = T.rec.size() * sizeof(float4), count_bytes = T.parent.size() * sizeof(unsigned int);
+    const size_t at_rec = take(rec_bytes), at_root = take(sizeof(T.root)),
+                 at_index = take((size_t)n_slots * sizeof(int32_t)),
+                 at_parent = take(T.parent.size() * sizeof(int32_t)),
+                 at_refs = take(T.leaf_refs.size() * sizeof(int32_t)),
+                 at_links = take(T.leaf_links.size() * sizeof(uint32_t)), at_count = take(count_bytes);
+    HIPCHECK(c, hipMalloc(&c->tree_mem, bytes));
+    char *m = (char *)c->tree_mem;
+    c->records = (float4 *)(m + at_rec);
+    c->root = (float4 *)(m + at_root);
+    c->prim_index = (int32_t *)(m + at_index);
+    c->rec_parent = (int32_t *)(m + at_parent);
+    c->leaf_refs = (int32_t *)(m + at_refs);
+    c->leaf_links = (uint32_t *)(m + at_links);
+    c->counters = (unsigned int *)(m + at_count);
+    Upload up(c, m, at_count);
+    int st;
+    if ((st = up.put(c->records, T.rec.data(), rec_bytes))) return st;
+    if ((st = up.put(c->root, T.root, sizeof(T.root)))) return st;
+    if ((st = up.put(c->prim_index, slot_index, (size_t)n_slots * sizeof(int32_t)))) return st;
+    if ((st = up.put(c->rec_parent, T.parent.data(), T.parent.size() * sizeof(int32_t)))) return st;
+    if ((st = up.put(c->leaf_refs, T.leaf_refs.data(), T.leaf_refs.size() * sizeof(int32_t)))) return st;
+    if ((st = up.put(c->leaf_links, T.leaf_links.data(), T.leaf_links.size() * sizeof(uint32_t)))) return st;
+    if ((st = up.finish())) return st;
+    HIPCHECK(c, hipMemsetAsync(c->counters, 0, count_bytes, 0));
     return FCPW_HIP_OK;
 }
 
@@ -766,34 +834,29 @@ int fcpw_hip_upload_bvh(fcpw_hip_ctx *c, int dim, int n_nodes, const float *pmin
         if (prim_vertices[k] < 0 || prim_vertices[k] >= n_vertices)
             FAIL(c, FCPW_HIP_ERR_INVALID_ARGUMENT, "upload_bvh: vertex id out of range");
 
-    // primitive records in leaf-slot order
-    const int PR = dim == 3 ? 3 : 1;
-    std::vector<float4> prims((size_t)n_prims * PR);
-    for (int s = 0; s < n_prims; s++) {
-        if (dim == 3) {
-            for (int k = 0; k < 3; k++) {
-                const float *v = positions + (size_t)prim_vertices[(size_t)s * 3 + k] * 3;
-                prims[(size_t)s * 3 + k] = make_float4(v[0], v[1], v[2], 0.0f);
-            }
-        } else {
-            const float *a = positions + (size_t)prim_vertices[(size_t)s * 2] * 2;
-            const float *b = positions + (size_t)prim_vertices[(size_t)s * 2 + 1] * 2;
-            prims[s] = make_float4(a[0], a[1], b[0], b[1]);
-        }
-    }
-
     HIPCHECK(c, hipSetDevice(c->device));
     free_scene(c);
     st = upload_tree(c, T, prim_index, n_prims);
     if (st) return st;
-    HIPCHECK(c, hipMalloc((void **)&c->prims, prims.size() * sizeof(float4)));
-    HIPCHECK(c, hipMalloc((void **)&c->prim_vids, (size_t)n_prims * dim * sizeof(int32_t)));
-    HIPCHECK(c, hipMalloc((void **)&c->V, (size_t)n_vertices * dim * sizeof(float)));
-    HIPCHECK(c, hipMemcpy(c->prims, prims.data(), prims.size() * sizeof(float4), hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->prim_vids, prim_vertices, (size_t)n_prims * dim * sizeof(int32_t),
-                          hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->V, positions, (size_t)n_vertices * dim * sizeof(float), hipMemcpyHostToDevice));
-    HIPCHECK(c, hipDeviceSynchronize());
+    size_t bytes = 0;
+    auto take = [&bytes](size_t b) {
+        const size_t at = bytes;
+        bytes += (b + 255) / 256 * 256;
+        return at;
+    };
+    const size_t vid_bytes = (size_t)n_prims * dim * sizeof(int32_t),
+                 pos_bytes = (size_t)n_vertices * dim * sizeof(float);
+    const size_t at_vids = take(vid_bytes), at_pos = take(pos_bytes),
+                 at_prims = take((size_t)n_prims * (dim == 3 ? 3 : 1) * sizeof(float4));
+    HIPCHECK(c, hipMalloc(&c->geom_mem, bytes));
+    char *m = (char *)c->geom_mem;
+    c->prim_vids = (int32_t *)(m + at_vids);
+    c->V = (float *)(m + at_pos);
+    c->prims = (float4 *)(m + at_prims);
+    Upload up(c, m, at_prims);
+    if ((st = up.put(c->prim_vids, prim_vertices, vid_bytes))) return st;
+    if ((st = up.put(c->V, positions, pos_bytes))) return st;
+    if ((st = up.finish())) return st;
     set_query_grid(c, pmin, pmax, dim);
     c->dim = dim;
     c->n_records = T.n_rec;
@@ -804,7 +867,7 @@ int fcpw_hip_upload_bvh(fcpw_hip_ctx *c, int dim, int n_nodes, const float *pmin
     c->one_tree = T.one_tree;
     c->node_slot = std::move(T.node_slot);
     c->node_leaf_off = std::move(T.node_leaf_off);
-    if ((st = upload_ranges(c))) return st;
+    if ((st = upload_ranges(c, true))) return st;
     c->uploaded = true;
     c->generation++;
     c->positions_version++;
@@ -907,11 +970,11 @@ int fcpw_hip_upload_silhouettes(fcpw_hip_ctx *c, int n_nodes, const fcpw_hip_bou
     c->sil_open = n_refs > 0 ? (float)(open_sum / n_refs) : 1.0f;
     if (c->by_range && c->dim == 3) {
         HIPCHECK(c, hipMalloc((void **)&c->sil_faces, (size_t)2 * c->n_records * sizeof(float4)));
-        int *const kept = c->range_info; // [0] is zero where there are ranges
+        int *const kept = &c->slot_info->faces;
         int n_kept = 0;
+        HIPCHECK(c, hipMemsetAsync(kept, 0, sizeof(int), 0));
         if ((st = launch_faces(c, 0, kept))) return st;
         HIPCHECK(c, hipMemcpy(&n_kept, kept, sizeof(int), hipMemcpyDeviceToHost));
-        HIPCHECK(c, hipMemset(kept, 0, sizeof(int)));
         if (n_kept < (2 * c->n_records - c->n_big - c->n_top) / 2) { // see launch_silhouettes
             HIPCHECK(c, hipFree(c->sil_faces));
             c->sil_faces = nullptr;
@@ -926,10 +989,10 @@ static int launch_rebuild(fcpw_hip_ctx *c, hipStream_t s)
     int threads = 256, blocks = (c->n_prims + threads - 1) / threads;
     if (c->dim == 3)
         hipLaunchKernelGGL(k_rebuild_prims<3>, dim3(blocks), dim3(threads), 0, s, c->prims, c->prim_vids, c->V,
-                           c->n_prims, c->disk_limit);
+                           c->n_prims, &c->slot_info->disk_limit);
     else
         hipLaunchKernelGGL(k_rebuild_prims<2>, dim3(blocks), dim3(threads), 0, s, c->prims, c->prim_vids, c->V,
-                           c->n_prims, c->disk_limit);
+                           c->n_prims, &c->slot_info->disk_limit);
     HIPCHECK(c, hipGetLastError());
     return FCPW_HIP_OK;
 }
@@ -971,7 +1034,10 @@ int fcpw_hip_refit(fcpw_hip_ctx *c, void *stream)
     hipStream_t s = (hipStream_t)stream;
     if (c->instanced) return instances_refit(c, s);
     int threads = 256, blocks = (c->n_leaves + threads - 1) / threads;
-    if (c->by_range) {
+    const bool small = c->by_range && c->n_prims <= DISK_MAX_PRIMS;
+    if (small) {
+        if ((st = c->dim == 3 ? launch_refit_small<3>(c, s) : launch_refit_small<2>(c, s))) return st;
+    } else if (c->by_range) {
         const int n_slots = 2 * c->n_records;
         const dim3 gt((unsigned)(c->n_top / (DISK_BLOCK / 64) + 1));
         if (c->dim == 3) {
@@ -995,7 +1061,7 @@ int fcpw_hip_refit(fcpw_hip_ctx *c, void *stream)
                                c->leaf_refs, c->leaf_links, c->rec_parent, c->counters, c->n_leaves);
     }
     HIPCHECK(c, hipGetLastError());
-    if ((st = launch_disks(c, s))) return st;
+    if (c->by_range && !small && (st = launch_disks(c, s, 1))) return st;
     c->disks_off = !c->by_range; // where the new boxes' disks do not pay the kernels find them off
     if (c->has_silhouettes) {
         if ((st = launch_faces(c, s))) return st;

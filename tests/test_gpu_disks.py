@@ -194,3 +194,36 @@ def test_disks_off_where_few_slots_keep_one(gpu):
         b.update_vertices(W)
         b.refit()
         check(g, W, F, q, bvh=b)
+
+
+@pytest.mark.parametrize("n", [4, 5, 9, 17, 64, 65, 257, 1023, 1024, 1025, 1040])
+@pytest.mark.parametrize("mesh", ["torus", "star2d"])
+def test_trees_around_the_one_block_size(gpu, mesh, n):
+    """trees of at most DISK_MAX_PRIMS primitives get their ranges, disks and
+    refits from one block: uploaded, reordered and refitted, against the oracle"""
+    import torch
+    V, F = meshes.small_torus(65, 8) if mesh == "torus" else meshes.small_star(1040)
+    F = np.ascontiguousarray(F[:n])
+    assert len(F) == n
+    _, g = make_scene(V, F)
+    b = oracle.Bvh(V, F)
+    q = queries(V[np.unique(F)], 3000, 81)
+    check(g, V, F, q, bvh=b)
+    for k in range(3):
+        V = (V + synth.Rng(82 + k).uniform(V.size, -0.02, 0.02).reshape(V.shape)).astype(np.float32)
+        st = torch.cuda.current_stream().cuda_stream
+        dv = torch.from_numpy(V).cuda()
+        g._update_positions_device(dv.data_ptr(), len(V), st)
+        b.update_vertices(V)
+        if k:
+            g.set_option("layout", k % 2)
+        check(g, V, F, q, bvh=b)
+        g._refit_device(st)
+        b.refit()
+        check(g, V, F, q, bvh=b)
+    # the boxes themselves: the counting variant expands what the reference does
+    g.set_option("stats", 1)
+    check(g, V, F, q, bvh=b)
+    _, ni, npr, _ = b.closest_points_gpuorder(q, counters=True)
+    assert (g.info("stat_internal_nodes"), g.info("stat_prim_tests")) == (int(ni.sum()), int(npr.sum()))
+    g.set_option("stats", 0)
