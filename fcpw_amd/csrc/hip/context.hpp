@@ -51,6 +51,9 @@ struct fcpw_hip_ctx {
     unsigned long long *stats = nullptr; // internal nodes, primitive tests, queries (option "stats")
     // silhouettes (fcpw_hip_upload_silhouettes): cones per child slot and root, leaf ranges, records
     float4 *cones = nullptr, *sils = nullptr;
+    // in one allocation
+    void *sil_mem = nullptr;
+    uint32_t *sil_first = nullptr; // records before each primitive's leaf (for sil_faces)
     float4 *sil_faces = nullptr; // facing entries per child slot (3D trees with ranges, where they pay)
     int sil_unit = 0;            // no record has a normal longer than one
     float sil_open = 1.0f;       // mean of (1 - n0.n1) / 2 over the records
@@ -142,9 +145,9 @@ static std::string g_create_error;
 
 static void free_silhouettes(fcpw_hip_ctx *c)
 {
-    void *bufs[] = {c->cones, c->sils, c->sil_leaf, c->sil_faces};
-    for (void *b : bufs)
-        if (b) (void)hipFree(b);
+    if (c->sil_mem) (void)hipFree(c->sil_mem);
+    c->sil_mem = nullptr;
+    c->sil_first = nullptr;
     c->cones = c->sils = nullptr;
     c->sil_leaf = nullptr;
     c->sil_faces = nullptr;

@@ -139,8 +139,11 @@ static int launch_disks(fcpw_hip_ctx *c, hipStream_t s, int refitted)
 static int launch_faces(fcpw_hip_ctx *c, hipStream_t s, int *kept = nullptr)
 {
     if (!c->sil_faces) return FCPW_HIP_OK;
-    hipLaunchKernelGGL(k_build_faces, slot_grid(c), dim3(DISK_BLOCK), 0, s, c->records, c->ranges, 2 * c->n_records,
-                       c->big, c->n_big, slot_own_blocks(c), c->sil_leaf, c->sils, c->sil_faces, kept);
+    const int n_slots = 2 * c->n_records, own = (n_slots + FACE_BLOCK_SLOTS - 1) / FACE_BLOCK_SLOTS;
+    const int waves = DISK_BLOCK / 64;
+    hipLaunchKernelGGL(k_build_faces, dim3((unsigned)(own + (c->n_big + waves - 1) / waves)), dim3(DISK_BLOCK), 0, s,
+                       c->records, c->ranges, n_slots, c->big, c->n_big, own, c->sil_first, c->sils, c->sil_faces,
+                       kept);
     HIPCHECK(c, hipGetLastError());
     return FCPW_HIP_OK;
 }
@@ -955,30 +958,72 @@ int fcpw_hip_upload_silhouettes(fcpw_hip_ctx *c, int n_nodes, const fcpw_hip_bou
                             : 0.5 * (1.0 - (double)(e.n0.x * e.n1.x + e.n0.y * e.n1.y + e.n0.z * e.n1.z));
         }
     }
+    // where facing entries may be built, the records of a subtree have to lie
+    // together: their numbers before each primitive's leaf, and the records in leaf
+    // order where the caller's are not
+    bool want_faces = c->by_range && c->dim == 3;
+    std::vector<uint32_t> first_rec;
+    if (want_faces) {
+        first_rec.assign((size_t)c->n_prims + 1, 0u);
+        uint64_t run = 0;
+        bool in_order = true;
+        for (int s = 0; s < c->n_prims; s++) {
+            first_rec[s] = (uint32_t)run;
+            if (leaf_buf[s].y && leaf_buf[s].x != run) in_order = false;
+            run += leaf_buf[s].y;
+        }
+        first_rec[c->n_prims] = (uint32_t)run;
+        if (run > (uint64_t)n_refs) { // leaves that share records: without entries
+            want_faces = false;
+            first_rec.clear();
+        } else if (!in_order) {
+            std::vector<float4> by_leaf(std::max<size_t>(run, 1) * RW, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
+            for (int s = 0; s < c->n_prims; s++) {
+                std::copy_n(rec_buf.begin() + (size_t)leaf_buf[s].x * RW, (size_t)leaf_buf[s].y * RW,
+                            by_leaf.begin() + (size_t)first_rec[s] * RW);
+                leaf_buf[s].x = first_rec[s];
+            }
+            rec_buf.swap(by_leaf);
+        }
+    }
     HIPCHECK(c, hipSetDevice(c->device));
     HIPCHECK(c, hipDeviceSynchronize());
     free_silhouettes(c);
-    HIPCHECK(c, hipMalloc((void **)&c->cones, cone_buf.size() * sizeof(float4)));
-    HIPCHECK(c, hipMalloc((void **)&c->sil_leaf, leaf_buf.size() * sizeof(uint2)));
-    HIPCHECK(c, hipMalloc((void **)&c->sils, rec_buf.size() * sizeof(float4)));
-    HIPCHECK(c, hipMemcpy(c->cones, cone_buf.data(), cone_buf.size() * sizeof(float4), hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->sil_leaf, leaf_buf.data(), leaf_buf.size() * sizeof(uint2), hipMemcpyHostToDevice));
-    HIPCHECK(c, hipMemcpy(c->sils, rec_buf.data(), rec_buf.size() * sizeof(float4), hipMemcpyHostToDevice));
+    // one allocation: facing entries, cones, records, leaf ranges, first_rec
+    size_t bytes = 0;
+    auto take = [&bytes](size_t b) {
+        const size_t at = bytes;
+        bytes += (b + 255) / 256 * 256;
+        return at;
+    };
+    const size_t face_bytes = want_faces ? (size_t)2 * c->n_records * sizeof(float4) : 0;
+    const size_t at_faces = take(face_bytes), at_cones = take(cone_buf.size() * sizeof(float4)),
+                 at_sils = take(rec_buf.size() * sizeof(float4)), at_leaf = take(leaf_buf.size() * sizeof(uint2)),
+                 at_first = take(first_rec.size() * sizeof(uint32_t));
+    HIPCHECK(c, hipMalloc(&c->sil_mem, bytes));
+    char *m = (char *)c->sil_mem;
+    c->cones = (float4 *)(m + at_cones);
+    c->sils = (float4 *)(m + at_sils);
+    c->sil_leaf = (uint2 *)(m + at_leaf);
+    c->sil_first = (uint32_t *)(m + at_first);
+    Upload up(c, m + at_cones, bytes - at_cones);
+    if ((st = up.put(c->cones, cone_buf.data(), cone_buf.size() * sizeof(float4)))) return st;
+    if ((st = up.put(c->sils, rec_buf.data(), rec_buf.size() * sizeof(float4)))) return st;
+    if ((st = up.put(c->sil_leaf, leaf_buf.data(), leaf_buf.size() * sizeof(uint2)))) return st;
+    if ((st = up.put(c->sil_first, first_rec.data(), first_rec.size() * sizeof(uint32_t)))) return st;
+    if ((st = up.finish())) return st;
     c->n_sil_refs = n_refs;
     c->sil_leaf_max = leaf_max;
     c->sil_unit = unit ? 1 : 0;
     c->sil_open = n_refs > 0 ? (float)(open_sum / n_refs) : 1.0f;
-    if (c->by_range && c->dim == 3) {
-        HIPCHECK(c, hipMalloc((void **)&c->sil_faces, (size_t)2 * c->n_records * sizeof(float4)));
+    if (want_faces) {
         int *const kept = &c->slot_info->faces;
         int n_kept = 0;
+        c->sil_faces = (float4 *)(m + at_faces);
         HIPCHECK(c, hipMemsetAsync(kept, 0, sizeof(int), 0));
         if ((st = launch_faces(c, 0, kept))) return st;
         HIPCHECK(c, hipMemcpy(&n_kept, kept, sizeof(int), hipMemcpyDeviceToHost));
-        if (n_kept < (2 * c->n_records - c->n_big - c->n_top) / 2) { // see launch_silhouettes
-            HIPCHECK(c, hipFree(c->sil_faces));
-            c->sil_faces = nullptr;
-        }
+        if (n_kept < (2 * c->n_records - c->n_big - c->n_top) / 2) c->sil_faces = nullptr; // see launch_silhouettes
     }
     c->has_silhouettes = true;
     return FCPW_HIP_OK;

@@ -207,3 +207,46 @@ def test_silhouettes_with_leaves_out_of_order(gpu, mesh):
         ref = b.closest_silhouettes(q, flip=flip)
         same = (out[0]["index"].view(np.int32) == ref["index"]) & (out[0]["d"] == ref["d"])
         assert (~same).sum() <= MAX_ULP_FLIPS
+
+
+@pytest.mark.parametrize("shared", [False, True])
+def test_silhouettes_out_of_leaf_order(gpu, shared):
+    """a caller's records in another order than the leaves (they are laid out in
+    leaf order), and leaves that share records (no facing entries): the oracle's
+    silhouettes, before and after a refit"""
+    V, F = MESHES["torus"]()
+    b = oracle.Bvh(V, F)
+    b.build_silhouettes()
+    cones, count, offset, rec = b.silhouettes()
+    if shared:  # one leaf also lists the record that follows its own
+        leaf = np.nonzero(count)[0]
+        count[leaf[np.argmin(offset[leaf])]] += 1
+    else:
+        order = np.random.default_rng(5).permutation(np.nonzero(count)[0])
+        new, at = np.empty_like(rec), 0
+        for i in order:
+            new[at:at + count[i]] = rec[offset[i]:offset[i] + count[i]]
+            offset[i], at = at, at + count[i]
+        rec = new
+    q = queries(V, 4000, 64)
+    s = np.full((len(q), 4), np.finfo(np.float32).max, np.float32)
+    s[:, :3] = q
+    flip = np.zeros(len(q), np.uint32)
+    with Context(3) as c:
+        c.upload(Tree(b, F), V)
+        c.ok(c.lib.fcpw_hip_upload_silhouettes(c.h, len(count), cones.ctypes.data, count.ctypes.data,
+                                               offset.ctypes.data, len(rec), rec.ctypes.data))
+        for refitted in (False, True):
+            out = []
+            for coop in (1, 0):
+                c.option("coop", coop)
+                o = np.zeros(len(q), fcpw.INTERACTION_DTYPE)
+                c.ok(c.lib.fcpw_hip_closest_silhouette_points(c.h, s.ctypes.data, flip.ctypes.data, len(q), 0.0,
+                                                              1e-3, o.ctypes.data))
+                out.append(o)
+            assert out[0].tobytes() == out[1].tobytes()
+            if not refitted:
+                ref = b.closest_silhouettes(q, flip=flip)
+                same = (out[0]["index"].view(np.int32) == ref["index"]) & (out[0]["d"] == ref["d"])
+                assert (~same).sum() <= MAX_ULP_FLIPS
+            c.refit()
