@@ -817,6 +817,26 @@ static void set_query_grid(fcpw_hip_ctx *c, const float *pmin, const float *pmax
     }
 }
 
+// what launch_silhouettes has to know of the edges: whether all normals are at most
+// one long, and how far apart the faces of a record lie, over at most 8,192 of them
+static void silhouette_facts(fcpw_hip_ctx *c, const fcpw_hip_edge *edges, int n)
+{
+    c->sil_unit = 0;
+    c->sil_open = 1.0f;
+    if (!edges || n == 0) return;
+    const auto dot3 = [](const fcpw_hip_float3 &a, const fcpw_hip_float3 &b) { return a.x * b.x + a.y * b.y + a.z * b.z; };
+    bool longer = false; // or a NaN
+    for (int r = 0; r < n; r++)
+        longer |= !(dot3(edges[r].n0, edges[r].n0) < 1.0002f) | !(dot3(edges[r].n1, edges[r].n1) < 1.0002f);
+    c->sil_unit = longer ? 0 : 1;
+    const int stride = std::max(1, n / 8192);
+    double sum = 0.0; // (1 - n0.n1) / 2, of a boundary 1
+    int count = 0;
+    for (int r = 0; r < n; r += stride, count++)
+        sum += edges[r].has_one_adjacent_face == 1u ? 1.0 : 0.5 * (1.0 - (double)dot3(edges[r].n0, edges[r].n1));
+    c->sil_open = (float)(sum / count);
+}
+
 extern "C" {
 
 int fcpw_hip_upload_bvh(fcpw_hip_ctx *c, int dim, int n_nodes, const float *pmin, const float *pmax,
@@ -937,25 +957,22 @@ int fcpw_hip_upload_silhouettes(fcpw_hip_ctx *c, int n_nodes, const fcpw_hip_bou
     }
     const int RW = c->dim == 3 ? 4 : 2;
     std::vector<float4> rec_buf((size_t)std::max(n_refs, 1) * RW, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
-    bool unit = true;
-    double open_sum = 0.0; // (1 - n0.n1) / 2 of the records, 1 of a boundary's
-    const auto at_most_one = [](const fcpw_hip_float3 &n) { return n.x * n.x + n.y * n.y + n.z * n.z < 1.0002f; };
-    for (int r = 0; r < n_refs; r++) {
-        if (c->dim == 2) {
-            const fcpw_hip_vertex &v = ((const fcpw_hip_vertex *)silhouettes)[r];
+    if (c->dim == 2) {
+        const fcpw_hip_vertex *in = (const fcpw_hip_vertex *)silhouettes;
+        for (int r = 0; r < n_refs; r++) {
+            const fcpw_hip_vertex &v = in[r];
             rec_buf[(size_t)r * 2] = make_float4(v.p.x, v.p.y, v.n0.x, v.n0.y);
             rec_buf[(size_t)r * 2 + 1] =
                 make_float4(v.n1.x, v.n1.y, bits_as_float(v.index), bits_as_float(v.has_one_adjacent_face));
-        } else {
-            const fcpw_hip_edge &e = ((const fcpw_hip_edge *)silhouettes)[r];
+        }
+    } else {
+        const fcpw_hip_edge *in = (const fcpw_hip_edge *)silhouettes;
+        for (int r = 0; r < n_refs; r++) {
+            const fcpw_hip_edge &e = in[r];
             rec_buf[(size_t)r * 4] = make_float4(e.pa.x, e.pa.y, e.pa.z, bits_as_float(e.index));
             rec_buf[(size_t)r * 4 + 1] = make_float4(e.pb.x, e.pb.y, e.pb.z, bits_as_float(e.has_one_adjacent_face));
             rec_buf[(size_t)r * 4 + 2] = make_float4(e.n0.x, e.n0.y, e.n0.z, 0.0f);
             rec_buf[(size_t)r * 4 + 3] = make_float4(e.n1.x, e.n1.y, e.n1.z, 0.0f);
-            unit = unit && at_most_one(e.n0) && at_most_one(e.n1);
-            open_sum += e.has_one_adjacent_face == 1u
-                            ? 1.0
-                            : 0.5 * (1.0 - (double)(e.n0.x * e.n1.x + e.n0.y * e.n1.y + e.n0.z * e.n1.z));
         }
     }
     // where facing entries may be built, the records of a subtree have to lie
@@ -1014,8 +1031,7 @@ int fcpw_hip_upload_silhouettes(fcpw_hip_ctx *c, int n_nodes, const fcpw_hip_bou
     if ((st = up.finish())) return st;
     c->n_sil_refs = n_refs;
     c->sil_leaf_max = leaf_max;
-    c->sil_unit = unit ? 1 : 0;
-    c->sil_open = n_refs > 0 ? (float)(open_sum / n_refs) : 1.0f;
+    silhouette_facts(c, (const fcpw_hip_edge *)(c->dim == 3 ? silhouettes : nullptr), n_refs);
     if (want_faces) {
         int *const kept = &c->slot_info->faces;
         int n_kept = 0;
