@@ -1156,7 +1156,10 @@ static dim3 grid_for(fcpw_hip_ctx *, int64_t n, int block)
 // 118; 12,000 on 300,000 triangles 64 a wave 840 us, 4 690; 65,537 occlusion
 // rays 64 a wave 270 us, 32 242, 16 265; 100,003 closest points 64 a wave 171
 // us, 32 163, 16 171.  With the chip full a part-filled wave only wastes issue:
-// 4.2M rays 64 a wave 1.96 ms, 32 2.48 ms.
+// 4.2M rays 64 a wave 1.96 ms, 32 2.48 ms.  Where the number halves the two sides
+// differ little: rays through 131,072 triangles 65,535 (16 a wave) 257 us, 65,537 (32)
+// 263, 131,071 289; through 20,000 162, 158, 180; all against 334 to 349 and 219 to 229
+// with 64 a wave.
 static int wave_queries(const fcpw_hip_ctx *c, int64_t n)
 {
     int q = 64;

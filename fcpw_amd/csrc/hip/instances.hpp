@@ -1301,10 +1301,12 @@ static int launch_instances_closest(fcpw_hip_ctx *c, const void *spheres, int64_
     DevScene T = dev_scene(c);
     // with ordered queries and inst_seed = B: each block's representatives, then
     // the rest with radii lowered from them (seeded_r2); otherwise one launch.
-    // Two launches end twice with their longest walks (2.4 ms with 256 instances
-    // of 20,480 triangles, where one launch of 16,384 queries takes all of that),
-    // so unless the caller chose a block the batch has to be large: 1M queries
-    // there 8.6 ms in one launch against 9.8 in two, 4M 24.0 against 20.5.
+    // Two launches end twice with their longest walks, so unless the caller chose a
+    // block the batch has to be large.  Over 20 scenes (2, 32, 256 and 2,000 instances of
+    // spheres of 1,280 and 20,480 triangles, a rough one, a soup and a torus of 100,000)
+    // two launches take 0.92 to 1.24 times as long as one with 1M queries, 0.83 to 1.11
+    // with 2M, and 0.64 to 0.92 with 4M; 256 of the 20,480-triangle sphere: 1M 8.10 ms in
+    // one and 9.75 in two, 2M 12.8 and 13.2, 4M 21.9 and 18.5.
     const bool seed = c->inst_seed > 0 && (c->inst_seed != INST_SEED_DEFAULT || n >= ((int64_t)1 << 21));
     const int block = order && seed ? c->inst_seed : 0;
     c->launch.block = block;
