@@ -163,6 +163,7 @@ static int compute_ranges(fcpw_hip_ctx *c)
         memset(&info, 0, sizeof(info));
         info.disk_limit = -1.0f;
         HIPCHECK(c, hipMemcpy(c->slot_info, &info, sizeof(info), hipMemcpyHostToDevice));
+        HIPCHECK(c, hipDeviceSynchronize());
         return FCPW_HIP_OK;
     }
     const int n_slots = 2 * c->n_records, t = 256;
@@ -1633,7 +1634,7 @@ static int launch_silhouettes(fcpw_hip_ctx *c, const void *spheres, const uint32
                               float prec, void *out, hipStream_t s)
 {
     DevScene S = dev_scene(c);
-    SilScene T = {c->cones, c->sil_leaf, c->sils, c->sil_faces, c->sil_unit};
+    SilScene T = {c->cones, c->sil_leaf, c->sils, c->sil_faces};
     const uint32_t *order = nullptr;
     int st = morton_order(c, (const float *)spheres, 4, n, s, &order);
     if (st) return st;
@@ -1660,7 +1661,8 @@ static int launch_silhouettes(fcpw_hip_ctx *c, const void *spheres, const uint32
         // Four LDS entries, which keep eight waves a SIMD, for the last kind (1M queries on
         // the sphere of 0.33: 1.82 ms, eight entries 1.97), eight with the others,
         // whose spills cost more (131,072-triangle torus 11.0 ms, four 13.0).
-        const bool faces = c->sil_faces, pre = c->dim == 3 && (faces || c->sil_open < 0.315f);
+        // certainly_off needs normals of at most one, so without them neither.
+        const bool faces = c->sil_faces && c->sil_unit, pre = faces || (c->sil_unit && c->sil_open < 0.315f);
         const int k = c->dim == 2 ? 8 : c->sil_stack != SIL_STACK_DEFAULT ? c->sil_stack : pre ? 8 : 4;
         c->launch = {k, c->sil_hold_min, wq, 0};
 #define FCPW_SIL(DIM, K, FACES, PREPASS)                                                                      \

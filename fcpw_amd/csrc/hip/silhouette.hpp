@@ -27,7 +27,6 @@ struct SilScene {
     const uint2 *sil_leaf;
     const float4 *sils;
     const float4 *faces; // facing entries of the child slots (faces_away)
-    int unit;            // no record has a normal longer than one (certainly_off needs it)
 };
 
 constexpr float PI_F = 3.14159265358979323846f;   // M_PI (math-constants.slang)
@@ -572,7 +571,7 @@ __global__ __launch_bounds__(64) FCPW_EIGHT_WAVES void k_closest_silhouettes_coo
             if (h2) sh.item[i2] = (uint16_t)((lane << 10) | (j0 + 2));
             if (h3) sh.item[i3] = (uint16_t)((lane << 10) | (j0 + 3));
             __syncthreads();
-            if (PREPASS && T.unit) {
+            if constexpr (PREPASS) {
                 uint32_t n_left = 0;
                 for (uint32_t pass = 0; pass < total; pass += 64) {
                     const uint32_t kk = pass + (uint32_t)lane;
