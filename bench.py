@@ -231,7 +231,7 @@ def cpu_baseline(V, F, q, r2, sample, runs=5):
 # rocprofv3 summaries (no GPU needed): turn the SQLite output of a kernel-trace
 # run or of FETCH_SIZE / WRITE_SIZE counter runs into the text kept in profiles/
 # ---------------------------------------------------------------------------
-MAIN_KERNEL = r"k_closest_points_coop<3, \d+, 0, false>"  # any LDS stack depth
+MAIN_KERNEL = r"k_closest_points_coop<3, \d+, 0, false, true>"  # any LDS stack depth
 
 
 def _db(path):
@@ -441,7 +441,8 @@ def run_torus(args, torch):
     I = gpu.info("stat_internal_nodes") / gpu.info("stat_queries")
     P = gpu.info("stat_prim_tests") / gpu.info("stat_queries")
     waves = max(gpu.info("stat_waves"), 1)
-    log(f"[fwd] per wave: {gpu.info('stat_wave_iterations') / waves:.1f} loop iterations, "
+    log(f"[fwd] the counting variant's walk, the reference's, per wave: "
+        f"{gpu.info('stat_wave_iterations') / waves:.1f} loop iterations, "
         f"{gpu.info('stat_leaf_passes') / waves:.1f} leaf passes, {gpu.info('stat_leaf_groups') / waves:.1f} "
         f"64-item groups (one query per lane, no refill)")
     gpu.set_option("stats", 0)

@@ -138,9 +138,10 @@ int fcpw_hip_update_positions_device(fcpw_hip_ctx *ctx, const float *positions, 
                                      void *stream);
 
 /* Replaces runBvhUpdate + the refit entry point (bvh_interop_structures.h:891-934,
-   bvh.cs.slang:135-149): one bottom-up launch recomputes every box; with
-   silhouettes uploaded, a second one recomputes every cone from the current
-   silhouette records (Bvh.refit, bvh.slang:27-141). */
+   bvh.cs.slang:135-149): recomputes every box and the tight bounds of small
+   subtrees, in one to three launches; with silhouettes uploaded, further ones
+   recompute every cone (and facing entry) from the current silhouette records
+   (Bvh.refit, bvh.slang:27-141). */
 int fcpw_hip_refit(fcpw_hip_ctx *ctx, void *stream);
 
 /*
