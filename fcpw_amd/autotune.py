@@ -7,7 +7,7 @@ the same order), so tuning is a pure timing search:
     times the single-scene closest-point launch over candidate settings of
     ``layout`` (the order of the tree's records in memory: DFS or treelets),
     ``coop`` (wave-cooperative leaves or not), ``stack`` (traversal-stack
-    entries kept in LDS), ``hold_min`` (held leaves before a cooperative leaf
+    entries kept in LDS; 6 leaves small batches to the size rule), ``hold_min`` (held leaves before a cooperative leaf
     pass), ``xcds`` (how many ranges of the ordered queries the XCDs split
     into) and, without coop, ``block``; applies and returns the fastest.
     Candidates are grouped by layout, so the records are reordered once per
