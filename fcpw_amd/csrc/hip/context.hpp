@@ -54,7 +54,7 @@ struct fcpw_hip_ctx {
     // in one allocation
     void *sil_mem = nullptr;
     uint32_t *sil_first = nullptr; // records before each primitive's leaf (for sil_faces)
-    float4 *sil_faces = nullptr; // facing entries per child slot (3D trees with ranges, where they pay)
+    float4 *sil_faces = nullptr; // facing entries per child slot (trees with ranges, where they pay)
     int sil_unit = 0;            // no record has a normal longer than one
     float sil_open = 1.0f;       // mean of (1 - n0.n1) / 2 over the records
     uint2 *sil_leaf = nullptr;

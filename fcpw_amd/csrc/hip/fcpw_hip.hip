@@ -141,9 +141,13 @@ static int launch_faces(fcpw_hip_ctx *c, hipStream_t s, int *kept = nullptr)
     if (!c->sil_faces) return FCPW_HIP_OK;
     const int n_slots = 2 * c->n_records, own = (n_slots + FACE_BLOCK_SLOTS - 1) / FACE_BLOCK_SLOTS;
     const int waves = DISK_BLOCK / 64;
-    hipLaunchKernelGGL(k_build_faces, dim3((unsigned)(own + (c->n_big + waves - 1) / waves)), dim3(DISK_BLOCK), 0, s,
-                       c->records, c->ranges, n_slots, c->big, c->n_big, own, c->sil_first, c->sils, c->sil_faces,
-                       kept);
+    const dim3 g((unsigned)(own + (c->n_big + waves - 1) / waves));
+    if (c->dim == 3)
+        hipLaunchKernelGGL(k_build_faces<3>, g, dim3(DISK_BLOCK), 0, s, c->records, c->ranges, n_slots, c->big,
+                           c->n_big, own, c->sil_first, c->sils, c->sil_faces, kept);
+    else
+        hipLaunchKernelGGL(k_build_faces<2>, g, dim3(DISK_BLOCK), 0, s, c->records, c->ranges, n_slots, c->big,
+                           c->n_big, own, c->sil_first, c->sils, c->sil_faces, kept);
     HIPCHECK(c, hipGetLastError());
     return FCPW_HIP_OK;
 }
@@ -818,6 +822,9 @@ static void set_query_grid(fcpw_hip_ctx *c, const float *pmin, const float *pmax
     }
 }
 
+// segments up to which 2D silhouettes take facing entries (launch_silhouettes)
+constexpr int SIL_FACES_MAX_2D = 1 << 15;
+
 // what launch_silhouettes has to know of the edges: whether all normals are at most
 // one long, and how far apart the faces of a record lie, over at most 8,192 of them
 static void silhouette_facts(fcpw_hip_ctx *c, const fcpw_hip_edge *edges, int n)
@@ -979,7 +986,7 @@ int fcpw_hip_upload_silhouettes(fcpw_hip_ctx *c, int n_nodes, const fcpw_hip_bou
     // where facing entries may be built, the records of a subtree have to lie
     // together: their numbers before each primitive's leaf, and the records in leaf
     // order where the caller's are not
-    bool want_faces = c->by_range && c->dim == 3;
+    bool want_faces = c->by_range && (c->dim == 3 || c->n_prims <= SIL_FACES_MAX_2D);
     std::vector<uint32_t> first_rec;
     if (want_faces) {
         first_rec.assign((size_t)c->n_prims + 1, 0u);
@@ -1655,14 +1662,19 @@ static int launch_silhouettes(fcpw_hip_ctx *c, const void *spheres, const uint32
         //    3.27 -> 2.77 ms, of 0.29 200 -> 181, of 0.31 29.5 -> 27.0 (but 0.80 -> 0.90
         //    if all queries are near); of 0.33 1.00 -> 1.11, a soup (all boundary, 1)
         //    0.33 -> 0.39;
-        //  - neither otherwise, and in 2D, whose records are cheap: 262,144 queries on
-        //    a star of 200,000 segments 0.96 ms with both, 0.93 with facing entries, 0.85
-        //    with neither; on a ring of 30,000 0.97, 0.89, 0.97.
+        //  - neither otherwise.
+        // In 2D, whose records are cheap, never the prepass (262,144 queries on a star of
+        // 30,000 segments 0.81 ms with both, 0.75 with facing entries, 0.71 with neither),
+        // and facing entries for at most SIL_FACES_MAX_2D segments: 1,000 queries on stars of 1,000
+        // and 13,511 segments 79 us with them and 89 without, 137 and 142, on a ring of
+        // 30,000 332 and 350, 262,144 there 0.87 and 0.96 ms; on stars of 60,000 and 200,000
+        // 0.65 and 0.61, 0.93 and 0.81.
         // Four LDS entries, which keep eight waves a SIMD, for the last kind (1M queries on
         // the sphere of 0.33: 1.82 ms, eight entries 1.97), eight with the others,
         // whose spills cost more (131,072-triangle torus 11.0 ms, four 13.0).
         // certainly_off needs normals of at most one, so without them neither.
-        const bool faces = c->sil_faces && c->sil_unit, pre = faces || (c->sil_unit && c->sil_open < 0.315f);
+        const bool pre = c->sil_unit && (c->sil_faces || c->sil_open < 0.315f);
+        const bool faces = c->sil_faces && (pre || c->dim == 2);
         const int k = c->dim == 2 ? 8 : c->sil_stack != SIL_STACK_DEFAULT ? c->sil_stack : pre ? 8 : 4;
         c->launch = {k, c->sil_hold_min, wq, 0};
 #define FCPW_SIL(DIM, K, FACES, PREPASS)                                                                      \
@@ -1675,7 +1687,8 @@ static int launch_silhouettes(fcpw_hip_ctx *c, const void *spheres, const uint32
         else if (pre) FCPW_SIL(3, K, false, true);                                                            \
         else FCPW_SIL(3, K, false, false);                                                                    \
     } while (0)
-        if (c->dim == 2) FCPW_SIL(2, 8, false, false);
+        if (c->dim == 2 && faces) FCPW_SIL(2, 8, true, false);
+        else if (c->dim == 2) FCPW_SIL(2, 8, false, false);
         else if (k == 4) FCPW_SIL(3, 4, false, false);
         else if (k == 8) FCPW_SIL3(8);
         else FCPW_SIL3(12);

@@ -279,7 +279,7 @@ __device__ __forceinline__ bool silhouette_test(const SilRecord &s, v3 x, float 
 //   - rounding, here and in the reference's evaluation: 1e-5 of the lengths, and
 //     4e-6 of the coordinates, which F and B hold already.
 // Subtrees with boundary edges, faces without a normal or angles above 60 degrees
-// have none (T infinite), and 2D scenes (launch_silhouettes).  Visits on the 131,072-triangle torus, 262,144 queries:
+// have none (T infinite).  Visits on the 131,072-triangle torus, 262,144 queries:
 // 281 expanded records and 638 record tests a query without, 176 and 332 with.
 //
 // 16 bytes a slot: {a.x, a.y (f16)} {a.z (f16), T (bf16)} {B, F (bf16)}
@@ -667,6 +667,7 @@ __global__ __launch_bounds__(64) FCPW_EIGHT_WAVES void k_closest_silhouettes_coo
 // kept (when not null) counts the former that have an entry.
 constexpr int FACE_LANES = 8, FACE_BLOCK_SLOTS = DISK_BLOCK / FACE_LANES;
 
+template <int DIM>
 __global__ __launch_bounds__(DISK_BLOCK) void k_build_faces(const float4 *records, const int2 *ranges, int n_slots,
                                                             const int *big, int n_big, int own_blocks,
                                                             const uint32_t *first_rec, const float4 *sils,
@@ -691,11 +692,11 @@ __global__ __launch_bounds__(DISK_BLOCK) void k_build_faces(const float4 *record
     }
     const uint32_t begin = first_rec[rg.x] + (uint32_t)lane, end = first_rec[rg.x + rg.y];
     v3 lo, hi;
-    load_slot_box<3>(records, slot, lo, hi);
+    load_slot_box<DIM>(records, slot, lo, hi);
     const v3 c = {0.5f * (lo.x + hi.x), 0.5f * (lo.y + hi.y), 0.5f * (lo.z + hi.z)};
     v3 sum = {0.0f, 0.0f, 0.0f};
     for (uint32_t k = begin; k < end; k += (uint32_t)lanes) {
-        const SilRecord r = load_silhouette<3>(sils, k);
+        const SilRecord r = load_silhouette<DIM>(sils, k);
         sum = {sum.x + r.n0.x + r.n1.x, sum.y + r.n0.y + r.n1.y, sum.z + r.n0.z + r.n1.z};
     }
     for (int off = lanes / 2; off > 0; off >>= 1) {
@@ -710,14 +711,14 @@ __global__ __launch_bounds__(DISK_BLOCK) void k_build_faces(const float4 *record
     float cosine = 1.0f, front = 0.0f, back = 0.0f, far2 = 0.0f, coord = 0.0f;
     int bad = 0;
     for (uint32_t k = begin; k < end; k += (uint32_t)lanes) {
-        const SilRecord r = load_silhouette<3>(sils, k);
+        const SilRecord r = load_silhouette<DIM>(sils, k);
         if (r.one == 1u) bad = 1;
         for (int f = 0; f < 2; f++) {
             const v3 n = f ? r.n1 : r.n0;
             const float nn = dot(n, n);
             if (!(nn > 0.99999f && nn < 1.00001f)) bad = 1;
             cosine = fminf(cosine, dot(n, a));
-            for (int e = 0; e < 2; e++) {
+            for (int e = 0; e < (DIM == 3 ? 2 : 1); e++) {
                 const v3 p = e ? r.pb : r.pa, w = sub(p, c);
                 const float o = dot(n, w);
                 if (!(fabsf(o) < 1e18f)) bad = 1;

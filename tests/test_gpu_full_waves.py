@@ -26,7 +26,7 @@ def noisy_sphere(amplitude):
     return synth.f32(synth.radial_noise(v, amplitude, synth.Rng(9))), f.astype(np.int32)
 
 
-# with facing entries and prepass, with the prepass alone, and with neither
+# with facing entries and prepass, with the prepass alone, with neither; in 2D with the entries alone
 SILHOUETTES = {
     "torus": (lambda: meshes.small_torus(64, 32), 8),
     "noisy": (lambda: noisy_sphere(0.05), 8),
@@ -34,6 +34,7 @@ SILHOUETTES = {
     "soup": (CASES["soup"], 4),
     "open_plate": (CASES["plate_tilted"], 8),
     "star2d": (CASES["star2d"], 8),
+    "star2d_past_the_line": (lambda: meshes.small_star((1 << 15) + 1), 8),  # no facing entries
 }
 
 
